@@ -1,14 +1,12 @@
-// sell.hip -- SELL-C matrices for the row-parallel kernels: SpMV and the
-// level-blocked matrix powers (MPK).
+// sell.hip -- SELL-C matrices for the row-parallel kernels: SpMV, SymmSpMV,
+// SpMTV, the refinement's residual and the matrix powers (MPK).
 //
 // A chunk is up to 64 consecutive rows (one wavefront, one row per lane);
 // its entries are stored column-major, entry j of lane i at off + 64 j + i,
 // so every load instruction of a wave reads one contiguous 512-byte line of
 // values (256 of indices).  Rows shorter than the chunk's widest row are
-// padded with value 0 on the row's own column.  Chunks never cross a "cut"
-// row (the level-group boundaries for MPK), so a row range made of whole
-// groups is a contiguous range of chunks.  Rows keep their order (sigma = 1:
-// the level ordering is what the MPK blocking relies on).
+// padded with value 0 on the row's own column.  Rows keep their order
+// (sigma = 1): RACE's level order keeps the x entries of a chunk close.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -61,33 +59,27 @@ struct SellMatrix {
     int maxW = 0;               // the widest chunk
     bool narrow() const { return maxW <= 8; }
     long entries = 0;
-    std::vector<int> cutChunk;  // chunk index of every cut
     DevBuf<SellChunk> chunks;
     DevBuf<int> col;
     DevBuf<VT> val;
 
-    // cuts: sorted row boundaries starting with 0 and ending with n.  With
-    // one range and chunk widths close to each other (padding every chunk to
-    // the widest adds at most 1/8), all chunks get the widest width: the
-    // kernels then compute a chunk's place instead of loading it.
-    int build(const race_kernel_desc& d, const std::vector<int>& cuts, bool allowUniform = false) {
+    // With chunk widths close to each other (padding every chunk to the
+    // widest adds at most 1/8), all chunks get the widest width: the kernels
+    // then compute a chunk's place instead of loading it.
+    int build(const race_kernel_desc& d, bool allowUniform = true) {
         n = d.nrow;
         const int* rp = d.rowPtr;
         std::vector<SellChunk> ch;
-        cutChunk.clear();
         long total = 0;
-        for (size_t k = 0; k + 1 < cuts.size(); ++k) {
-            cutChunk.push_back((int)ch.size());
-            for (int r0 = cuts[k]; r0 < cuts[k + 1]; r0 += kC) {
-                const int rows = std::min(kC, cuts[k + 1] - r0);
-                int w = 0;
-                for (int i = 0; i < rows; ++i) w = std::max(w, rp[r0 + i + 1] - rp[r0 + i]);
-                ch.push_back(SellChunk{r0, rows, w, (int)(total / kC)});
-                total += (long)w * kC;
-            }
+        for (int r0 = 0; r0 < n; r0 += kC) {
+            const int rows = std::min(kC, n - r0);
+            int w = 0;
+            for (int i = 0; i < rows; ++i) w = std::max(w, rp[r0 + i + 1] - rp[r0 + i]);
+            ch.push_back(SellChunk{r0, rows, w, (int)(total / kC)});
+            total += (long)w * kC;
         }
         uniformW = -1;
-        if (allowUniform && cuts.size() == 2 && !ch.empty()) {
+        if (allowUniform && !ch.empty()) {
             int wmax = 0;
             for (const SellChunk& c : ch) wmax = std::max(wmax, c.width);
             const long padded = (long)wmax * kC * (long)ch.size();
@@ -101,7 +93,6 @@ struct SellMatrix {
                 }
             }
         }
-        cutChunk.push_back((int)ch.size());
         nChunk = (int)ch.size();
         entries = total;
         maxW = 0;
@@ -261,57 +252,6 @@ __global__ void __launch_bounds__(kBlock) k_sell_symm_atomic(const SellChunk* __
     }
 }
 
-// One wavefront step of the matrix powers: segment s computes power q_s on
-// chunks [c0, c1) (whole level groups) from power q_s - 1.
-struct MpkSeg {
-    int c0, c1, q, blockStart;
-};
-
-// Up to kSegArgs segments of a step travel by value in the kernel
-// arguments, so finding a block's segment costs no memory round trip; a
-// step with more segments (powers above 16) reads them from the device
-// table.
-constexpr int kSegArgs = 16;
-struct MpkSegArgs {
-    MpkSeg s[kSegArgs];
-};
-
-// Power q is stored in vector slot q % nslot: nslot = k + 1 keeps every
-// power, nslot = 2 keeps the last two (the only-highest variant).
-template <typename VT, typename XT, bool TABLE, bool NARROW>
-__global__ void __launch_bounds__(kBlock) k_sell_mpk_step(const SellChunk* __restrict__ chunks,
-                                                          const int* __restrict__ col,
-                                                          const VT* __restrict__ val, XT* __restrict__ x, long n,
-                                                          int nslot, const MpkSeg* __restrict__ segs,
-                                                          MpkSegArgs inl, int nseg) {
-    // the block's segment: the last one starting at or before it (by
-    // value: selects over arguments that are all loaded, no branches)
-    MpkSeg sg;
-    if (TABLE) {
-        int s = 0;
-        while (s + 1 < nseg && (int)blockIdx.x >= segs[s + 1].blockStart) ++s;
-        sg = segs[s];
-    } else {
-        sg = inl.s[0];
-#pragma unroll
-        for (int q = 1; q < kSegArgs; ++q) {
-            const MpkSeg o = inl.s[q];
-            const bool take = q < nseg && (int)blockIdx.x >= o.blockStart;
-            sg.c0 = take ? o.c0 : sg.c0;
-            sg.c1 = take ? o.c1 : sg.c1;
-            sg.q = take ? o.q : sg.q;
-            sg.blockStart = take ? o.blockStart : sg.blockStart;
-        }
-    }
-    const int c = sg.c0 + ((int)blockIdx.x - sg.blockStart) * kWavesPerBlock + (int)threadIdx.x / kC;
-    const int lane = threadIdx.x % kC;
-    if (c >= sg.c1) return;
-    const SellChunk k = chunks[c];
-    const XT* __restrict__ xin = x + (long)((sg.q - 1) % nslot) * n;
-    const XT t = sellRow<NARROW>(k, lane, col, val, xin);
-    if (lane < k.rows) x[(long)(sg.q % nslot) * n + k.row0 + lane] = t;
-}
-
 // one launch of y = A x or y += A x over a single-range SELL matrix
 template <bool ACC, bool NARROW, typename VT, typename XT>
 void launchSellShape(const SellMatrix<VT>& A, const void* x, void* y, int nrhs, hipStream_t st) {
@@ -342,7 +282,7 @@ class SellSpmvFn : public DeviceFn {
         x = d.x;
         b = d.b;
         nrhs = d.nrhs > 0 ? d.nrhs : 1;
-        return A.build(d, {0, d.nrow}, true);
+        return A.build(d);
     }
     int run(bool, hipStream_t st) override {
         launchSell<false, VT, XT>(A, x, b, nrhs, st);
@@ -370,7 +310,7 @@ class SymmSellFn : public DeviceFn {
         const int n = d.nrow;
         if (mode == 2) {
             if (!std::is_same<VT, double>::value || !std::is_same<XT, double>::value) return ERR_NOT_IMPLEMENTED;
-            return A.build(d, {0, n});
+            return A.build(d, false);
         }
         // full pattern: row r holds its upper entries, then the transposed
         // entries (c, r) of rows c < r, each in increasing c
@@ -400,7 +340,7 @@ class SymmSellFn : public DeviceFn {
         f.rowPtr = rp.data();
         f.col = fc.data();
         f.val = fv.data();
-        return A.build(f, {0, n}, true);
+        return A.build(f);
     }
     int run(bool, hipStream_t st) override {
         if constexpr (std::is_same<VT, double>::value && std::is_same<XT, double>::value) {
@@ -418,26 +358,22 @@ class SymmSellFn : public DeviceFn {
     }
 };
 
-// Level-blocked matrix powers x_q = A x_{q-1}, q = 1..k, x_q at x + q n.
-// Level group g at power q reads power q - 1 of groups g - 1, g, g + 1
-// (BFS levels only touch neighbouring levels): the dependency rule of the
-// reference's trapezoidal wavefront (src/functionManager.cpp:618-822).  Step
-// L computes power q on group L - 2 (q - 1); its inputs were written by steps
-// L - 3 .. L - 1, so the segments of a step are independent and run as one
-// launch.  A step touches at most 2k consecutive level groups, which the
-// cache model (src/matrixPower.cpp:88-140, 685-940) sized to stay in the
-// Infinity Cache, so A is read from HBM about once per call.
+// Matrix powers x_q = A x_{q-1}, q = 1..k, x_q at x + q n: one SpMV launch
+// per power.  RACE blocks the powers by level groups so that A stays in a
+// CPU cache between them (src/matrixPower.cpp:88-140, 685-940); the host
+// executor follows that schedule, the device does not.  Per row and power
+// the products and their order are the same, only the launches differ.  A
+// slope-2 wavefront over the groups (power q on group L - 2 (q - 1) in launch
+// L) was measured on 7-point 192^3, k = 8, 256 MB blocking, FP64: 100 launches,
+// 1.23 ms, against 1.02 ms for 8 launches; 27-point 33^3, k = 5, 4 MB, FP32:
+// 31 launches, 139.7 us, against 19.3 us.  The 256 MB Infinity Cache serves a
+// gathering SpMV little faster than HBM, so the reuse does not pay for the
+// extra launches (3-5 us each) at any size.
 //
 // Only-highest variant (MAT_SPMV_KERNEL_only_highest
 // examples/src/helpers/kernels.cpp:706-734): two vector slots, power q in
-// slot q % 2.  Writing (g, q) overwrites (g, q - 2), whose readers (g - 1 .. g
-// + 1 at power q - 1) ran at steps up to L - 1, and (g, q) is overwritten by
-// (g, q + 2) at step L + 4 after its readers (steps up to L + 3).  Inside a
-// step, a segment reads slot (q' - 1) % 2 of groups g' - 1 .. g' + 1 while
-// another writes slot q % 2 of group g = g' + 2 (q' - q); the slots differ
-// unless q' = q, so no segment reads what another writes.
+// slot q % 2.
 //
-// The step tables of every power 1..k are built at registration, so
 // setPower(p <= k) runs the first p powers.  With FP32 / BF16 values the
 // powers are FP32 vectors accumulated in FP32.
 template <typename VT, typename XT>
@@ -445,10 +381,6 @@ class MpkFn : public DeviceFn {
   public:
     SellMatrix<VT> A;
     int nslot = 2;
-    // for power p: segments stepSeg[p][L] .. stepSeg[p][L+1] of step L
-    std::vector<std::vector<int>> stepSeg, stepBlocks;
-    std::vector<MpkSeg> hostSegs;
-    DevBuf<MpkSeg> segs;
     int init(const race_kernel_desc& d, const ExecContext& ctx) {
         kind = d.kind;
         x = d.x;
@@ -464,10 +396,11 @@ class MpkFn : public DeviceFn {
         const std::vector<int>& gp = ctx.mpk->groupPtr;
         if (gp.size() < 2 || gp.front() != 0 || gp.back() != d.nrow) return ERR_INVALID_ARG;
         const int G = (int)gp.size() - 1;
-        // The wavefront needs every entry of group g in groups g-1..g+1.
-        // BFS levels guarantee it; with mtxType "L" / "U" (row order as
-        // levels) it holds only for matrices whose entries stay within
-        // neighbouring groups, so anything else is refused here.
+        // RACE's schedule computes power q of a group from power q - 1 of
+        // the neighbouring groups.  BFS levels guarantee that this is enough;
+        // with mtxType "L" / "U" (row order as levels) it holds only for
+        // matrices whose entries stay within neighbouring groups, so
+        // anything else is refused, as the schedule cannot run it.
         {
             std::vector<int> grp(d.nrow);
             for (int g = 0; g < G; ++g)
@@ -478,63 +411,19 @@ class MpkFn : public DeviceFn {
                     if (dg < -1 || dg > 1) return ERR_INCOMPATIBILITY;
                 }
         }
-        int e;
-        if ((e = A.build(d, gp))) return e;
-        std::vector<MpkSeg>& all = hostSegs;
-        all.clear();
-        stepSeg.assign(powerMax + 1, {});
-        stepBlocks.assign(powerMax + 1, {});
-        for (int p = 1; p <= powerMax; ++p) {
-            stepSeg[p].assign(1, (int)all.size());
-            for (int L = 0; L < G + 2 * (p - 1); ++L) {
-                int blocks = 0;
-                for (int q = 1; q <= p; ++q) {
-                    const int g = L - 2 * (q - 1);
-                    if (g < 0 || g >= G) continue;
-                    const int c0 = A.cutChunk[g], c1 = A.cutChunk[g + 1];
-                    if (c1 <= c0) continue;
-                    all.push_back(MpkSeg{c0, c1, q, blocks});
-                    blocks += (c1 - c0 + kWavesPerBlock - 1) / kWavesPerBlock;
-                }
-                stepSeg[p].push_back((int)all.size());
-                stepBlocks[p].push_back(blocks);
-            }
-        }
-        return upload(segs, all.data(), all.size());
+        return A.build(d);
     }
     bool graphable() const override { return true; }
     int launches(bool) const override {
         const int steps = power * subPower;
-        if (steps < 1 || steps > powerMax) return 0;
-        int k = 0;
-        for (int nb : stepBlocks[steps]) k += nb > 0;
-        return k;
+        return steps < 1 || steps > powerMax ? 0 : steps;
     }
     int run(bool, hipStream_t st) override {
         const int steps = power * subPower;
         if (steps < 1 || steps > powerMax) return ERR_INVALID_ARG;
-        const std::vector<int>& sg = stepSeg[steps];
-        const std::vector<int>& nb = stepBlocks[steps];
-        for (int L = 0; L + 1 < (int)sg.size(); ++L) {
-            if (nb[L] == 0) continue;
-            const int ns = sg[L + 1] - sg[L];
-            MpkSegArgs inl{};
-            if (ns <= kSegArgs) std::copy(hostSegs.begin() + sg[L], hostSegs.begin() + sg[L + 1], inl.s);
-            const dim3 grid(nb[L]), block(kBlock);
-            const MpkSeg* tab = segs.p + sg[L];
-            if (ns <= kSegArgs && A.narrow())
-                hipLaunchKernelGGL((k_sell_mpk_step<VT, XT, false, true>), grid, block, 0, st, A.chunks.p, A.col.p,
-                                   A.val.p, (XT*)x, (long)A.n, nslot, tab, inl, ns);
-            else if (ns <= kSegArgs)
-                hipLaunchKernelGGL((k_sell_mpk_step<VT, XT, false, false>), grid, block, 0, st, A.chunks.p,
-                                   A.col.p, A.val.p, (XT*)x, (long)A.n, nslot, tab, inl, ns);
-            else if (A.narrow())
-                hipLaunchKernelGGL((k_sell_mpk_step<VT, XT, true, true>), grid, block, 0, st, A.chunks.p, A.col.p,
-                                   A.val.p, (XT*)x, (long)A.n, nslot, tab, inl, ns);
-            else
-                hipLaunchKernelGGL((k_sell_mpk_step<VT, XT, true, false>), grid, block, 0, st, A.chunks.p,
-                                   A.col.p, A.val.p, (XT*)x, (long)A.n, nslot, tab, inl, ns);
-        }
+        for (int q = 1; q <= steps; ++q)
+            launchSell<false, VT, XT>(A, (const XT*)x + (size_t)((q - 1) % nslot) * A.n,
+                                      (XT*)x + (size_t)(q % nslot) * A.n, 1, st);
         RACE_HIP(hipGetLastError());
         return OK;
     }
@@ -573,7 +462,7 @@ class SpmtvFn : public DeviceFn {
         t.rowPtr = rp.data();
         t.col = tc.data();
         t.val = tv.data();
-        return A.build(t, {0, n}, true);
+        return A.build(t);
     }
     int run(bool, hipStream_t st) override {
         launchSell<true, VT, XT>(A, x, b, nrhs, st);
@@ -631,7 +520,7 @@ __global__ void __launch_bounds__(kBlock) k_sell_residual(const SellChunk* __res
 class SellResidual : public ResidualOp {
   public:
     SellMatrix<double> A;
-    int init(const race_kernel_desc& d) { return A.build(d, {0, d.nrow}, true); }
+    int init(const race_kernel_desc& d) { return A.build(d); }
     template <typename RT, bool NARROW>
     void launch(const double* x, const double* b, void* r, int nrhs, double* norms, hipStream_t st) {
         const int blocks = std::max(1, std::min(4096, (A.nChunk + kWavesPerBlock - 1) / kWavesPerBlock));
