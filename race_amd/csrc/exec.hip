@@ -176,29 +176,6 @@ __global__ void __launch_bounds__(kBlock) k_symmspmv_chunks(
     }
 }
 
-// b = A x over all rows
-template <int TPR>
-__global__ void __launch_bounds__(kBlock) k_spmv(const int* __restrict__ rp,
-                                                 const int* __restrict__ col,
-                                                 const double* __restrict__ val,
-                                                 const double* __restrict__ x, double* __restrict__ b,
-                                                 int n, int nrhs, int rowLo, int rowHi, long xoff,
-                                                 long boff) {
-    const int lane = threadIdx.x % TPR;
-    const int row = rowLo + (blockIdx.x * blockDim.x + threadIdx.x) / TPR;
-    if (row >= rowHi) return;
-    const int s = rp[row], e = rp[row + 1];
-    for (int k = 0; k < nrhs; ++k) {
-        const size_t off = (size_t)k * n;
-        double t = 0.0;
-        for (int j = s + lane; j < e; j += TPR) t += val[j] * x[xoff + off + col[j]];
-        t = groupSum<TPR>(t);
-        if (lane == 0) b[boff + off + row] = t;
-    }
-}
-
-
-
 // device CRS copy of a caller matrix
 struct DevCrs {
     int n = 0;
@@ -335,42 +312,6 @@ class SymmSpmvFn : public DeviceFn {
     }
 };
 
-class SpmvFn : public DeviceFn {
-  public:
-    DevCrs A;
-    int nrhs = 1, tpr = 8;
-    int init(const race_kernel_desc& d) {
-        kind = d.kind;
-        nrhs = d.nrhs > 0 ? d.nrhs : 1;
-        x = d.x;
-        b = d.b;
-        int e;
-        if ((e = A.load(d))) return e;
-        tpr = pickTpr(A.nnz, A.n);
-        return OK;
-    }
-    template <int TPR>
-    void launch(int lo, int hi, long xo, long bo, double* xx, double* bb, hipStream_t st) {
-        const long threads = (long)(hi - lo) * TPR;
-        hipLaunchKernelGGL(k_spmv<TPR>, dim3(gridFor(threads)), dim3(kBlock), 0, st, A.rp.p,
-                           A.col.p, A.val.p, xx, bb, A.n, nrhs, lo, hi, xo, bo);
-    }
-    void rows(int lo, int hi, long xo, long bo, double* xx, double* bb, hipStream_t st) {
-        if (hi <= lo) return;
-        switch (tpr) {
-            case 4: launch<4>(lo, hi, xo, bo, xx, bb, st); break;
-            case 8: launch<8>(lo, hi, xo, bo, xx, bb, st); break;
-            case 16: launch<16>(lo, hi, xo, bo, xx, bb, st); break;
-            default: launch<32>(lo, hi, xo, bo, xx, bb, st); break;
-        }
-    }
-    int run(bool, hipStream_t st) override {
-        rows(0, A.n, 0, 0, (double*)x, (double*)b, st);
-        RACE_HIP(hipGetLastError());
-        return OK;
-    }
-};
-
 }  // namespace
 
 int makeWaveFn(const race_kernel_desc& d, const ExecContext& ctx, std::unique_ptr<DeviceFn>* out) {
@@ -436,16 +377,9 @@ int makeDeviceFn(const race_kernel_desc& d, const ExecContext& ctx, std::unique_
             *out = std::move(f);
             break;
         }
-        case RACE_K_SPMV: {
-            if (d.nrhs <= 1 || !fp64) {
-                e = makeSellSpmvFn(d, out);
-                break;
-            }
-            auto f = std::make_unique<SpmvFn>();
-            e = f->init(d);
-            *out = std::move(f);
+        case RACE_K_SPMV:
+            e = makeSellSpmvFn(d, out);
             break;
-        }
         case RACE_K_SPMTV:
             e = makeSpmtvFn(d, out);
             break;

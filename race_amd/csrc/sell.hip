@@ -1,16 +1,29 @@
 // sell.hip -- SELL-C matrices for the row-parallel kernels: SpMV, SymmSpMV,
 // SpMTV, the refinement's residual and the matrix powers (MPK).
 //
-// A chunk is up to 64 consecutive rows (one wavefront, one row per lane);
-// its entries are stored column-major, entry j of lane i at off + 64 j + i,
-// so every load instruction of a wave reads one contiguous 512-byte line of
-// values (256 of indices).  Rows shorter than the chunk's widest row are
-// padded with value 0 on the row's own column.  Rows keep their order
-// (sigma = 1): RACE's level order keeps the x entries of a chunk close.
+// A chunk is 64 consecutive rows, one wavefront, one row per lane.  Rows keep
+// their order (sigma = 1): RACE's level order keeps the x entries of a chunk
+// close.  The entries of a chunk are cut into blocks of 8 entries per row and
+// one last block each of 4, 2 and 1 (the binary digits of width % 8); inside a
+// block a lane's entries are packed so that it reads them 16 bytes at a time
+// (packPos).  Column ids are 16-bit offsets from the smallest column of their
+// slot (entry position j of the chunk), whose 32-bit base comes through the
+// scalar unit; matrices with a slot wider than 65535 columns keep 32-bit ids.
+//
+// What bounds these kernels is memory: per entry a value and a column id, per
+// row its x and y.  One 64-lane load instruction costs the address unit 16
+// cycles whatever its width, so with 2-byte and 4-byte loads per entry the
+// 27-point BF16 product (81 loads per row) was bound by that unit and not by
+// its bytes.  Measured against one 4-byte column id and one value load per
+// entry (both on the same matrices): SpMTV 27-point 96^3 BF16 30.6 -> 21.6 us,
+// SpMV 27-point 96^3 FP64 51.0 -> 38.4 us, 8 right-hand sides 524 -> 135 us
+// (the entries were read once per right-hand side), 7-point 192^3 FP64 130.2 ->
+// 116.9 us, SymmSpMV 7-point 64^3 FP64 6.9 -> 6.5 us.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <cstdint>
+#include <thread>
 #include <type_traits>
 
 #include "exec.hpp"
@@ -22,13 +35,6 @@ namespace {
 
 constexpr int kC = 64;               // rows per chunk (one wavefront)
 constexpr int kWavesPerBlock = kBlock / kC;
-
-// 16 bytes, one load: entry offset in units of 64 (every chunk stores
-// 64 * width entries, so offsets are multiples of 64)
-struct SellChunk {
-    int row0, rows, width, off64;
-    __host__ __device__ long off() const { return (long)off64 * kC; }
-};
 
 // matrix value storage (double, float, or bfloat16 bits); the arithmetic
 // runs in the vector type XT: FP64, or FP32 accumulation for FP32 / BF16
@@ -52,164 +58,294 @@ __device__ __forceinline__ XT fromStorage(uint16_t v) {
     return (XT)__uint_as_float((unsigned)v << 16);
 }
 
+// f(lo, hi) over [0, n) in contiguous parts on up to 8 host threads
+template <class F>
+void parallelRanges(int n, int grain, F&& f) {
+    const int want = std::min({8, (int)std::max(1u, std::thread::hardware_concurrency()), n / std::max(1, grain)});
+    if (want <= 1) {
+        f(0, n);
+        return;
+    }
+    std::vector<std::thread> ts;
+    ts.reserve(want);
+    for (int t = 0; t < want; ++t)
+        ts.emplace_back([&f, n, want, t] { f((int)((long)n * t / want), (int)((long)n * (t + 1) / want)); });
+    for (std::thread& t : ts) t.join();
+}
+
+// A block of E entries per lane of elements T: a lane reads V of them at once
+template <typename T>
+constexpr int packWidth(int E) {
+    return E * (int)sizeof(T) <= 16 ? E : 16 / (int)sizeof(T);
+}
+template <typename T>
+__host__ __device__ inline int packPos(int E, int e, int lane) {
+    const int V = packWidth<T>(E);
+    return (e / V) * kC * V + lane * V + e % V;
+}
+// entry j of a chunk of width W: the block's first entry and its size
+__host__ __device__ inline void blockOf(int W, int j, int& j0, int& E) {
+    const int full = W & ~7;
+    if (j < full) {
+        j0 = j & ~7;
+        E = 8;
+        return;
+    }
+    j0 = full;
+    E = W & 4;
+    if (E == 0 || j >= j0 + 4) {
+        j0 += E;
+        E = W & 2;
+        if (E == 0 || j >= j0 + 2) {
+            j0 += E;
+            E = 1;
+        }
+    }
+}
+
+struct SellChunk {
+    int width, off64;  // entry offset in units of 64
+};
+
+// what a kernel needs of a SELL matrix
+template <typename CT, typename VT>
+struct SellView {
+    const SellChunk* chunks;
+    const int* base;      // smallest column of every slot (CT uint16_t), at off64 + j
+    const CT* col;
+    const VT* val;
+    const uint8_t* pad;   // per row: chunk width - row length, or null:
+    const int* rowPtr;    // then the row length from the row pointers
+    int n, nChunk, W;     // W >= 0: every chunk has this width
+};
+
 template <typename VT>
 struct SellMatrix {
     int n = 0, nChunk = 0;
     int uniformW = -1;          // >= 0: every chunk has this width, chunk c at c * 64 * width
-    int maxW = 0;               // the widest chunk
-    bool narrow() const { return maxW <= 8; }
-    long entries = 0;
+    bool narrowIds = false;     // 16-bit column ids
+    long bytes = 0;             // stored entries
     DevBuf<SellChunk> chunks;
-    DevBuf<int> col;
+    DevBuf<int> base, rowPtr;
+    DevBuf<uint16_t> col16;
+    DevBuf<int> col32;
     DevBuf<VT> val;
+    DevBuf<uint8_t> pad;
+
+    template <typename CT>
+    SellView<CT, VT> view() const {
+        const CT* c;
+        if constexpr (sizeof(CT) == 2)
+            c = col16.p;
+        else
+            c = col32.p;
+        return SellView<CT, VT>{chunks.p, base.p, c, val.p, pad.n ? pad.p : nullptr, rowPtr.p, n, nChunk, uniformW};
+    }
 
     // With chunk widths close to each other (padding every chunk to the
     // widest adds at most 1/8), all chunks get the widest width: the kernels
     // then compute a chunk's place instead of loading it.
-    int build(const race_kernel_desc& d, bool allowUniform = true) {
+    int build(const race_kernel_desc& d) {
         n = d.nrow;
         const int* rp = d.rowPtr;
-        std::vector<SellChunk> ch;
+        nChunk = (n + kC - 1) / kC;
+        std::vector<SellChunk> ch(nChunk);
         long total = 0;
-        for (int r0 = 0; r0 < n; r0 += kC) {
-            const int rows = std::min(kC, n - r0);
+        int wmax = 0;
+        for (int c = 0; c < nChunk; ++c) {
             int w = 0;
-            for (int i = 0; i < rows; ++i) w = std::max(w, rp[r0 + i + 1] - rp[r0 + i]);
-            ch.push_back(SellChunk{r0, rows, w, (int)(total / kC)});
-            total += (long)w * kC;
+            for (int r = c * kC; r < std::min(n, (c + 1) * kC); ++r) w = std::max(w, rp[r + 1] - rp[r]);
+            ch[c] = SellChunk{w, (int)total};
+            total += w;
+            wmax = std::max(wmax, w);
         }
         uniformW = -1;
-        if (allowUniform && !ch.empty()) {
-            int wmax = 0;
-            for (const SellChunk& c : ch) wmax = std::max(wmax, c.width);
-            const long padded = (long)wmax * kC * (long)ch.size();
-            if (padded * 8 <= total * 9) {
-                uniformW = wmax;
-                total = 0;
-                for (SellChunk& c : ch) {
-                    c.width = wmax;
-                    c.off64 = (int)(total / kC);
-                    total += (long)wmax * kC;
+        if ((long)wmax * nChunk * 8 <= total * 9) {
+            uniformW = wmax;
+            for (int c = 0; c < nChunk; ++c) ch[c] = SellChunk{wmax, (int)std::min<long>((long)c * wmax, INT32_MAX)};
+            total = (long)wmax * nChunk;
+        }
+        if (total > (long)INT32_MAX) return ERR_INVALID_ARG;  // offsets in units of 64 must fit an int
+        // per slot its smallest column; 16-bit ids if no slot spans more
+        std::vector<int> lo((size_t)total, 0);
+        std::vector<uint8_t> pd((size_t)nChunk * kC, 0);
+        std::vector<char> wide(nChunk, 0), deep(nChunk, 0);
+        parallelRanges(nChunk, 256, [&](int c0, int c1) {
+            std::vector<int> hi;
+            for (int c = c0; c < c1; ++c) {
+                const int w = ch[c].width;
+                int* l = lo.data() + ch[c].off64;
+                std::fill(l, l + w, INT32_MAX);
+                hi.assign(w, -1);
+                for (int i = 0; i < kC && c * kC + i < n; ++i) {
+                    const int r = c * kC + i, len = rp[r + 1] - rp[r];
+                    for (int j = 0; j < len; ++j) {
+                        l[j] = std::min(l[j], d.col[rp[r] + j]);
+                        hi[j] = std::max(hi[j], d.col[rp[r] + j]);
+                    }
+                    if (w - len > 255) deep[c] = 1;
+                    pd[(size_t)c * kC + i] = (uint8_t)std::min(w - len, 255);
+                }
+                for (int j = 0; j < w; ++j) {
+                    if (hi[j] < 0) l[j] = 0;  // no row reaches this slot (uniform widths)
+                    if (hi[j] - l[j] > 65535) wide[c] = 1;
                 }
             }
-        }
-        nChunk = (int)ch.size();
-        entries = total;
-        maxW = 0;
-        for (const SellChunk& c : ch) maxW = std::max(maxW, c.width);
-        if (total / kC > (long)INT32_MAX) return ERR_INVALID_ARG;  // offsets in units of 64 must fit an int
-        std::vector<int> hc((size_t)total);
-        std::vector<VT> hv((size_t)total);
-        for (const SellChunk& c : ch)
-            for (int i = 0; i < kC; ++i) {
-                const int r = c.row0 + std::min(i, c.rows - 1);
-                const int len = i < c.rows ? rp[r + 1] - rp[r] : 0;
-                for (int j = 0; j < c.width; ++j) {
-                    const long pos = c.off() + (long)j * kC + i;
-                    if (j < len) {
-                        hc[pos] = d.col[rp[r] + j];
-                        hv[pos] = toStorage<VT>(d.val[rp[r] + j]);
-                    } else {
-                        hc[pos] = r;
-                        hv[pos] = toStorage<VT>(0.0);
+        });
+        narrowIds = std::find(wide.begin(), wide.end(), 1) == wide.end();
+        bytes = total * kC * (long)((narrowIds ? sizeof(uint16_t) : sizeof(int)) + sizeof(VT));
+        const bool shallow = std::find(deep.begin(), deep.end(), 1) == deep.end();
+        std::vector<uint16_t> h16(narrowIds ? (size_t)total * kC : 0);
+        std::vector<int> h32(narrowIds ? 0 : (size_t)total * kC);
+        std::vector<VT> hv((size_t)total * kC);
+        parallelRanges(nChunk, 256, [&](int c0, int c1) {
+            for (int c = c0; c < c1; ++c) {
+                const int w = ch[c].width;
+                for (int j = 0; j < w; ++j) {
+                    int j0, E;
+                    blockOf(w, j, j0, E);
+                    const size_t at = (size_t)(ch[c].off64 + j0) * kC;
+                    const int l = lo[ch[c].off64 + j];
+                    for (int i = 0; i < kC; ++i) {
+                        const int r = c * kC + i;
+                        const bool live = r < n && j < rp[r + 1] - rp[r];
+                        const int col = live ? d.col[rp[r] + j] : l;
+                        if (narrowIds)
+                            h16[at + packPos<uint16_t>(E, j - j0, i)] = (uint16_t)(col - l);
+                        else
+                            h32[at + packPos<int>(E, j - j0, i)] = col;
+                        hv[at + packPos<VT>(E, j - j0, i)] = live ? toStorage<VT>(d.val[rp[r] + j]) : VT(0);
                     }
                 }
             }
+        });
         int e;
         if ((e = upload(chunks, ch.data(), ch.size()))) return e;
-        if ((e = upload(col, hc.data(), hc.size()))) return e;
-        if ((e = upload(val, hv.data(), hv.size()))) return e;
-        return OK;
+        if (narrowIds && (e = upload(base, lo.data(), lo.size()))) return e;
+        if (narrowIds && (e = upload(col16, h16.data(), h16.size()))) return e;
+        if (!narrowIds && (e = upload(col32, h32.data(), h32.size()))) return e;
+        if (shallow && (e = upload(pad, pd.data(), pd.size()))) return e;
+        if (!shallow && (e = upload(rowPtr, rp, (size_t)n + 1))) return e;
+        return upload(val, hv.data(), hv.size());
     }
 };
 
-// G entries of a row from entry j0: the column ids and values are loaded
-// together, then the x gathers, so each group is two dependent memory
-// levels and its loads need no branch.  CLAMP (the row's last group): past
-// the chunk's width a lane re-reads the chunk's last entry and multiplies
-// its value by 0 (a product, not a select on the loaded value, which the
-// compiler would turn into a branch around the gathers); t + (+-0) * x == t
-// for finite values (t starts at +0, and a sum that starts at +0 is never
-// -0).
-template <int G, bool CLAMP, typename VT, typename XT>
-__device__ __forceinline__ void sellGroup(const int* __restrict__ cc, const VT* __restrict__ vv, int j0, int width,
-                                          const XT* __restrict__ x, XT& t) {
-    int c[G];
-    XT v[G];
+// E consecutive entries of every lane of a block (NT: with non-temporal loads)
+template <int E, bool NT, typename T>
+__device__ __forceinline__ void loadPack(const T* __restrict__ p, int lane, T (&out)[E]) {
+    constexpr int V = packWidth<T>(E), B = V * (int)sizeof(T);
+    typedef unsigned W4 __attribute__((ext_vector_type(4)));
+    using P = std::conditional_t<B == 16, W4,
+                                 std::conditional_t<B == 8, uint64_t, std::conditional_t<B == 4, uint32_t, uint16_t>>>;
+    const P* __restrict__ q = reinterpret_cast<const P*>(p) + lane;
 #pragma unroll
-    for (int u = 0; u < G; ++u) {
-        const int j = CLAMP ? min(j0 + u, width - 1) : j0 + u;
-        c[u] = cc[j * kC];
-        const XT a = fromStorage<XT>(vv[j * kC]);
-        v[u] = CLAMP ? a * (j0 + u < width ? XT(1) : XT(0)) : a;
+    for (int s = 0; s < E / V; ++s) {
+        const P a = NT ? __builtin_nontemporal_load(q + s * kC) : q[s * kC];
+        __builtin_memcpy(out + s * V, &a, B);
     }
+}
+
+// t[q] += the products of one block with NR right-hand sides (x[q] their
+// vectors).  Entries past the row's length multiply 0 by 0: a padding entry
+// never brings an x that the row does not have into its sum.
+template <int E, int NR, typename CT, typename VT, typename XT>
+__device__ __forceinline__ void sellBlock(const CT (&c)[E], const VT (&v)[E], const int* __restrict__ base, int left,
+                                          const XT* const (&x)[NR], XT (&t)[NR]) {
 #pragma unroll
-    for (int u = 0; u < G; ++u) t += v[u] * x[c[u]];
-}
-
-// y[row] = sum_j a_j x[c_j] for the rows of one chunk; sequential in j, as
-// the CRS row order.  NARROW (no chunk wider than 8 entries): one clamped
-// group of 8, two dependent memory levels per row.  Otherwise whole groups
-// of 8, then clamped groups of 4 (at most 3 entries re-read per row).  The
-// two shapes are separate kernels: in one kernel the compiler merges the
-// tails and gathers part of the group in a second round.  The padding lanes
-// of a chunk hold value-0 entries on a real row, so every lane of the chunk
-// may compute; callers guard the store.
-template <bool NARROW, typename VT, typename XT>
-__device__ __forceinline__ XT sellRow(const SellChunk& k, int lane, const int* __restrict__ col,
-                                      const VT* __restrict__ val, const XT* __restrict__ x) {
-    const int* __restrict__ cc = col + k.off() + lane;
-    const VT* __restrict__ vv = val + k.off() + lane;
-    XT t = XT(0);
-    if (NARROW) {
-        if (k.width > 0) sellGroup<8, true>(cc, vv, 0, k.width, x, t);
-    } else {
-        int j0 = 0;
-        for (; j0 + 8 <= k.width; j0 += 8) sellGroup<8, false>(cc, vv, j0, k.width, x, t);
-        for (; j0 < k.width; j0 += 4) sellGroup<4, true>(cc, vv, j0, k.width, x, t);
-    }
-    return t;
-}
-
-// y = A x (ACC: y += A x) for nrhs right-hand sides (vectors column-major,
-// v[r + k n])
-template <bool ACC, bool NARROW, typename VT, typename XT>
-__global__ void __launch_bounds__(kBlock) k_sell_spmv(const SellChunk* __restrict__ chunks, int nChunk,
-                                                      const int* __restrict__ col, const VT* __restrict__ val,
-                                                      const XT* __restrict__ x, XT* __restrict__ y, long n,
-                                                      int nrhs) {
-    const int c = blockIdx.x * kWavesPerBlock + threadIdx.x / kC;
-    const int lane = threadIdx.x % kC;
-    if (c >= nChunk) return;
-    const SellChunk k = chunks[c];
-    for (int q = 0; q < nrhs; ++q) {
-        const XT t = sellRow<NARROW>(k, lane, col, val, x + q * n);
-        if (lane >= k.rows) continue;
-        if (ACC)
-            y[q * n + k.row0 + lane] += t;
-        else
-            y[q * n + k.row0 + lane] = t;
+    for (int q = 0; q < NR; ++q) {
+        XT g[E];
+#pragma unroll
+        for (int e = 0; e < E; ++e) g[e] = x[q][sizeof(CT) == 2 ? (unsigned)base[e] + (unsigned)c[e] : (unsigned)c[e]];
+#pragma unroll
+        for (int e = 0; e < E; ++e) t[q] += fromStorage<XT>(v[e]) * (e < left ? g[e] : XT(0));
     }
 }
 
-// the same over uniform chunks: chunk c holds rows [64 c, 64 c + 64) at
-// c * 64 * W, no chunk records to load
-template <bool ACC, bool NARROW, typename VT, typename XT>
-__global__ void __launch_bounds__(kBlock) k_sell_spmv_u(int W, const int* __restrict__ col,
-                                                        const VT* __restrict__ val, const XT* __restrict__ x,
-                                                        XT* __restrict__ y, int n, int nrhs) {
-    const int c = blockIdx.x * kWavesPerBlock + threadIdx.x / kC;
-    const int lane = threadIdx.x % kC;
+// the row sums of one chunk for NR right-hand sides; sequential in the
+// row's entries, as the CRS row order.  The entries of the last blocks are
+// requested first, those of each full block while the x entries of the one
+// before it arrive.
+template <int NR, bool NT, typename CT, typename VT, typename XT>
+__device__ __forceinline__ void sellRow(const SellView<CT, VT>& A, int c, int lane, const XT* const (&x)[NR],
+                                        XT (&t)[NR]) {
+    int W = A.W;
+    long s0 = (long)c * W;  // first slot
+    if (W < 0) {
+        const SellChunk k = A.chunks[c];
+        W = __builtin_amdgcn_readfirstlane(k.width);
+        s0 = __builtin_amdgcn_readfirstlane(k.off64);
+    }
     const int r = c * kC + lane;
-    if (c * kC >= n) return;  // a whole wave past the last chunk
-    const SellChunk k{0, kC, W, c * W};
-    for (int q = 0; q < nrhs; ++q) {
-        const XT t = sellRow<NARROW>(k, lane, col, val, x + (long)q * n);
-        if (r >= n) continue;  // padding lanes of the last chunk
-        if (ACC)
-            y[(long)q * n + r] += t;
-        else
-            y[(long)q * n + r] = t;
+    const int len = A.pad ? W - (int)A.pad[r] : r < A.n ? A.rowPtr[r + 1] - A.rowPtr[r] : 0;
+    const CT* __restrict__ col = A.col + s0 * kC;
+    const VT* __restrict__ val = A.val + s0 * kC;
+    const int* __restrict__ base = A.base + (sizeof(CT) == 2 ? s0 : 0);
+    const int full = W & ~7, at2 = full + (W & 4), at1 = at2 + (W & 2);
+    CT c4[4], c2[2], c1[1];
+    VT v4[4], v2[2], v1[1];
+    if (W & 4) {
+        loadPack<4, NT>(col + (long)full * kC, lane, c4);
+        loadPack<4, NT>(val + (long)full * kC, lane, v4);
+    }
+    if (W & 2) {
+        loadPack<2, NT>(col + (long)at2 * kC, lane, c2);
+        loadPack<2, NT>(val + (long)at2 * kC, lane, v2);
+    }
+    if (W & 1) {
+        loadPack<1, NT>(col + (long)at1 * kC, lane, c1);
+        loadPack<1, NT>(val + (long)at1 * kC, lane, v1);
+    }
+    if (full) {
+        CT c8[8];
+        VT v8[8];
+        loadPack<8, NT>(col, lane, c8);
+        loadPack<8, NT>(val, lane, v8);
+        for (int j = 0; j < full; j += 8) {
+            CT cn[8] = {};
+            VT vn[8] = {};
+            if (j + 8 < full) {
+                loadPack<8, NT>(col + (long)(j + 8) * kC, lane, cn);
+                loadPack<8, NT>(val + (long)(j + 8) * kC, lane, vn);
+            }
+            sellBlock<8, NR>(c8, v8, base + j, len - j, x, t);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                c8[e] = cn[e];
+                v8[e] = vn[e];
+            }
+        }
+    }
+    if (W & 4) sellBlock<4, NR>(c4, v4, base + full, len - full, x, t);
+    if (W & 2) sellBlock<2, NR>(c2, v2, base + at2, len - at2, x, t);
+    if (W & 1) sellBlock<1, NR>(c1, v1, base + at1, len - at1, x, t);
+}
+
+// y = A x (acc: y += A x) for nrhs right-hand sides (vectors column-major,
+// v[r + k n]), NR at a time: the entries are read once for NR of them.
+template <int NR, bool NT, typename CT, typename VT, typename XT>
+__global__ void __launch_bounds__(kBlock) k_sell(SellView<CT, VT> A, const XT* __restrict__ x, XT* __restrict__ y,
+                                                 int nrhs, int acc, int perXcd) {
+    // the chunk is uniform over its wavefront: its tables load through the scalar unit
+    const int blk = perXcd ? ((int)blockIdx.x & 7) * perXcd + ((int)blockIdx.x >> 3) : (int)blockIdx.x;
+    const int c = blk * kWavesPerBlock + __builtin_amdgcn_readfirstlane(threadIdx.x / kC);
+    const int lane = threadIdx.x % kC;
+    if (c >= A.nChunk) return;
+    const int r = c * kC + lane;
+    for (int q0 = 0; q0 < nrhs; q0 += NR) {
+        const XT* xq[NR];
+        XT t[NR], old[NR];
+#pragma unroll
+        for (int q = 0; q < NR; ++q) {
+            const long vo = (long)min(q0 + q, nrhs - 1) * A.n;
+            xq[q] = x + vo;
+            t[q] = XT(0);
+            old[q] = acc && r < A.n ? y[vo + r] : XT(0);
+        }
+        sellRow<NR, NT>(A, c, lane, xq, t);
+        if (r < A.n)
+#pragma unroll
+            for (int q = 0; q < NR; ++q)
+                if (q0 + q < nrhs) y[(long)(q0 + q) * A.n + r] = old[q] + t[q];
     }
 }
 
@@ -218,29 +354,28 @@ __global__ void __launch_bounds__(kBlock) k_sell_spmv_u(int W, const int* __rest
 // SYMM_SPMV_KERNEL (examples/src/helpers/kernels.cpp:403-427).  Rows of
 // different leaves of a distance-2 colour never write the same b entry, but
 // rows inside a leaf do, and all rows run at once here: every write to b is
-// a device-scope FP64 atomic add.  Padding entries (value 0 on the row's
-// own column) add nothing.
-__global__ void __launch_bounds__(kBlock) k_sell_symm_atomic(const SellChunk* __restrict__ chunks, int nChunk,
-                                                             const int* __restrict__ col,
-                                                             const double* __restrict__ val,
-                                                             const double* __restrict__ x, double* b, long n,
-                                                             int nrhs) {
+// a device-scope FP64 atomic add.
+template <typename CT>
+__global__ void __launch_bounds__(kBlock) k_sell_symm_atomic(SellView<CT, double> A, const double* __restrict__ x,
+                                                             double* b, int nrhs) {
     const int c = blockIdx.x * kWavesPerBlock + threadIdx.x / kC;
     const int lane = threadIdx.x % kC;
-    if (c >= nChunk) return;
-    const SellChunk k = chunks[c];
-    if (lane >= k.rows) return;
-    const int r = k.row0 + lane;
-    const int* __restrict__ cc = col + k.off() + lane;
-    const double* __restrict__ vv = val + k.off() + lane;
+    const int r = c * kC + lane;
+    if (c >= A.nChunk || r >= A.n) return;
+    const int W = A.W >= 0 ? A.W : A.chunks[c].width;
+    const long s0 = A.W >= 0 ? (long)c * W : A.chunks[c].off64;
+    const int len = A.pad ? W - (int)A.pad[r] : A.rowPtr[r + 1] - A.rowPtr[r];
     for (int q = 0; q < nrhs; ++q) {
-        const double* __restrict__ xq = x + q * n;
-        double* bq = b + q * n;
+        const double* __restrict__ xq = x + (long)q * A.n;
+        double* bq = b + (long)q * A.n;
         const double xr = xq[r];
         double t = 0.0;
-        for (int j = 0; j < k.width; ++j) {
-            const int cj = cc[j * kC];
-            const double v = vv[j * kC];
+        for (int j = 0; j < len; ++j) {
+            int j0, E;
+            blockOf(W, j, j0, E);
+            const int cj = (sizeof(CT) == 2 ? A.base[s0 + j] : 0) +
+                           (int)A.col[(s0 + j0) * kC + packPos<CT>(E, j - j0, lane)];
+            const double v = A.val[(s0 + j0) * kC + packPos<double>(E, j - j0, lane)];
             if (cj == r) {
                 t += v * xr;
             } else {
@@ -252,23 +387,51 @@ __global__ void __launch_bounds__(kBlock) k_sell_symm_atomic(const SellChunk* __
     }
 }
 
-// one launch of y = A x or y += A x over a single-range SELL matrix
-template <bool ACC, bool NARROW, typename VT, typename XT>
-void launchSellShape(const SellMatrix<VT>& A, const void* x, void* y, int nrhs, hipStream_t st) {
-    const unsigned g = (unsigned)std::max(1, (A.nChunk + kWavesPerBlock - 1) / kWavesPerBlock);
-    if (A.uniformW >= 0)
-        hipLaunchKernelGGL((k_sell_spmv_u<ACC, NARROW, VT, XT>), dim3(g), dim3(kBlock), 0, st, A.uniformW,
-                           A.col.p, A.val.p, (const XT*)x, (XT*)y, A.n, nrhs);
+// Where the matrix stays between calls decides how it is read.  Larger than
+// the 256 MB Infinity Cache it comes from HBM every time: non-temporal loads
+// keep x and y in the caches instead (7-point 192^3 FP64 125.5 -> 116.9 us,
+// 160^3 75.9 -> 70.6; below 256 MB they cost: 140^3 47.9 -> 50.9).  Between the
+// 32 MB of the eight L2 caches and 256 MB every XCD gets one contiguous part
+// of the rows (workgroups are dealt round-robin over the XCDs), so that an
+// x line is fetched by one L2 and not by all whose rows touch it (140^3 47.9 ->
+// 41.0 us, 100^3 20.1 -> 18.4; 27-point 96^3 40.5 -> 38.4).  Above 256 MB eight
+// such streams are slower than one (192^3 125.5 -> 134.8), below 32 MB the
+// mapping only unbalances a short launch (7-point 64^3 5.2 -> 6.1).
+constexpr long kL2Bytes = 32l << 20, kInfinityCacheBytes = 256l << 20;
+
+// one launch of y = A x or y += A x.  Right-hand sides are taken 1, 2, 4 or 8
+// at a time, the smallest block that covers them (8 for 5 to 8, blocks of 4
+// otherwise): a pass over the entries costs more than idle columns of a block.
+template <int NR, typename CT, typename VT, typename XT>
+void launchSellNr(const SellMatrix<VT>& A, const void* x, void* y, int nrhs, bool acc, hipStream_t st) {
+    const int g = std::max(1, (A.nChunk + kWavesPerBlock - 1) / kWavesPerBlock);
+    const long all = A.bytes + 2l * nrhs * A.n * (long)sizeof(XT);
+    const int perXcd = A.bytes <= kInfinityCacheBytes && all > kL2Bytes ? (g + 7) / 8 : 0;
+    const dim3 grid(perXcd ? 8 * perXcd : g);
+    if (A.bytes > kInfinityCacheBytes)
+        hipLaunchKernelGGL((k_sell<NR, true, CT, VT, XT>), grid, dim3(kBlock), 0, st, A.template view<CT>(),
+                           (const XT*)x, (XT*)y, nrhs, (int)acc, perXcd);
     else
-        hipLaunchKernelGGL((k_sell_spmv<ACC, NARROW, VT, XT>), dim3(g), dim3(kBlock), 0, st, A.chunks.p,
-                           A.nChunk, A.col.p, A.val.p, (const XT*)x, (XT*)y, (long)A.n, nrhs);
+        hipLaunchKernelGGL((k_sell<NR, false, CT, VT, XT>), grid, dim3(kBlock), 0, st, A.template view<CT>(),
+                           (const XT*)x, (XT*)y, nrhs, (int)acc, perXcd);
+}
+template <typename CT, typename VT, typename XT>
+void launchSellIds(const SellMatrix<VT>& A, const void* x, void* y, int nrhs, bool acc, hipStream_t st) {
+    if (nrhs == 1)
+        launchSellNr<1, CT, VT, XT>(A, x, y, nrhs, acc, st);
+    else if (nrhs == 2)
+        launchSellNr<2, CT, VT, XT>(A, x, y, nrhs, acc, st);
+    else if (nrhs <= 4 || (nrhs > 8 && nrhs % 8 >= 1 && nrhs % 8 <= 4))
+        launchSellNr<4, CT, VT, XT>(A, x, y, nrhs, acc, st);
+    else
+        launchSellNr<8, CT, VT, XT>(A, x, y, nrhs, acc, st);
 }
 template <bool ACC, typename VT, typename XT>
 void launchSell(const SellMatrix<VT>& A, const void* x, void* y, int nrhs, hipStream_t st) {
-    if (A.narrow())
-        launchSellShape<ACC, true, VT, XT>(A, x, y, nrhs, st);
+    if (A.narrowIds)
+        launchSellIds<uint16_t, VT, XT>(A, x, y, nrhs, ACC, st);
     else
-        launchSellShape<ACC, false, VT, XT>(A, x, y, nrhs, st);
+        launchSellIds<int, VT, XT>(A, x, y, nrhs, ACC, st);
 }
 
 // b = A x
@@ -310,7 +473,7 @@ class SymmSellFn : public DeviceFn {
         const int n = d.nrow;
         if (mode == 2) {
             if (!std::is_same<VT, double>::value || !std::is_same<XT, double>::value) return ERR_NOT_IMPLEMENTED;
-            return A.build(d, false);
+            return A.build(d);
         }
         // full pattern: row r holds its upper entries, then the transposed
         // entries (c, r) of rows c < r, each in increasing c
@@ -346,8 +509,12 @@ class SymmSellFn : public DeviceFn {
         if constexpr (std::is_same<VT, double>::value && std::is_same<XT, double>::value) {
             if (mode == 2) {
                 const unsigned g = (unsigned)std::max(1, (A.nChunk + kWavesPerBlock - 1) / kWavesPerBlock);
-                hipLaunchKernelGGL(k_sell_symm_atomic, dim3(g), dim3(kBlock), 0, st, A.chunks.p, A.nChunk,
-                                   A.col.p, A.val.p, (const double*)x, (double*)b, (long)A.n, nrhs);
+                if (A.narrowIds)
+                    hipLaunchKernelGGL(k_sell_symm_atomic<uint16_t>, dim3(g), dim3(kBlock), 0, st,
+                                       A.template view<uint16_t>(), (const double*)x, (double*)b, nrhs);
+                else
+                    hipLaunchKernelGGL(k_sell_symm_atomic<int>, dim3(g), dim3(kBlock), 0, st,
+                                       A.template view<int>(), (const double*)x, (double*)b, nrhs);
                 RACE_HIP(hipGetLastError());
                 return OK;
             }
@@ -365,8 +532,9 @@ class SymmSellFn : public DeviceFn {
 // the products and their order are the same, only the launches differ.  A
 // slope-2 wavefront over the groups (power q on group L - 2 (q - 1) in launch
 // L) was measured on 7-point 192^3, k = 8, 256 MB blocking, FP64: 100 launches,
-// 1.23 ms, against 1.02 ms for 8 launches; 27-point 33^3, k = 5, 4 MB, FP32:
-// 31 launches, 139.7 us, against 19.3 us.  The 256 MB Infinity Cache serves a
+// 1.23 ms, against 1.02 ms for 8 launches over the same SELL layout (0.95 ms
+// with packed entries); 27-point 33^3, k = 5, 4 MB, FP32: 31 launches,
+// 139.7 us, against 19.3 us.  The 256 MB Infinity Cache serves a
 // gathering SpMV little faster than HBM, so the reuse does not pay for the
 // extra launches (3-5 us each) at any size.
 //
@@ -474,27 +642,25 @@ class SpmtvFn : public DeviceFn {
 // r = b - A x (FP64 product, r stored as RT) and the sums of r^2 and b^2
 // for the refinement; grid-stride over chunks so few workgroups add to the
 // two norm accumulators
-template <typename RT, bool NARROW>
-__global__ void __launch_bounds__(kBlock) k_sell_residual(const SellChunk* __restrict__ chunks, int nChunk,
-                                                          int W, const int* __restrict__ col,
-                                                          const double* __restrict__ val,
-                                                          const double* __restrict__ x,
-                                                          const double* __restrict__ b, RT* __restrict__ r,
-                                                          long n, int nrhs, double* __restrict__ norms) {
+template <typename RT, bool NT, typename CT>
+__global__ void __launch_bounds__(kBlock) k_sell_residual(SellView<CT, double> A, const double* __restrict__ x,
+                                                          const double* __restrict__ b, RT* __restrict__ r, int nrhs,
+                                                          double* __restrict__ norms) {
     __shared__ double sr[kWavesPerBlock], sb[kWavesPerBlock];
-    const int lane = threadIdx.x % kC, wv = threadIdx.x / kC;
+    const int lane = threadIdx.x % kC, wv = __builtin_amdgcn_readfirstlane(threadIdx.x / kC);
     double rr = 0.0, bb = 0.0;
-    for (int c = blockIdx.x * kWavesPerBlock + wv; c < nChunk; c += gridDim.x * kWavesPerBlock) {
-        const SellChunk k =
-            W >= 0 ? SellChunk{c * kC, (int)std::min<long>(kC, n - (long)c * kC), W, c * W} : chunks[c];
-        const bool live = lane < k.rows;  // padding lanes compute, store nothing
-        const long row = k.row0 + (live ? lane : 0);
+    for (int c = blockIdx.x * kWavesPerBlock + wv; c < A.nChunk; c += gridDim.x * kWavesPerBlock) {
+        const int row = c * kC + lane;
+        const bool live = row < A.n;  // lanes past the last row compute, store nothing
         for (int q = 0; q < nrhs; ++q) {
-            const double t = sellRow<NARROW>(k, lane, col, val, x + q * n);
-            const double bv = b[q * n + row];
+            const long vo = (long)q * A.n;
+            const double* const xq[1] = {x + vo};
+            double t[1] = {0.0};
+            const double bv = b[vo + (live ? row : 0)];
+            sellRow<1, NT>(A, c, lane, xq, t);
             if (!live) continue;
-            const double rv = bv - t;
-            r[q * n + row] = (RT)rv;
+            const double rv = bv - t[0];
+            r[vo + row] = (RT)rv;
             rr += rv * rv;
             bb += bv * bv;
         }
@@ -521,22 +687,26 @@ class SellResidual : public ResidualOp {
   public:
     SellMatrix<double> A;
     int init(const race_kernel_desc& d) { return A.build(d); }
-    template <typename RT, bool NARROW>
+    template <typename RT, typename CT>
     void launch(const double* x, const double* b, void* r, int nrhs, double* norms, hipStream_t st) {
         const int blocks = std::max(1, std::min(4096, (A.nChunk + kWavesPerBlock - 1) / kWavesPerBlock));
-        hipLaunchKernelGGL((k_sell_residual<RT, NARROW>), dim3(blocks), dim3(kBlock), 0, st, A.chunks.p, A.nChunk,
-                           A.uniformW, A.col.p, A.val.p, x, b, (RT*)r, (long)A.n, nrhs, norms);
+        if (A.bytes > kInfinityCacheBytes)
+            hipLaunchKernelGGL((k_sell_residual<RT, true, CT>), dim3(blocks), dim3(kBlock), 0, st,
+                               A.template view<CT>(), x, b, (RT*)r, nrhs, norms);
+        else
+            hipLaunchKernelGGL((k_sell_residual<RT, false, CT>), dim3(blocks), dim3(kBlock), 0, st,
+                               A.template view<CT>(), x, b, (RT*)r, nrhs, norms);
     }
     int run(const double* x, const double* b, void* r, bool rFp32, int nrhs, double* norms,
             hipStream_t st) override {
-        if (rFp32 && A.narrow())
-            launch<float, true>(x, b, r, nrhs, norms, st);
+        if (rFp32 && A.narrowIds)
+            launch<float, uint16_t>(x, b, r, nrhs, norms, st);
         else if (rFp32)
-            launch<float, false>(x, b, r, nrhs, norms, st);
-        else if (A.narrow())
-            launch<double, true>(x, b, r, nrhs, norms, st);
+            launch<float, int>(x, b, r, nrhs, norms, st);
+        else if (A.narrowIds)
+            launch<double, uint16_t>(x, b, r, nrhs, norms, st);
         else
-            launch<double, false>(x, b, r, nrhs, norms, st);
+            launch<double, int>(x, b, r, nrhs, norms, st);
         RACE_HIP(hipGetLastError());
         return OK;
     }
