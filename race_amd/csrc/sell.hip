@@ -28,6 +28,8 @@
 
 #include "exec.hpp"
 #include "exec_common.hpp"
+#include "rowblock.hpp"
+#include "sell_common.hpp"
 
 namespace race {
 
@@ -35,28 +37,6 @@ namespace {
 
 constexpr int kC = 64;               // rows per chunk (one wavefront)
 constexpr int kWavesPerBlock = kBlock / kC;
-
-// matrix value storage (double, float, or bfloat16 bits); the arithmetic
-// runs in the vector type XT: FP64, or FP32 accumulation for FP32 / BF16
-template <typename VT>
-VT toStorage(double v) {
-    if constexpr (sizeof(VT) == 2)
-        return toBf16(v);
-    else
-        return (VT)v;
-}
-template <typename XT>
-__device__ __forceinline__ XT fromStorage(double v) {
-    return (XT)v;
-}
-template <typename XT>
-__device__ __forceinline__ XT fromStorage(float v) {
-    return (XT)v;
-}
-template <typename XT>
-__device__ __forceinline__ XT fromStorage(uint16_t v) {
-    return (XT)__uint_as_float((unsigned)v << 16);
-}
 
 // f(lo, hi) over [0, n) in contiguous parts on up to 8 host threads
 template <class F>
@@ -426,19 +406,57 @@ void launchSellIds(const SellMatrix<VT>& A, const void* x, void* y, int nrhs, bo
     else
         launchSellNr<8, CT, VT, XT>(A, x, y, nrhs, acc, st);
 }
-template <bool ACC, typename VT, typename XT>
-void launchSell(const SellMatrix<VT>& A, const void* x, void* y, int nrhs, hipStream_t st) {
+template <typename VT, typename XT>
+void launchSell(const SellMatrix<VT>& A, const void* x, void* y, int nrhs, bool acc, hipStream_t st) {
     if (A.narrowIds)
-        launchSellIds<uint16_t, VT, XT>(A, x, y, nrhs, ACC, st);
+        launchSellIds<uint16_t, VT, XT>(A, x, y, nrhs, acc, st);
     else
-        launchSellIds<int, VT, XT>(A, x, y, nrhs, ACC, st);
+        launchSellIds<int, VT, XT>(A, x, y, nrhs, acc, st);
 }
+
+// A matrix that is multiplied with vectors, in the layout its rows ask for:
+// row blocks where the chunks would store more than 5 slots for 4 entries,
+// otherwise SELL chunks.  Both measured on both sides of the line (us, SELL
+// chunks / row blocks, FP64): Chung-Lu graphs (2 to 5 slots an entry) of 150000
+// rows 111 / 22.8, 20000 rows 41.4 / 8.1; random banded (1.25 to 1.35) of 90001
+// rows, 21 entries a row 7.4 / 6.5, of 200000 rows, 40 entries 25.9 / 26.2;
+// 27-point grids (1.0 to 1.1) 64^3 13.6 / 18.7, 96^3 37.5 / 49.6.
+template <typename VT, typename XT>
+struct Product {
+    SellMatrix<VT> sell;
+    RowBlocks<VT> blocks;
+    int n = 0;
+    bool useBlocks = false;
+    int build(const race_kernel_desc& d) {
+        n = d.nrow;
+        useBlocks = ragged(d);
+        if (!useBlocks) return sell.build(d);
+        blocks.add(n, d.rowPtr, d.col, d.val, 0);
+        return blocks.finish();
+    }
+    static bool ragged(const race_kernel_desc& d) {
+        long slots = 0;
+        for (int r0 = 0; r0 < d.nrow; r0 += kC) {
+            int w = 0;
+            for (int r = r0; r < std::min(d.nrow, r0 + kC); ++r) w = std::max(w, d.rowPtr[r + 1] - d.rowPtr[r]);
+            slots += w;
+        }
+        return slots * kC * 4 > (long)d.rowPtr[d.nrow] * 5;
+    }
+    // y = A x (acc: y += A x)
+    void run(const void* x, void* y, int nrhs, bool acc, hipStream_t st) const {
+        if (useBlocks)
+            launchRowBlk<false, VT, XT>(blocks, nullptr, x, y, n, nrhs, acc, st);
+        else
+            launchSell<VT, XT>(sell, x, y, nrhs, acc, st);
+    }
+};
 
 // b = A x
 template <typename VT, typename XT>
 class SellSpmvFn : public DeviceFn {
   public:
-    SellMatrix<VT> A;
+    Product<VT, XT> A;
     int nrhs = 1;
     int init(const race_kernel_desc& d) {
         kind = d.kind;
@@ -448,7 +466,7 @@ class SellSpmvFn : public DeviceFn {
         return A.build(d);
     }
     int run(bool, hipStream_t st) override {
-        launchSell<false, VT, XT>(A, x, b, nrhs, st);
+        A.run(x, b, nrhs, false, st);
         RACE_HIP(hipGetLastError());
         return OK;
     }
@@ -462,7 +480,7 @@ class SellSpmvFn : public DeviceFn {
 template <typename VT, typename XT>
 class SymmSellFn : public DeviceFn {
   public:
-    SellMatrix<VT> A;
+    Product<VT, XT> A;
     int mode = 2, nrhs = 1;
     int init(const race_kernel_desc& d, int mode_) {
         kind = d.kind;
@@ -473,7 +491,7 @@ class SymmSellFn : public DeviceFn {
         const int n = d.nrow;
         if (mode == 2) {
             if (!std::is_same<VT, double>::value || !std::is_same<XT, double>::value) return ERR_NOT_IMPLEMENTED;
-            return A.build(d);
+            return A.sell.build(d);
         }
         // full pattern: row r holds its upper entries, then the transposed
         // entries (c, r) of rows c < r, each in increasing c
@@ -508,18 +526,18 @@ class SymmSellFn : public DeviceFn {
     int run(bool, hipStream_t st) override {
         if constexpr (std::is_same<VT, double>::value && std::is_same<XT, double>::value) {
             if (mode == 2) {
-                const unsigned g = (unsigned)std::max(1, (A.nChunk + kWavesPerBlock - 1) / kWavesPerBlock);
-                if (A.narrowIds)
+                const unsigned g = (unsigned)std::max(1, (A.sell.nChunk + kWavesPerBlock - 1) / kWavesPerBlock);
+                if (A.sell.narrowIds)
                     hipLaunchKernelGGL(k_sell_symm_atomic<uint16_t>, dim3(g), dim3(kBlock), 0, st,
-                                       A.template view<uint16_t>(), (const double*)x, (double*)b, nrhs);
+                                       A.sell.template view<uint16_t>(), (const double*)x, (double*)b, nrhs);
                 else
                     hipLaunchKernelGGL(k_sell_symm_atomic<int>, dim3(g), dim3(kBlock), 0, st,
-                                       A.template view<int>(), (const double*)x, (double*)b, nrhs);
+                                       A.sell.template view<int>(), (const double*)x, (double*)b, nrhs);
                 RACE_HIP(hipGetLastError());
                 return OK;
             }
         }
-        launchSell<true, VT, XT>(A, x, b, nrhs, st);
+        A.run(x, b, nrhs, true, st);
         RACE_HIP(hipGetLastError());
         return OK;
     }
@@ -547,7 +565,7 @@ class SymmSellFn : public DeviceFn {
 template <typename VT, typename XT>
 class MpkFn : public DeviceFn {
   public:
-    SellMatrix<VT> A;
+    Product<VT, XT> A;
     int nslot = 2;
     int init(const race_kernel_desc& d, const ExecContext& ctx) {
         kind = d.kind;
@@ -590,8 +608,7 @@ class MpkFn : public DeviceFn {
         const int steps = power * subPower;
         if (steps < 1 || steps > powerMax) return ERR_INVALID_ARG;
         for (int q = 1; q <= steps; ++q)
-            launchSell<false, VT, XT>(A, (const XT*)x + (size_t)((q - 1) % nslot) * A.n,
-                                      (XT*)x + (size_t)(q % nslot) * A.n, 1, st);
+            A.run((const XT*)x + (size_t)((q - 1) % nslot) * A.n, (XT*)x + (size_t)(q % nslot) * A.n, 1, false, st);
         RACE_HIP(hipGetLastError());
         return OK;
     }
@@ -607,7 +624,7 @@ class MpkFn : public DeviceFn {
 template <typename VT, typename XT>
 class SpmtvFn : public DeviceFn {
   public:
-    SellMatrix<VT> A;
+    Product<VT, XT> A;
     int nrhs = 1;
     int init(const race_kernel_desc& d) {
         kind = d.kind;
@@ -633,7 +650,7 @@ class SpmtvFn : public DeviceFn {
         return A.build(t);
     }
     int run(bool, hipStream_t st) override {
-        launchSell<true, VT, XT>(A, x, b, nrhs, st);
+        A.run(x, b, nrhs, true, st);
         RACE_HIP(hipGetLastError());
         return OK;
     }
@@ -790,7 +807,12 @@ static void expandUpper(const race_kernel_desc& d, std::vector<int>& rp, std::ve
 }
 
 // SpMV (b = A x) or SymmSpMV (b += A x, expanded from the upper triangle)
-// on a batch of matrices in one launch.
+// on a batch of matrices: one launch over the SELL chunks of all matrices
+// that fit the layout, one over the row blocks of those whose chunks would
+// store more than 5 slots for 4 entries (Product's rule) or be wider than 64
+// entries: with 8 right-hand sides a chunk holding a hub row runs its up to
+// 400 steps once per right-hand side.  16 matrices of 2000 to 40000 rows, FP32,
+// 8 right-hand sides: 864 us in chunks alone, 124 us.
 template <typename XT>
 class SellBatchFn : public DeviceFn {
   public:
@@ -801,6 +823,8 @@ class SellBatchFn : public DeviceFn {
     DevBuf<XT> val;
     DevBuf<const XT*> mx;
     DevBuf<XT*> my;
+    RowBlocks<XT> blocks;
+    DevBuf<RowBlkVecs> vecs;
 
     int init(const std::vector<BatchItem>& items, const ExecContext& ctx) {
         kind = items[0].d.kind;
@@ -814,6 +838,7 @@ class SellBatchFn : public DeviceFn {
         std::vector<XT> hval;
         std::vector<const XT*> hx;
         std::vector<XT*> hy;
+        std::vector<RowBlkVecs> hv;
         std::vector<int> rp, fc, order;
         std::vector<double> fv;
         for (size_t m = 0; m < items.size(); ++m) {
@@ -837,6 +862,22 @@ class SellBatchFn : public DeviceFn {
                         return R[a + 1] - R[a] > R[b + 1] - R[b];
                     });
                 }
+            long slots = 0;
+            int widest = 0;
+            for (int r0 = 0; r0 < n; r0 += C) {
+                int w = 0;
+                for (int r = r0; r < std::min(n, r0 + C); ++r) w = std::max(w, R[order[r] + 1] - R[order[r]]);
+                slots += (long)w * C;
+                widest = std::max(widest, w);
+            }
+            hx.push_back((const XT*)d.x);
+            hy.push_back((XT*)d.b);
+            hn.push_back(n);
+            hv.push_back(RowBlkVecs{d.x, d.b, n});
+            if (widest > 64 || slots * 4 > (long)R[n] * 5) {
+                blocks.add(n, R, Cc, V, (int)m);
+                continue;
+            }
             for (int r0 = 0; r0 < n; r0 += C) {
                 const int rows = std::min(C, n - r0);
                 int w = 0;
@@ -857,12 +898,11 @@ class SellBatchFn : public DeviceFn {
                     if (perm && i < rows) hrow.push_back(r);
                 }
             }
-            hx.push_back((const XT*)d.x);
-            hy.push_back((XT*)d.b);
-            hn.push_back(n);
         }
         nChunk = (int)hc.size();
         int e;
+        if ((e = blocks.finish())) return e;
+        if ((e = upload(vecs, hv.data(), hv.size()))) return e;
         if ((e = upload(chunks, hc.data(), hc.size()))) return e;
         if ((e = upload(rowOf, hrow.data(), hrow.size()))) return e;
         if ((e = upload(col, hcol.data(), hcol.size()))) return e;
@@ -883,7 +923,15 @@ class SellBatchFn : public DeviceFn {
             hipLaunchKernelGGL((k_sellg_spmv<CC, P, XT, false>), dim3(g), dim3(kBlock), 0, st, chunks.p, nChunk,
                                rowOf.p, col.p, val.p, mx.p, my.p, mn.p, nrhs);
     }
+    int launches(bool) const override { return (nChunk > 0) + (blocks.nBlk > 0); }
     int run(bool, hipStream_t st) override {
+        if (blocks.nBlk > 0)
+            launchRowBlk<true, XT, XT>(blocks, vecs.p, nullptr, nullptr, 0, nrhs, kind == RACE_K_SYMMSPMV, st);
+        if (nChunk > 0) runChunks(st);
+        RACE_HIP(hipGetLastError());
+        return OK;
+    }
+    void runChunks(hipStream_t st) {
         switch (C * 2 + (perm ? 1 : 0)) {
             case 16: launch<8, false>(st); break;
             case 17: launch<8, true>(st); break;
@@ -894,8 +942,6 @@ class SellBatchFn : public DeviceFn {
             case 128: launch<64, false>(st); break;
             default: launch<64, true>(st); break;
         }
-        RACE_HIP(hipGetLastError());
-        return OK;
     }
 };
 

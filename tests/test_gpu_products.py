@@ -127,3 +127,36 @@ def test_infinity_stays_in_its_rows():
     ce.executeFunction(fid)
     touched = np.array([np.isinf(x[col[rp[r]:rp[r + 1]]]).any() for r in range(n)])
     assert np.array_equal(np.isinf(db.download()), touched) and not np.isnan(db.download()).any()
+
+
+RAGGED = {
+    # blocks of one, two and three rows, exactly and just over 1024 entries
+    "one_row_blocks": [1024, 1, 1023, 1025, 3000, 0, 5],
+    "two_and_three": [512, 512, 341, 342, 341, 600, 424, 1],
+    # more empty rows than a block holds, at the start and at the end
+    "empty_ends": [0] * 300 + [40] + [0] * 600,
+    "all_empty": [0] * 700,
+    # a block that ends by its row count, and hub rows among short ones
+    "short_rows": [1, 0, 2] * 200 + [900] + [3] * 50,
+}
+
+
+@pytest.mark.parametrize("kind", [R.K_SPMV, R.K_SPMTV])
+@pytest.mark.parametrize("name", sorted(RAGGED))
+def test_row_blocks(name, kind):
+    lengths = RAGGED[name]
+    lengths = lengths + [1] * max(0, 3100 - len(lengths)) if max(lengths) > 900 else lengths
+    for prec, nrhs in ((R.FP64, 1), (R.FP32, 1), (R.BF16, 1), (R.FP64, 3), (R.FP32, 2), (R.FP32, 8), (R.BF16, 11)):
+        print("case ragged", name, kind, prec, nrhs, flush=True)
+        _check(*_random(len(lengths), lengths, len(name)), kind, prec, nrhs)
+
+
+def test_row_blocks_wide_ids():
+    """ragged rows over more than 65535 columns: 32-bit ids"""
+    n = 200000
+    lengths = [(r % 97 == 0) * 60 + r % 3 for r in range(n)]
+    rng = np.random.default_rng(4)
+    rp = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int32)
+    col = rng.integers(0, n, rp[-1]).astype(np.int32)
+    for prec, nrhs in ((R.FP64, 1), (R.FP32, 4)):
+        _check(rp, col, rng.uniform(-1, 1, len(col)), R.K_SPMV, prec, nrhs)
