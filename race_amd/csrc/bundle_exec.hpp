@@ -1,4 +1,8 @@
-// bundle_exec.hip -- Gauss-Seidel and Kaczmarz over leaf bundles.
+// bundle_exec.hpp -- Gauss-Seidel and Kaczmarz over leaf bundles.
+//
+// Included once per pair of value and vector type (bundle_f64.hip,
+// bundle_f32.hip, bundle_bf16.hip), so that the instantiations compile in
+// parallel.
 //
 // One workgroup runs one bundle (a run of whole, mutually independent
 // leaves of one colour phase).  TPR lanes share a row; each lane keeps E
@@ -7,6 +11,7 @@
 // leaves (rows of equal depth in RACE's sequential leaf order) run one after
 // the other with a workgroup barrier in between.  Only the prologue touches
 // HBM: the entry block, the outside columns of x, and the write-back.
+#pragma once
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -17,6 +22,7 @@
 #include <type_traits>
 
 #include "bundle.hpp"
+#include "bundle_make.hpp"
 #include "exec.hpp"
 #include "exec_common.hpp"
 
@@ -91,6 +97,67 @@ __device__ __forceinline__ int bundleOfBlock(int nbnd, int xcd) {
 
 // the lane of a row that reads and writes its x (the first of its lanes)
 __device__ __forceinline__ bool own(bool active, int lane) { return active && lane == 0; }
+
+// ---------------------------------------------------------------------------
+// The dependency waves of a bundle.  Slots are sorted by wave, so the lanes of
+// a wave are contiguous and each wavefront holds a contiguous range of waves.
+// A wavefront's LDS accesses execute in order, so waves that lie inside one
+// wavefront need no workgroup barrier between them: only that wavefront runs
+// them while the others wait at the next barrier.  A wave spread over several
+// wavefronts is run by all of them between two barriers.  That is at most two
+// barriers per wavefront of the workgroup instead of two per wave.  A wave is
+// bound by its chain of LDS reads, products, the sum over the lanes of a row
+// and LDS writes.  Used with variable lanes per row, whose waves needed two
+// barriers and a serial sum: a forward Kaczmarz sweep over a Chung-Lu graph of
+// 36425 rows (one chain of 7009 waves), FP32, 6.76 ms before, 4.34 ms with this,
+// rowSum and the batched column gathers.  Not used with uniform lanes, where one
+// barrier per wave is cheaper than finding the spans for some ten waves a
+// launch (Gauss-Seidel, 27-point 14^3: 124.3 us a step, 143.3 us with spans).
+//
+// WaveSpans: first and last wave of every wavefront, in LDS; set before a
+// barrier and read by runWaves after it.
+template <int NW>
+struct WaveSpans {
+    int first[NW], last[NW];
+};
+template <int NW>
+__device__ __forceinline__ void setSpans(WaveSpans<NW>& sp, bool active, int myWave) {
+    const unsigned long long m = __ballot(active);
+    const int v = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    // active lanes are the first of their wavefront
+    const int end = 64 - (m ? __clzll((long long)m) : 64);
+    if (lane == 0) sp.first[v] = m ? myWave : INT32_MAX;
+    if (lane == (m ? end - 1 : 0)) sp.last[v] = m ? myWave : -1;
+}
+// row(w, spread) runs wave w on the lanes that belong to it; spread: several
+// wavefronts run it at once and every thread of the workgroup calls it (it
+// may hold barriers then).  Ends with a barrier if the bundle has any wave.
+template <int NW, class Row>
+__device__ __forceinline__ void runWaves(const WaveSpans<NW>& sp, int nw, Row&& row) {
+    const int me = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int lf = lane < NW ? sp.first[lane] : INT32_MAX, ll = lane < NW ? sp.last[lane] : -1;
+    int next = 0;
+    for (int v = 0; v < NW && next < nw;) {
+        const int vl = __builtin_amdgcn_readlane(ll, v);
+        if (vl < next) {
+            ++v;
+            continue;
+        }
+        // waves of v alone, then the one it shares with its successors
+        const bool shares = v + 1 < NW && __builtin_amdgcn_readlane(lf, v + 1) == vl;
+        const bool spread = shares && next == vl;
+        const int end = spread ? vl : shares ? vl - 1 : vl;
+        if (spread || me == v)
+            for (int w = next; w <= end; ++w) {
+                row(w, spread);
+                // the next wave's reads stay behind this one's writes
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+            }
+        next = end + 1;
+        __syncthreads();
+    }
+}
 
 // Vectors of a bundle: the launch's x, b and n, or, for a batch of matrices
 // (BATCH), the bundle's own (each matrix keeps its vectors).
@@ -417,82 +484,154 @@ __global__ void __launch_bounds__(BS) k_gs_flow(
     }
 }
 
-// Loads and stores of x in a bundle body.  FLOW: the column id may carry
+// Loads and stores of x in a Kaczmarz chain.  FLOW: the column id may carry
 // bit 31 (written earlier in the one-launch sweep: read coherently), and
 // every store is coherent; otherwise plain accesses.
 template <bool FLOW, typename XT>
-__device__ __forceinline__ XT ldX(const XT* x, size_t vo, unsigned id) {
+__device__ __forceinline__ XT ldX(const XT* x, unsigned id) {
     if constexpr (FLOW) {
-        const XT* p = x + vo + (id & 0x7fffffffu);
+        const XT* p = x + (id & 0x7fffffffu);
         return (id >> 31) ? ldCoh(p) : *p;
     } else {
-        return x[vo + id];
+        return x[id];
     }
 }
 template <bool FLOW, typename XT>
-__device__ __forceinline__ void stX(XT* x, size_t vo, unsigned id, XT v) {
+__device__ __forceinline__ void stX(XT* x, unsigned id, XT v) {
     if constexpr (FLOW)
-        stCoh(x + vo + (id & 0x7fffffffu), v);
+        stCoh(x + (id & 0x7fffffffu), v);
     else
-        x[vo + id] = v;
+        x[id] = v;
 }
-// nothing to wait for (the phase launches)
-struct NoWait {
-    __device__ __forceinline__ void operator()() const {}
-};
 
-// Kaczmarz: every column the bundle touches lives in LDS; rows of one wave
-// share no column.  The row norms stay FP64.  One bundle for the right-hand
-// sides [k0, k1); wait() runs between the prologue's matrix loads and the
-// gathers of x.
-template <int BS, int TPR, int E, typename VT, typename XT, bool BATCH, bool FLOW, class Wait>
-__device__ __forceinline__ void kaczBundle(
-    const int bnd, const int k0, const int k1, XT* xl, Wait&& wait, const int* __restrict__ bSlot,
+// The local columns of a Kaczmarz bundle.  Each thread holds the ids of up to
+// kColSlots columns (a bundle has at most 6144 by default, 4096 of them in one
+// batch of 512 threads), so that all gathers of x are in flight together: one
+// column per thread and round cost two dependent memory round trips per round,
+// and the bundles of a long leaf have 4000 to 6000 columns
+// (the graph of WaveSpans: 6.02 -> 5.60 ms).
+constexpr int kColSlots = 8;
+template <int BS>
+__device__ __forceinline__ void loadCols(const int* __restrict__ ext, int e0, int ne, unsigned (&ex)[kColSlots]) {
+    const int t = threadIdx.x;
+#pragma unroll
+    for (int k = 0; k < 2; ++k) ex[k] = (unsigned)ext[t + k * BS < ne ? e0 + t + k * BS : 0];
+    if (ne > 2 * BS)
+#pragma unroll
+        for (int k = 2; k < kColSlots; ++k) ex[k] = (unsigned)ext[t + k * BS < ne ? e0 + t + k * BS : 0];
+}
+// x of the columns: to g first (issued together), then to LDS
+template <int BS, bool FLOW, typename XT>
+__device__ __forceinline__ void gatherCols(const XT* x, int ne, const unsigned (&ex)[kColSlots], XT (&g)[kColSlots]) {
+    const int t = threadIdx.x;
+    auto slots = [&](auto k0, auto k1) {
+#pragma unroll
+        for (int k = k0; k < k1; ++k) g[k] = x[t + k * BS < ne && !(FLOW && ex[k] >> 31) ? ex[k] : 0u];
+        if constexpr (FLOW)
+#pragma unroll
+            for (int k = k0; k < k1; ++k)
+                if (t + k * BS < ne && ex[k] >> 31) g[k] = ldCoh(&x[ex[k] & 0x7fffffffu]);
+    };
+    slots(std::integral_constant<int, 0>{}, std::integral_constant<int, 2>{});
+    if (ne > 2 * BS) slots(std::integral_constant<int, 2>{}, std::integral_constant<int, kColSlots>{});
+}
+template <int BS, bool FLOW, typename XT>
+__device__ __forceinline__ void placeCols(const XT* x, const int* __restrict__ ext, int e0, int ne,
+                                          const XT (&g)[kColSlots], XT* xl) {
+    const int t = threadIdx.x;
+#pragma unroll
+    for (int k = 0; k < kColSlots; ++k)
+        if (t + k * BS < ne) xl[t + k * BS] = g[k];
+    for (int c = t + kColSlots * BS; c < ne; c += BS) xl[c] = ldX<FLOW>(x, (unsigned)ext[e0 + c]);
+}
+template <int BS, bool FLOW, typename XT>
+__device__ __forceinline__ void storeCols(XT* x, const int* __restrict__ ext, int e0, int ne,
+                                          const unsigned (&ex)[kColSlots], const XT* xl) {
+    const int t = threadIdx.x;
+#pragma unroll
+    for (int k = 0; k < kColSlots; ++k)
+        if (t + k * BS < ne) stX<FLOW>(x, ex[k], xl[t + k * BS]);
+    for (int c = t + kColSlots * BS; c < ne; c += BS) stX<FLOW>(x, (unsigned)ext[e0 + c], xl[c]);
+}
+
+// The quotient d / rn by the row norm of which inv is the reciprocal: a
+// division costs a wave's chain some twenty dependent FP64 operations, this
+// three.  One Newton step makes it as exact as the division; a norm whose
+// reciprocal is not finite is divided by.  For FP32 vectors the product alone
+// is exact beyond the rounding to FP32.
+template <typename XT>
+__device__ __forceinline__ XT rowScale(double d, double rn, double inv) {
+    const double q = d * inv;
+    if constexpr (sizeof(XT) == 4) return (XT)q;
+    if (!(inv <= 1.7976931348623157e308)) return (XT)(d / rn);
+    const double c = __builtin_fma(__builtin_fma(-q, rn, d), inv, q);
+    return (XT)(c == c ? c : q);  // an infinite quotient has no remainder
+}
+
+// Kaczmarz, the bundles [cLo, cHi) of a chain for right-hand side k: every
+// column a bundle touches lives in LDS; rows of one wave share no column.  The
+// row norms stay FP64.  The next bundle's offsets, column ids and row ids are
+// requested before the current one's waves run, so that a bundle starts with
+// the gathers of x and the entries.
+template <int BS, int TPR, int E, typename VT, typename XT, bool BATCH, bool FLOW>
+__device__ __forceinline__ void kaczChain(
+    const int cLo, const int cHi, const int k, XT* xl, const int spare, const int* __restrict__ bSlot,
     const int* __restrict__ bWave, const long* __restrict__ bOff, const int* __restrict__ bLen,
     const int* __restrict__ bExt, const uint16_t* __restrict__ slotWave, const int* __restrict__ rowId,
     const double* __restrict__ rowNorm, const int* __restrict__ ext, const uint16_t* __restrict__ sidx,
     const VT* __restrict__ sval, long zero, XT* x0, const XT* __restrict__ b0, int n0, XT* const* __restrict__ bX,
     const XT* const* __restrict__ bB, const int* __restrict__ bN) {
-    const BundleVec<BATCH, XT> vec(x0, b0, n0, bX, bB, bN, bnd);
-    XT* __restrict__ x = vec.x;
-    const XT* __restrict__ b = vec.b;
-    const int n = vec.n;
-    const int s0 = bSlot[bnd], nb = bSlot[bnd + 1] - s0;
-    const long off = bOff[bnd];
-    const int wb = bLen[bnd];
-    const int nw = bWave[bnd + 1] - bWave[bnd];
-    const int e0 = bExt[bnd], ne = bExt[bnd + 1] - e0;
-    const int t = threadIdx.x, i = t / TPR, l = t % TPR;
-    const bool active = i < nb;
-    const long lanes = (long)nb * TPR;
-    (void)l;
+    if (cLo >= cHi) return;
+    const BundleVec<BATCH, XT> vec(x0, b0, n0, bX, bB, bN, cLo);
+    const size_t vo = (size_t)k * vec.n;
+    XT* __restrict__ x = vec.x + vo;
+    const XT* __restrict__ b = vec.b + vo;
+    const int t = threadIdx.x, i = t / TPR;
 
-    // branch-free prologue, ids first (as in k_gs_bundle)
-    const int sr = active ? s0 + i : 0;
-    const unsigned row = (unsigned)rowId[sr];
-    const unsigned ex0 = (unsigned)ext[t < ne ? e0 + t : 0];
-    const unsigned ex1 = (unsigned)ext[t + BS < ne ? e0 + t + BS : 0];
-    int li[E];
-    typename ValBits<VT>::T lv[E];
+    int s0 = bSlot[cLo], nb = bSlot[cLo + 1] - s0;
+    int e0 = bExt[cLo], ne = bExt[cLo + 1] - e0;
+    unsigned ex[kColSlots], row = (unsigned)rowId[i < nb ? s0 + i : 0];
+    loadCols<BS>(ext, e0, ne, ex);
+    for (int bnd = cLo;;) {
+        const long off = bOff[bnd];
+        const int wb = bLen[bnd];
+        const int nw = bWave[bnd + 1] - bWave[bnd];
+        const bool active = i < nb;
+        const long lanes = (long)nb * TPR;
+        // branch-free entry loads (as in k_gs_bundle)
+        const int sr = active ? s0 + i : 0;
+        int li[E];
+        typename ValBits<VT>::T lv[E];
 #pragma unroll
-    for (int u = 0; u < E; ++u) {
-        const long e = (active && u < wb) ? off + (long)u * lanes + t : zero;
-        li[u] = (int)sidx[e];
-        lv[u] = sval[e];
-    }
-    const double rn = rowNorm[sr];
-    const int myWave = (int)slotWave[sr];
-    wait();
-
-    for (int k = k0; k < k1; ++k) {
-        const size_t vo = (size_t)k * n;
-        const XT g0 = ldX<FLOW>(x, vo, t < ne ? ex0 : 0u);
-        const XT g1 = ldX<FLOW>(x, vo, t + BS < ne ? ex1 : 0u);
-        const XT br = b[vo + (active ? row : 0u)];
-        if (t < ne) xl[t] = g0;
-        if (t + BS < ne) xl[t + BS] = g1;
-        for (int c = t + 2 * BS; c < ne; c += BS) xl[c] = ldX<FLOW>(x, vo, (unsigned)ext[e0 + c]);
+        for (int u = 0; u < E; ++u) {
+            const long e = (active && u < wb) ? off + (long)u * lanes + t : zero;
+            li[u] = (int)sidx[e];
+            lv[u] = sval[e];
+        }
+        const double rn = rowNorm[sr];
+        const int myWave = (int)slotWave[sr];
+        XT g[kColSlots];
+        gatherCols<BS, FLOW>(x, ne, ex, g);
+        const XT br = b[active ? row : 0u];
+        placeCols<BS, FLOW>(x, ext, e0, ne, g, xl);
+        // behind the gathers, as these wait for the entries
+        const double rnInv = 1.0 / rn;
+        // where an entry's update goes: an entry of value 0 (a padding entry
+        // may name a column another row updates) to a spare place behind the
+        // columns
+        int lw[E];
+#pragma unroll
+        for (int u = 0; u < E; ++u) lw[u] = valOf<XT>(lv[u]) != XT(0) ? li[u] : ne + (t & (spare - 1));
         __syncthreads();
+        const bool more = bnd + 1 < cHi;
+        int s0n = 0, nbn = 0, e0n = 0, nen = 0;
+        unsigned exn[kColSlots] = {}, rown = 0;
+        if (more) {
+            s0n = bSlot[bnd + 1], nbn = bSlot[bnd + 2] - s0n;
+            e0n = bExt[bnd + 1], nen = bExt[bnd + 2] - e0n;
+            rown = (unsigned)rowId[i < nbn ? s0n + i : 0];
+            loadCols<BS>(ext, e0n, nen, exn);
+        }
         for (int w = 0; w < nw; ++w) {
             if (active && myWave == w) {
                 // the row's x entries, read once in one batch (no other
@@ -500,25 +639,28 @@ __device__ __forceinline__ void kaczBundle(
                 XT cur[E];
 #pragma unroll
                 for (int u = 0; u < E; ++u) cur[u] = xl[li[u]];
-                XT dot = XT(0);
+                // two partial sums: half the dependent FMA chain
+                XT sa = XT(0), sb = XT(0);
 #pragma unroll
-                for (int u = 0; u < E; ++u) dot += valOf<XT>(lv[u]) * cur[u];
-                dot = laneSum<TPR>(dot);
-                const XT scale = (XT)(((double)dot - (double)br) / rn);
-                // write back the entries with a nonzero value only: a
-                // padding entry may name a column another row updates
-#pragma unroll
-                for (int u = 0; u < E; ++u) {
-                    const XT a = valOf<XT>(lv[u]);
-                    if (a != XT(0)) xl[li[u]] = cur[u] - scale * a;
+                for (int u = 0; u + 1 < E; u += 2) {
+                    sa += valOf<XT>(lv[u]) * cur[u];
+                    sb += valOf<XT>(lv[u + 1]) * cur[u + 1];
                 }
+                if (E % 2) sa += valOf<XT>(lv[E - 1]) * cur[E - 1];
+                const XT dot = laneSum<TPR>(sa + sb);
+                const XT scale = rowScale<XT>((double)dot - (double)br, rn, rnInv);
+#pragma unroll
+                for (int u = 0; u < E; ++u) xl[lw[u]] = cur[u] - scale * valOf<XT>(lv[u]);
             }
             __syncthreads();
         }
-        if (t < ne) stX<FLOW>(x, vo, ex0, xl[t]);
-        if (t + BS < ne) stX<FLOW>(x, vo, ex1, xl[t + BS]);
-        for (int c = t + 2 * BS; c < ne; c += BS) stX<FLOW>(x, vo, (unsigned)ext[e0 + c], xl[c]);
+        storeCols<BS, FLOW>(x, ext, e0, ne, ex, xl);
         __syncthreads();
+        if (!more) break;
+        ++bnd;
+        s0 = s0n, nb = nbn, e0 = e0n, ne = nen, row = rown;
+#pragma unroll
+        for (int q = 0; q < kColSlots; ++q) ex[q] = exn[q];
     }
 }
 
@@ -529,34 +671,18 @@ __global__ void __launch_bounds__(BS) k_kacz_bundle(
     const int* __restrict__ rowId, const double* __restrict__ rowNorm, const int* __restrict__ ext,
     const uint16_t* __restrict__ sidx, const VT* __restrict__ sval, long zero, XT* __restrict__ x0,
     const XT* __restrict__ b0, int n0, int nrhs, const int* __restrict__ chainPtr, int chain0, int nchain, int xcd,
-    int ldsLocal,
-    XT* const* __restrict__ bX, const XT* const* __restrict__ bB, const int* __restrict__ bN) {
+    int spare, XT* const* __restrict__ bX, const XT* const* __restrict__ bB, const int* __restrict__ bN) {
     extern __shared__ __align__(16) unsigned char smem[];
     XT* xl = reinterpret_cast<XT*>(smem);
-    (void)ldsLocal;
 
     const int q = bundleOfBlock(nchain, xcd);
     if (q < 0) return;
     // a chain: one bundle, or the segments of a leaf too large for one bundle,
     // run in order (each segment reads what the previous one wrote)
     const int cLo = chainPtr[chain0 + q], cHi = chainPtr[chain0 + q + 1];
-    // right-hand sides are independent: grid.y splits them over workgroups
-    const int k0 = (int)blockIdx.y;
-    const int k1 = gridDim.y > 1 ? k0 + 1 : nrhs;
-    auto runBundle = [&](const int bnd) {
-        kaczBundle<BS, TPR, E, VT, XT, BATCH, false>(bnd, k0, k1, xl, NoWait{}, bSlot, bWave, bOff, bLen, bExt,
-                                                       slotWave, rowId, rowNorm, ext, sidx, sval, zero, x0, b0, n0,
-                                                       bX, bB, bN);
-    };
-    // the common case, one bundle per workgroup, as its own straight-line copy
-    if (cHi == cLo + 1) {
-        runBundle(cLo);
-    } else {
-        for (int bnd = cLo; bnd < cHi; ++bnd) {
-            runBundle(bnd);
-            __syncthreads();
-        }
-    }
+    // right-hand sides are independent: one per grid.y
+    kaczChain<BS, TPR, E, VT, XT, BATCH, false>(cLo, cHi, (int)blockIdx.y, xl, spare, bSlot, bWave, bOff, bLen, bExt,
+                                                slotWave, rowId, rowNorm, ext, sidx, sval, zero, x0, b0, n0, bX, bB, bN);
 }
 
 // Readiness-driven one-launch sweep.  A workgroup takes a queue position
@@ -615,8 +741,7 @@ __device__ __forceinline__ void readyLoop(const ReadyTables& r, Body&& body) {
         const int c = __builtin_amdgcn_readfirstlane(sChain);
         if (c < 0) break;
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-        const int cLo = r.lo[c], cHi = r.hi[c];
-        for (int bnd = cLo; bnd < cHi; ++bnd) body(bnd, NoWait{});
+        body(r.lo[c], r.hi[c]);
         // every wave's stores of x are complete before any successor is released
         __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
@@ -652,24 +777,70 @@ __global__ void __launch_bounds__(BS) k_kacz_flow(
     const int* __restrict__ bLen, const int* __restrict__ bExt, const uint16_t* __restrict__ slotWave,
     const int* __restrict__ rowId, const double* __restrict__ rowNorm, const int* __restrict__ ext,
     const uint16_t* __restrict__ sidx, const VT* __restrict__ sval, long zero, XT* x0, const XT* __restrict__ b0,
-    int n0, XT* const* __restrict__ bX, const XT* const* __restrict__ bB, const int* __restrict__ bN,
+    int n0, int spare, XT* const* __restrict__ bX, const XT* const* __restrict__ bB, const int* __restrict__ bN,
     ReadyTables rt) {
     extern __shared__ __align__(16) unsigned char smem[];
     XT* xl = reinterpret_cast<XT*>(smem);
     const int k = (int)blockIdx.y;
-    readyLoop<BS>(rt, [&](int bnd, auto wait) {
-        kaczBundle<BS, TPR, E, VT, XT, BATCH, true>(bnd, k, k + 1, xl, wait, bSlot, bWave, bOff, bLen, bExt,
-                                                      slotWave, rowId, rowNorm, ext, sidx, sval, zero, x0, b0, n0,
-                                                      bX, bB, bN);
+    readyLoop<BS>(rt, [&](int cLo, int cHi) {
+        kaczChain<BS, TPR, E, VT, XT, BATCH, true>(cLo, cHi, k, xl, spare, bSlot, bWave, bOff, bLen, bExt, slotWave,
+                                                   rowId, rowNorm, ext, sidx, sval, zero, x0, b0, n0, bX, bB, bN);
     });
+}
+
+// v of the lane that the DPP control names; 0 where there is none (MASK: the
+// 16-lane rows that take part)
+template <int CTRL, int MASK>
+__device__ __forceinline__ float dppMove(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, MASK, 0xF, false));
+}
+template <int CTRL, int MASK>
+__device__ __forceinline__ double dppMove(double v) {
+    const unsigned long long u = (unsigned long long)__double_as_longlong(v);
+    const unsigned lo = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)u, CTRL, MASK, 0xF, false);
+    const unsigned hi = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)(u >> 32), CTRL, MASK, 0xF, false);
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
+// The sum over the lanes [lo, hi) of a row, for all of them, in a fixed order
+// without atomics; lanes of rows that are not summed now pass mine = false.
+// A row inside one wavefront: a segmented scan with DPP moves (VALU, no LDS
+// round trips), whose last lane's total goes to the others (the graph of
+// WaveSpans: 5.60 ms with a tree of LDS shuffles, 4.36 with this).  Rows of a
+// wave spread over wavefronts: through LDS, with a barrier for every thread.
+template <typename XT>
+__device__ __forceinline__ XT rowSum(bool mine, bool spread, XT v, XT* part, int lo, int hi) {
+    const int t = threadIdx.x;
+    if (!spread) {
+        const int lane = t & 63, l0 = mine ? lo & 63 : 64;
+        XT u;
+        u = dppMove<0x111, 0xF>(v);  // row_shr:1, 2, 4, 8: inside 16 lanes
+        v += lane - 1 >= l0 ? u : XT(0);
+        u = dppMove<0x112, 0xF>(v);
+        v += lane - 2 >= l0 ? u : XT(0);
+        u = dppMove<0x114, 0xF>(v);
+        v += lane - 4 >= l0 ? u : XT(0);
+        u = dppMove<0x118, 0xF>(v);
+        v += lane - 8 >= l0 ? u : XT(0);
+        u = dppMove<0x142, 0xA>(v);  // row_bcast:15: lane 15 to 16-31, 47 to 48-63
+        v += (lane & 48) > l0 ? u : XT(0);
+        u = dppMove<0x143, 0xC>(v);  // row_bcast:31: lane 31 to 32-63
+        v += (lane & 32) > l0 ? u : XT(0);
+        return __shfl(v, mine ? (hi - 1) & 63 : 0);
+    }
+    if (mine) part[t] = v;
+    __syncthreads();
+    XT s = XT(0);
+    if (mine)
+        for (int l = lo; l < hi; ++l) s += part[l];
+    return s;
 }
 
 // ---------------------------------------------------------------------------
 // Variable lanes per row (matrices with a few very long rows): the row of
 // slot i owns lanes [lane0(i), lane0(i+1)) of the bundle, each holding up to
-// kVarE entries in registers.  Every lane stores its partial sum in LDS and
-// the row's sum is read back in lane order (deterministic, no atomics), so
-// every wave takes two barriers.
+// kVarE entries in registers, and the lanes of a row add up their partial sums
+// (rowSum).
 template <int BS, typename VT, typename XT, bool BATCH>
 __global__ void __launch_bounds__(BS) k_gs_bundle_vl(
     const int* __restrict__ bSlot, const int* __restrict__ bWave, const long* __restrict__ bOff,
@@ -681,6 +852,7 @@ __global__ void __launch_bounds__(BS) k_gs_bundle_vl(
     XT* const* __restrict__ bX, const XT* const* __restrict__ bB, const int* __restrict__ bN) {
     constexpr int E = kVarE;
     extern __shared__ __align__(16) unsigned char smem[];
+    __shared__ WaveSpans<BS / 64> spans;
     XT* xl = reinterpret_cast<XT*>(smem);
     XT* part = xl + ldsLocal;                               // BS partial sums
     int* rl0 = reinterpret_cast<int*>(part + BS);           // row -> first lane
@@ -734,6 +906,7 @@ __global__ void __launch_bounds__(BS) k_gs_bundle_vl(
             const XT g1 = x[vo + (t + BS < ne ? ex1 : 0u)];
             const XT gr = x[vo + (first ? row : 0u)];
             const XT br = b[vo + (first ? row : 0u)];
+            if (k == k0) setSpans(spans, active, myWave);
             if (t < ne) xl[nb + t] = g0;
             if (t + BS < ne) xl[nb + t + BS] = g1;
             if (first) xl[i] = gr;
@@ -743,21 +916,21 @@ __global__ void __launch_bounds__(BS) k_gs_bundle_vl(
                 rowL0 = rl0[i];
                 rowL1 = rl0[i + 1];
             }
-            for (int w = 0; w < nw; ++w) {
-                if (active && myWave == w) {
-                    XT sum = XT(0);
+            runWaves(spans, nw, [&](int w, bool spread) {
+                const bool mine = active && myWave == w;
+                XT sum = XT(0);
+                if (mine) {
+                    XT sb = XT(0);
 #pragma unroll
-                    for (int u = 0; u < E; ++u) sum += valOf<XT>(lv[u]) * xl[li[u]];
-                    part[t] = sum;
+                    for (int u = 0; u < E; u += 2) {
+                        sum += valOf<XT>(lv[u]) * xl[li[u]];
+                        sb += valOf<XT>(lv[u + 1]) * xl[li[u + 1]];
+                    }
+                    sum += sb;
                 }
-                __syncthreads();
-                if (first && myWave == w) {
-                    XT s = XT(0);
-                    for (int l = rowL0; l < rowL1; ++l) s += part[l];
-                    xl[i] = (br - s) * dg;
-                }
-                __syncthreads();
-            }
+                sum = rowSum(mine, spread, sum, part, rowL0, rowL1);
+                if (mine && first) xl[i] = (br - sum) * dg;
+            });
             if (first) x[vo + row] = xl[i];
             __syncthreads();
         }
@@ -772,11 +945,11 @@ __global__ void __launch_bounds__(BS) k_gs_bundle_vl(
     }
 }
 
-// Variable lanes per row, Kaczmarz (see kaczBundle).  part: BS partial
+// Variable lanes per row, Kaczmarz (see kaczChain).  part: BS partial
 // sums, rl0: the first lane of every row of the bundle.
-template <int BS, typename VT, typename XT, bool BATCH, bool FLOW, class Wait>
-__device__ __forceinline__ void kaczBundleVL(
-    const int bnd, const int k0, const int k1, XT* xl, XT* part, int* rl0, Wait&& wait,
+template <int BS, typename VT, typename XT, bool BATCH, bool FLOW>
+__device__ __forceinline__ void kaczChainVL(
+    const int cLo, const int cHi, const int k, XT* xl, const int spare, XT* part, int* rl0,
     const int* __restrict__ bSlot, const int* __restrict__ bWave, const long* __restrict__ bOff,
     const int* __restrict__ bLen, const int* __restrict__ bExt, const uint16_t* __restrict__ slotWave,
     const int* __restrict__ rowId, const double* __restrict__ rowNorm, const int* __restrict__ ext,
@@ -784,84 +957,92 @@ __device__ __forceinline__ void kaczBundleVL(
     int n0, const int* __restrict__ lanePtr, const uint16_t* __restrict__ laneSlot, XT* const* __restrict__ bX,
     const XT* const* __restrict__ bB, const int* __restrict__ bN) {
     constexpr int E = kVarE;
-    const BundleVec<BATCH, XT> vec(x0, b0, n0, bX, bB, bN, bnd);
-    XT* __restrict__ x = vec.x;
-    const XT* __restrict__ b = vec.b;
-    const int n = vec.n;
-    const int s0 = bSlot[bnd], nb = bSlot[bnd + 1] - s0;
-    const long off = bOff[bnd];
-    const int wb = bLen[bnd];
-    const int nw = bWave[bnd + 1] - bWave[bnd];
-    const int e0 = bExt[bnd], ne = bExt[bnd + 1] - e0;
-    const int lp = lanePtr[bnd], nl = lanePtr[bnd + 1] - lp;
+    __shared__ WaveSpans<BS / 64> spans;
+    if (cLo >= cHi) return;
+    const BundleVec<BATCH, XT> vec(x0, b0, n0, bX, bB, bN, cLo);
+    const size_t vo = (size_t)k * vec.n;
+    XT* __restrict__ x = vec.x + vo;
+    const XT* __restrict__ b = vec.b + vo;
     const int t = threadIdx.x;
-    const bool active = t < nl;
-    // branch-free prologue, ids first (as in k_gs_bundle_vl)
-    const unsigned ex0 = (unsigned)ext[t < ne ? e0 + t : 0];
-    const unsigned ex1 = (unsigned)ext[t + BS < ne ? e0 + t + BS : 0];
-    const int i = (int)laneSlot[active ? lp + t : 0];  // used by active lanes only
-    const int iPrev = (int)laneSlot[active && t > 0 ? lp + t - 1 : 0];
-    int li[E];
-    typename ValBits<VT>::T lv[E];
-#pragma unroll
-    for (int u = 0; u < E; ++u) {
-        const long e = (active && u < wb) ? off + (long)u * nl + t : zero;
-        li[u] = (int)sidx[e];
-        lv[u] = sval[e];
-    }
-    const int sr = active ? s0 + i : 0;
-    const unsigned row = (unsigned)rowId[sr];
-    const double rn = rowNorm[sr];
-    const int myWave = (int)slotWave[sr];
-    if (active && (t == 0 || iPrev != i)) rl0[i] = t;
-    if (t == 0) rl0[nb] = nl;
-    int rowL0 = 0, rowL1 = 0;
-    wait();
 
-    for (int k = k0; k < k1; ++k) {
-        const size_t vo = (size_t)k * n;
-        const XT g0 = ldX<FLOW>(x, vo, t < ne ? ex0 : 0u);
-        const XT g1 = ldX<FLOW>(x, vo, t + BS < ne ? ex1 : 0u);
-        const XT br = b[vo + (active ? row : 0u)];
-        if (t < ne) xl[t] = g0;
-        if (t + BS < ne) xl[t + BS] = g1;
-        for (int c = t + 2 * BS; c < ne; c += BS) xl[c] = ldX<FLOW>(x, vo, (unsigned)ext[e0 + c]);
-        __syncthreads();
-        if (k == k0 && active) {
-            rowL0 = rl0[i];
-            rowL1 = rl0[i + 1];
+    int s0 = bSlot[cLo], e0 = bExt[cLo], ne = bExt[cLo + 1] - e0;
+    int lp = lanePtr[cLo], nl = lanePtr[cLo + 1] - lp;
+    unsigned ex[kColSlots];
+    loadCols<BS>(ext, e0, ne, ex);
+    int i = (int)laneSlot[t < nl ? lp + t : 0];  // used by active lanes only
+    for (int bnd = cLo;;) {
+        const int nb = bSlot[bnd + 1] - s0;
+        const long off = bOff[bnd];
+        const int wb = bLen[bnd];
+        const int nw = bWave[bnd + 1] - bWave[bnd];
+        const bool active = t < nl;
+        const int sr = active ? s0 + i : 0;
+        const unsigned row = (unsigned)rowId[sr];
+        const double rn = rowNorm[sr];
+        const int myWave = (int)slotWave[sr];
+        const int iPrev = (int)laneSlot[active && t > 0 ? lp + t - 1 : 0];
+        int li[E];
+        typename ValBits<VT>::T lv[E];
+#pragma unroll
+        for (int u = 0; u < E; ++u) {
+            const long e = (active && u < wb) ? off + (long)u * nl + t : zero;
+            li[u] = (int)sidx[e];
+            lv[u] = sval[e];
         }
-        for (int w = 0; w < nw; ++w) {
+        XT g[kColSlots];
+        gatherCols<BS, FLOW>(x, ne, ex, g);
+        const XT br = b[active ? row : 0u];
+        placeCols<BS, FLOW>(x, ext, e0, ne, g, xl);
+        // behind the gathers, as in kaczChain
+        setSpans(spans, active, myWave);
+        if (active && (t == 0 || iPrev != i)) rl0[i] = t;
+        if (t == 0) rl0[nb] = nl;
+        const double rnInv = 1.0 / rn;
+        int lw[E];
+#pragma unroll
+        for (int u = 0; u < E; ++u) lw[u] = valOf<XT>(lv[u]) != XT(0) ? li[u] : ne + (t & (spare - 1));
+        __syncthreads();
+        const int rowL0 = active ? rl0[i] : 0, rowL1 = active ? rl0[i + 1] : 0;
+        const bool more = bnd + 1 < cHi;
+        int s0n = 0, e0n = 0, nen = 0, lpn = 0, nln = 0, in = 0;
+        unsigned exn[kColSlots] = {};
+        if (more) {
+            s0n = bSlot[bnd + 1];
+            e0n = bExt[bnd + 1], nen = bExt[bnd + 2] - e0n;
+            lpn = lanePtr[bnd + 1], nln = lanePtr[bnd + 2] - lpn;
+            loadCols<BS>(ext, e0n, nen, exn);
+            in = (int)laneSlot[t < nln ? lpn + t : 0];
+        }
+        runWaves(spans, nw, [&](int w, bool spread) {
+            const bool mine = active && myWave == w;
             // the lane's x entries, read once in one batch and kept
-            // across the barrier (no other row of this wave writes them)
-            XT cur[E];
-            if (active && myWave == w) {
+            // (no other row of this wave writes them)
+            XT cur[E], dot = XT(0);
+            if (mine) {
 #pragma unroll
                 for (int u = 0; u < E; ++u) cur[u] = xl[li[u]];
-                XT dot = XT(0);
+                XT sb = XT(0);
 #pragma unroll
-                for (int u = 0; u < E; ++u) dot += valOf<XT>(lv[u]) * cur[u];
-                part[t] = dot;
-            }
-            __syncthreads();
-            if (active && myWave == w) {
-                XT rowDot = XT(0);
-                for (int l = rowL0; l < rowL1; ++l) rowDot += part[l];
-                const XT scale = (XT)(((double)rowDot - (double)br) / rn);
-                // nonzero entries only: a padding entry may name a
-                // column another row updates
-#pragma unroll
-                for (int u = 0; u < E; ++u) {
-                    const XT a = valOf<XT>(lv[u]);
-                    if (a != XT(0)) xl[li[u]] = cur[u] - scale * a;
+                for (int u = 0; u < E; u += 2) {
+                    dot += valOf<XT>(lv[u]) * cur[u];
+                    sb += valOf<XT>(lv[u + 1]) * cur[u + 1];
                 }
+                dot += sb;
             }
-            __syncthreads();
-        }
-        if (t < ne) stX<FLOW>(x, vo, ex0, xl[t]);
-        if (t + BS < ne) stX<FLOW>(x, vo, ex1, xl[t + BS]);
-        for (int c = t + 2 * BS; c < ne; c += BS) stX<FLOW>(x, vo, (unsigned)ext[e0 + c], xl[c]);
+            const XT rowDot = rowSum(mine, spread, dot, part, rowL0, rowL1);
+            if (mine) {
+                const XT scale = rowScale<XT>((double)rowDot - (double)br, rn, rnInv);
+#pragma unroll
+                for (int u = 0; u < E; ++u) xl[lw[u]] = cur[u] - scale * valOf<XT>(lv[u]);
+            }
+        });
+        storeCols<BS, FLOW>(x, ext, e0, ne, ex, xl);
         __syncthreads();
+        if (!more) break;
+        ++bnd;
+        s0 = s0n, e0 = e0n, ne = nen, lp = lpn, nl = nln, i = in;
+#pragma unroll
+        for (int q = 0; q < kColSlots; ++q) ex[q] = exn[q];
     }
 }
 
@@ -872,32 +1053,19 @@ __global__ void __launch_bounds__(BS) k_kacz_bundle_vl(
     const int* __restrict__ rowId, const double* __restrict__ rowNorm, const int* __restrict__ ext,
     const uint16_t* __restrict__ sidx, const VT* __restrict__ sval, long zero, XT* __restrict__ x0,
     const XT* __restrict__ b0, int n0, int nrhs, const int* __restrict__ chainPtr, int chain0, int nchain, int xcd,
-    int ldsLocal, int ldsRows, const int* __restrict__ lanePtr, const uint16_t* __restrict__ laneSlot,
+    int ldsLocal, int spare, const int* __restrict__ lanePtr, const uint16_t* __restrict__ laneSlot,
     XT* const* __restrict__ bX, const XT* const* __restrict__ bB, const int* __restrict__ bN) {
     extern __shared__ __align__(16) unsigned char smem[];
     XT* xl = reinterpret_cast<XT*>(smem);
-    XT* part = xl + ldsLocal;                               // BS partial sums
+    XT* part = xl + ldsLocal + spare;                       // BS partial sums
     int* rl0 = reinterpret_cast<int*>(part + BS);           // row -> first lane
-    (void)ldsRows;
 
     const int q = bundleOfBlock(nchain, xcd);
     if (q < 0) return;
     const int cLo = chainPtr[chain0 + q], cHi = chainPtr[chain0 + q + 1];
-    const int k0 = (int)blockIdx.y;
-    const int k1 = gridDim.y > 1 ? k0 + 1 : nrhs;
-    auto runBundle = [&](const int bnd) {
-        kaczBundleVL<BS, VT, XT, BATCH, false>(bnd, k0, k1, xl, part, rl0, NoWait{}, bSlot, bWave, bOff, bLen, bExt,
-                                               slotWave, rowId, rowNorm, ext, sidx, sval, zero, x0, b0, n0, lanePtr,
-                                               laneSlot, bX, bB, bN);
-    };
-    if (cHi == cLo + 1) {
-        runBundle(cLo);
-    } else {
-        for (int bnd = cLo; bnd < cHi; ++bnd) {
-            runBundle(bnd);
-            __syncthreads();
-        }
-    }
+    kaczChainVL<BS, VT, XT, BATCH, false>(cLo, cHi, (int)blockIdx.y, xl, spare, part, rl0, bSlot, bWave, bOff, bLen,
+                                          bExt, slotWave, rowId, rowNorm, ext, sidx, sval, zero, x0, b0, n0, lanePtr,
+                                          laneSlot, bX, bB, bN);
 }
 
 // Kaczmarz with variable lanes per row, all phases of a sweep in one launch.
@@ -907,18 +1075,18 @@ __global__ void __launch_bounds__(BS) k_kacz_flow_vl(
     const int* __restrict__ bLen, const int* __restrict__ bExt, const uint16_t* __restrict__ slotWave,
     const int* __restrict__ rowId, const double* __restrict__ rowNorm, const int* __restrict__ ext,
     const uint16_t* __restrict__ sidx, const VT* __restrict__ sval, long zero, XT* x0, const XT* __restrict__ b0,
-    int n0, int ldsLocal, const int* __restrict__ lanePtr, const uint16_t* __restrict__ laneSlot,
+    int n0, int ldsLocal, int spare, const int* __restrict__ lanePtr, const uint16_t* __restrict__ laneSlot,
     XT* const* __restrict__ bX, const XT* const* __restrict__ bB, const int* __restrict__ bN,
     ReadyTables rt) {
     extern __shared__ __align__(16) unsigned char smem[];
     XT* xl = reinterpret_cast<XT*>(smem);
-    XT* part = xl + ldsLocal;
+    XT* part = xl + ldsLocal + spare;
     int* rl0 = reinterpret_cast<int*>(part + BS);
     const int k = (int)blockIdx.y;
-    readyLoop<BS>(rt, [&](int bnd, auto wait) {
-        kaczBundleVL<BS, VT, XT, BATCH, true>(bnd, k, k + 1, xl, part, rl0, wait, bSlot, bWave, bOff, bLen, bExt,
-                                              slotWave, rowId, rowNorm, ext, sidx, sval, zero, x0, b0, n0, lanePtr,
-                                              laneSlot, bX, bB, bN);
+    readyLoop<BS>(rt, [&](int cLo, int cHi) {
+        kaczChainVL<BS, VT, XT, BATCH, true>(cLo, cHi, k, xl, spare, part, rl0, bSlot, bWave, bOff, bLen, bExt, slotWave,
+                                             rowId, rowNorm, ext, sidx, sval, zero, x0, b0, n0, lanePtr, laneSlot, bX,
+                                             bB, bN);
     });
 }
 
@@ -932,6 +1100,20 @@ int pickE(int tpr, int need) {
     for (int q = 0; q < nc; ++q)
         if (c[q] >= need) return c[q];
     return -1;
+}
+
+// LDS of a workgroup: bytes, and the spare places behind the local columns
+// (one per lane of a wavefront, or what 32 bytes hold where LDS is short)
+struct LdsPlan {
+    size_t bytes;
+    int spare;
+};
+template <typename XT>
+LdsPlan ldsPlan(int local, int rows, int tpr, int bs) {
+    const size_t var = tpr == 0 ? (size_t)bs * sizeof(XT) + (size_t)(rows + 1) * sizeof(int) : 0;
+    const size_t need = (size_t)local * sizeof(XT) + var;
+    const int spare = need + 64 * sizeof(XT) <= kMaxLds ? 64 : 32 / (int)sizeof(XT);
+    return {need + spare * sizeof(XT), spare};
 }
 
 template <typename VT, typename XT>
@@ -995,12 +1177,9 @@ struct BundleDev {
             return (VT)v;
     }
     // LDS bytes of phase p for workgroups of bs threads: the local column
-    // space and, with variable lanes, a partial sum per lane and the first
-    // lane of every row
-    size_t lds(int p, int bs) const {
-        const size_t var = h.tpr == 0 ? (size_t)bs * sizeof(XT) + (size_t)(h.phRows[p] + 1) * sizeof(int) : 0;
-        return (size_t)h.phLocal[p] * sizeof(XT) + var + 32;
-    }
+    // space, the spare places behind it and, with variable lanes, a partial
+    // sum per lane and the first lane of every row
+    LdsPlan lds(int p, int bs) const { return ldsPlan<XT>(h.phLocal[p], h.phRows[p], h.tpr, bs); }
 };
 
 // one fused or plain launch of the chains [c0, c0 + nchain) of phase p
@@ -1012,25 +1191,24 @@ void launchBundles(int kind, int nrhs, const BundleDev<VT, XT>& d, int c0, int n
     const std::vector<int>& cp = d.h.chainPtr;
     const int bundle0 = cp[c0 + nchain] - cp[c0] == nchain ? cp[c0] : -1;
     if (kind == RACE_K_KACZ)
-        hipLaunchKernelGGL((k_kacz_bundle<BS, TPR, EE, VT, XT, BATCH>), grid, dim3(BS), d.lds(p, BS), st,
+        hipLaunchKernelGGL((k_kacz_bundle<BS, TPR, EE, VT, XT, BATCH>), grid, dim3(BS), d.lds(p, BS).bytes, st,
                            d.slot.p, d.wave.p, d.off.p, d.len.p, d.extPtr.p, d.slotWave.p, d.rowId.p,
                            d.rowNorm.p, d.ext.p, d.sidx.p, d.sval.p, d.zero, x, b, n, nrhs, d.chainPtr.p, c0, nchain, xcd,
-                           d.h.phLocal[p], bX, bB, bN);
+                           d.lds(p, BS).spare, bX, bB, bN);
     else if (nrhs == 1 && (BS == 256 || BS == 512) && !BATCH && d.h.phExt[p] > 2 * BS)
         // many outside columns: gather up to 1536 (256 threads) or 2048
         // (512 threads) of them in one batch
         hipLaunchKernelGGL((k_gs_bundle<BS, TPR, EE, VT, XT, true, BATCH, (BS == 256 ? 6 : 4)>), dim3(grid.x), dim3(BS),
-                           d.lds(p, BS),
-                           st, d.slot.p, d.wave.p, d.off.p, d.len.p, d.extPtr.p, d.slotWave.p, d.rowId.p, d.diag.p,
+                           d.lds(p, BS).bytes, st, d.slot.p, d.wave.p, d.off.p, d.len.p, d.extPtr.p, d.slotWave.p, d.rowId.p, d.diag.p,
                            d.ext.p, d.sidx.p, d.sval.p, d.zero, x, b, n, nrhs, d.chainPtr.p, c0, nchain, bundle0, xcd, bX,
                            bB, bN);
     else if (nrhs == 1)
-        hipLaunchKernelGGL((k_gs_bundle<BS, TPR, EE, VT, XT, true, BATCH>), dim3(grid.x), dim3(BS), d.lds(p, BS), st,
+        hipLaunchKernelGGL((k_gs_bundle<BS, TPR, EE, VT, XT, true, BATCH>), dim3(grid.x), dim3(BS), d.lds(p, BS).bytes, st,
                            d.slot.p, d.wave.p, d.off.p, d.len.p, d.extPtr.p, d.slotWave.p, d.rowId.p, d.diag.p,
                            d.ext.p, d.sidx.p, d.sval.p, d.zero, x, b, n, nrhs, d.chainPtr.p, c0, nchain, bundle0, xcd, bX,
                            bB, bN);
     else
-        hipLaunchKernelGGL((k_gs_bundle<BS, TPR, EE, VT, XT, false, BATCH>), grid, dim3(BS), d.lds(p, BS),
+        hipLaunchKernelGGL((k_gs_bundle<BS, TPR, EE, VT, XT, false, BATCH>), grid, dim3(BS), d.lds(p, BS).bytes,
                            st, d.slot.p, d.wave.p, d.off.p, d.len.p, d.extPtr.p, d.slotWave.p, d.rowId.p,
                            d.diag.p, d.ext.p, d.sidx.p, d.sval.p, d.zero, x, b, n, nrhs, d.chainPtr.p, c0, nchain, bundle0,
                            xcd, bX, bB, bN);
@@ -1042,12 +1220,12 @@ void launchBundlesVL(int kind, int nrhs, const BundleDev<VT, XT>& d, int c0, int
                      const XT* b, int n, XT* const* bX, const XT* const* bB, const int* bN, hipStream_t st) {
     const dim3 grid(xcd ? 8u * (unsigned)((nchain + 7) / 8) : (unsigned)nchain, (unsigned)std::max(1, nrhs));
     if (kind == RACE_K_KACZ)
-        hipLaunchKernelGGL((k_kacz_bundle_vl<BS, VT, XT, BATCH>), grid, dim3(BS), d.lds(p, BS), st, d.slot.p, d.wave.p,
+        hipLaunchKernelGGL((k_kacz_bundle_vl<BS, VT, XT, BATCH>), grid, dim3(BS), d.lds(p, BS).bytes, st, d.slot.p, d.wave.p,
                            d.off.p, d.len.p, d.extPtr.p, d.slotWave.p, d.rowId.p, d.rowNorm.p, d.ext.p, d.sidx.p,
-                           d.sval.p, d.zero, x, b, n, nrhs, d.chainPtr.p, c0, nchain, xcd, d.h.phLocal[p], d.h.phRows[p],
+                           d.sval.p, d.zero, x, b, n, nrhs, d.chainPtr.p, c0, nchain, xcd, d.h.phLocal[p], d.lds(p, BS).spare,
                            d.lanePtr.p, d.laneSlot.p, bX, bB, bN);
     else
-        hipLaunchKernelGGL((k_gs_bundle_vl<BS, VT, XT, BATCH>), grid, dim3(BS), d.lds(p, BS), st, d.slot.p, d.wave.p,
+        hipLaunchKernelGGL((k_gs_bundle_vl<BS, VT, XT, BATCH>), grid, dim3(BS), d.lds(p, BS).bytes, st, d.slot.p, d.wave.p,
                            d.off.p, d.len.p, d.extPtr.p, d.slotWave.p, d.rowId.p, d.diag.p, d.ext.p, d.sidx.p,
                            d.sval.p, d.zero, x, b, n, nrhs, d.chainPtr.p, c0, nchain, xcd, d.h.phLocal[p], d.h.phRows[p],
                            d.lanePtr.p, d.laneSlot.p, bX, bB, bN);
@@ -1105,7 +1283,7 @@ struct FlowDev {
     // readiness-driven: the longest dependency path of the sweep, in
     // dependency waves plus kBundleFixedWaves per bundle
     long longestPath = 0;
-    int nchain = 0, grid = 0, nrhs = 1, maxLocal = 0, maxRows = 0;
+    int nchain = 0, grid = 0, nrhs = 1, maxLocal = 0, maxRows = 0, spare = 64;
     size_t lds = 0;
     // chains whose conflicts lie inside one phase (0 for a valid colouring)
     long samePhase = 0;
@@ -1126,8 +1304,9 @@ struct FlowDev {
         }
         // one layout for every phase: the largest local column space, then
         // (variable lanes) the partial sums and the first lane of every row
-        lds = (size_t)maxLocal * sizeof(XT) + 32 +
-              (d.h.tpr == 0 ? (size_t)bs * sizeof(XT) + (size_t)(maxRows + 1) * sizeof(int) : 0);
+        const LdsPlan plan = ldsPlan<XT>(maxLocal, maxRows, d.h.tpr, bs);
+        lds = plan.bytes;
+        spare = plan.spare;
         if (lds > kMaxLds) return OK;  // not used (the caller checks lds)
         // as many workgroups per right-hand side as are resident at once,
         // all sides together (more would only find the tickets gone)
@@ -1252,12 +1431,12 @@ int launchKaczFlow(const BundleDev<VT, XT>& d, FlowDev& f, XT* x, const XT* b, i
     if constexpr (TPR == 0) {
         hipLaunchKernelGGL((k_kacz_flow_vl<BS, VT, XT, BATCH>), dim3(f.grid, f.nrhs), dim3(BS), f.lds, st, d.slot.p,
                            d.wave.p, d.off.p, d.len.p, d.extPtr.p, d.slotWave.p, d.rowId.p, d.rowNorm.p, f.ext.p,
-                           d.sidx.p, d.sval.p, d.zero, x, b, n, f.maxLocal, d.lanePtr.p, d.laneSlot.p, bX, bB, bN,
+                           d.sidx.p, d.sval.p, d.zero, x, b, n, f.maxLocal, f.spare, d.lanePtr.p, d.laneSlot.p, bX, bB, bN,
                            f.tables());
     } else {
         hipLaunchKernelGGL((k_kacz_flow<BS, TPR, EE, VT, XT, BATCH>), dim3(f.grid, f.nrhs), dim3(BS), f.lds, st,
                            d.slot.p, d.wave.p, d.off.p, d.len.p, d.extPtr.p, d.slotWave.p, d.rowId.p, d.rowNorm.p,
-                           f.ext.p, d.sidx.p, d.sval.p, d.zero, x, b, n, bX, bB, bN, f.tables());
+                           f.ext.p, d.sidx.p, d.sval.p, d.zero, x, b, n, f.spare, bX, bB, bN, f.tables());
     }
     RACE_HIP(hipGetLastError());
     return OK;
@@ -1391,9 +1570,9 @@ class BundleFn : public DeviceFn {
         if ((e = df.load(std::move(tf)))) return e;
         if ((e = dr.load(std::move(tr)))) return e;
         for (int p = 0; p < df.h.numPhases(); ++p)
-            if (df.lds(p, bs) > kMaxLds) return fallBack();
+            if (df.lds(p, bs).bytes > kMaxLds) return fallBack();
         for (int p = 0; p < dr.h.numPhases(); ++p)
-            if (dr.lds(p, bs) > kMaxLds) return fallBack();
+            if (dr.lds(p, bs).bytes > kMaxLds) return fallBack();
         const bool gsFlow = kind == RACE_K_GS && nrhs == 1 && bs == 256 && tpr > 0;
         const bool kaczFlow = kind == RACE_K_KACZ && kaczFlowBs(bs);
         if (ctx.flow && (gsFlow || kaczFlow)) {
@@ -1569,7 +1748,7 @@ class BundleBatchFn : public DeviceFn {
                 if ((e = upload(grp->bn[dir], hn.data(), hn.size()))) return e;
                 if ((e = grp->dev[dir].load(std::move(fused)))) return e;
                 for (int p = 0; p < grp->dev[dir].h.numPhases(); ++p)
-                    if (grp->dev[dir].lds(p, bs) > kMaxLds) return ERR_INCOMPATIBILITY;
+                    if (grp->dev[dir].lds(p, bs).bytes > kMaxLds) return ERR_INCOMPATIBILITY;
                 maxPhases[dir] = std::max(maxPhases[dir], grp->dev[dir].h.numPhases());
                 if (ctx.flow && kind == RACE_K_KACZ && kaczFlowBs(bs)) {
                     // every matrix its own range of row / column keys
@@ -1670,54 +1849,19 @@ class BundleBatchFn : public DeviceFn {
 
 }  // namespace
 
-int makeBundleBatchFn(const std::vector<BatchItem>& items, const ExecContext& ctx, std::unique_ptr<DeviceFn>* out) {
-    if (items.empty()) return ERR_INVALID_ARG;
-    if (ctx.bundleThreads != 64 && ctx.bundleThreads != 128 && ctx.bundleThreads != 256 && ctx.bundleThreads != 512 &&
-        ctx.bundleThreads != 1024)
-        return ERR_INVALID_ARG;
-    const race_kernel_desc& d0 = items[0].d;
-    for (const BatchItem& it : items)
-        if (it.d.kind != d0.kind || it.d.val_precision != d0.val_precision ||
-            it.d.vec_precision != d0.vec_precision || it.d.nrhs != d0.nrhs || !it.fwd || !it.rev)
-            return ERR_INVALID_ARG;
-    if (d0.kind != RACE_K_GS && d0.kind != RACE_K_KACZ) return ERR_INVALID_ARG;
-    int e;
-    if (d0.vec_precision == RACE_FP64) {
-        if (d0.val_precision != RACE_FP64) return ERR_NOT_IMPLEMENTED;
-        auto f = std::make_unique<BundleBatchFn<double, double>>();
-        e = f->init(items, ctx);
-        *out = std::move(f);
-    } else if (d0.val_precision == RACE_BF16) {
-        auto f = std::make_unique<BundleBatchFn<uint16_t, float>>();
-        e = f->init(items, ctx);
-        *out = std::move(f);
-    } else {
-        auto f = std::make_unique<BundleBatchFn<float, float>>();
-        e = f->init(items, ctx);
-        *out = std::move(f);
-    }
+template <typename VT, typename XT>
+int makeBundleOf(const race_kernel_desc& d, const ExecContext& ctx, std::unique_ptr<DeviceFn>* out) {
+    auto f = std::make_unique<BundleFn<VT, XT>>();
+    const int e = f->init(d, ctx);
+    *out = std::move(f);
     return e;
 }
 
-int makeBundleFn(const race_kernel_desc& d, const ExecContext& ctx, std::unique_ptr<DeviceFn>* out) {
-    if (ctx.bundleThreads != 64 && ctx.bundleThreads != 128 && ctx.bundleThreads != 256 && ctx.bundleThreads != 512 &&
-        ctx.bundleThreads != 1024)
-        return ERR_INVALID_ARG;
-    int e;
-    if (d.vec_precision == RACE_FP64) {
-        if (d.val_precision != RACE_FP64) return ERR_NOT_IMPLEMENTED;
-        auto f = std::make_unique<BundleFn<double, double>>();
-        e = f->init(d, ctx);
-        *out = std::move(f);
-    } else if (d.val_precision == RACE_BF16) {
-        auto f = std::make_unique<BundleFn<uint16_t, float>>();
-        e = f->init(d, ctx);
-        *out = std::move(f);
-    } else {
-        auto f = std::make_unique<BundleFn<float, float>>();
-        e = f->init(d, ctx);
-        *out = std::move(f);
-    }
+template <typename VT, typename XT>
+int makeBundleBatchOf(const std::vector<BatchItem>& items, const ExecContext& ctx, std::unique_ptr<DeviceFn>* out) {
+    auto f = std::make_unique<BundleBatchFn<VT, XT>>();
+    const int e = f->init(items, ctx);
+    *out = std::move(f);
     return e;
 }
 

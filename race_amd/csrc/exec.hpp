@@ -77,11 +77,11 @@ struct BatchItem {
     const Schedule* rev = nullptr;
     race_kernel_desc d{};
 };
-// GS / KACZ on a batch of matrices, fused launches per phase (bundle_exec.hip)
+// GS / KACZ on a batch of matrices, fused launches per phase (bundle_exec.hpp)
 int makeBundleBatchFn(const std::vector<BatchItem>& items, const ExecContext& ctx, std::unique_ptr<DeviceFn>* out);
 // SymmSpMV / SpMV on a batch of matrices, one launch (sell.hip)
 int makeSellBatchFn(const std::vector<BatchItem>& items, const ExecContext& ctx, std::unique_ptr<DeviceFn>* out);
-// Gauss-Seidel / Kaczmarz over leaf bundles (bundle_exec.hip)
+// Gauss-Seidel / Kaczmarz over leaf bundles (bundle_exec.hpp)
 int makeBundleFn(const race_kernel_desc& d, const ExecContext& ctx, std::unique_ptr<DeviceFn>* out);
 // FP64 iterative refinement around an inner GS/KACZ function (refine.hip)
 int makeRefineFn(const race_kernel_desc& d, DeviceFn* inner, int sweeps, std::unique_ptr<DeviceFn>* out);

@@ -812,7 +812,7 @@ static void expandUpper(const race_kernel_desc& d, std::vector<int>& rp, std::ve
 // store more than 5 slots for 4 entries (Product's rule) or be wider than 64
 // entries: with 8 right-hand sides a chunk holding a hub row runs its up to
 // 400 steps once per right-hand side.  16 matrices of 2000 to 40000 rows, FP32,
-// 8 right-hand sides: 864 us in chunks alone, 124 us.
+// 8 right-hand sides: 864 us in chunks alone, 176 us.
 template <typename XT>
 class SellBatchFn : public DeviceFn {
   public:
