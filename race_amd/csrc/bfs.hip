@@ -130,6 +130,7 @@ struct RangeJob {
 };
 
 constexpr int kBatchMaxJobs = 4096;
+constexpr int kSmallRange = 4096;  // rows up to which a workgroup of 256 threads traverses a range
 
 // bitonic sort of BS 64-bit keys in LDS (blockDim.x == BS)
 template <int BS>
@@ -741,6 +742,12 @@ int GpuTraverser::traverseBatch(int dist, const std::vector<std::pair<int, int>>
         }
     }
     if (small.empty()) return OK;
+    // ranges of more than kSmallRange rows first: they take workgroups of
+    // 1024 threads, the others 256
+    const auto firstSmall = std::stable_partition(small.begin(), small.end(), [&](size_t r) {
+        return ranges[r].second - ranges[r].first > kSmallRange;
+    });
+    const size_t nLarge = (size_t)(firstSmall - small.begin());
     auto t0 = std::chrono::steady_clock::now();
     const int two = (dist == DIST_TWO) ? 1 : 0;
     // distance-2 bridge slots: one n-entry array per concurrent range, at
@@ -761,7 +768,7 @@ int GpuTraverser::traverseBatch(int dist, const std::vector<std::pair<int, int>>
         const size_t nj = std::min(small.size() - c0, (size_t)maxJobs);
         std::vector<RangeJob> jobs(nj);
         long qTotal = 0, lvTotal = 0;
-        int spanLo = n, spanHi = 0, maxLen = 0;
+        int spanLo = n, spanHi = 0;
         for (size_t j = 0; j < nj; ++j) {
             const int lo = ranges[small[c0 + j]].first, hi = ranges[small[c0 + j]].second;
             const int len = hi - lo;
@@ -775,7 +782,6 @@ int GpuTraverser::traverseBatch(int dist, const std::vector<std::pair<int, int>>
             lvTotal += 3l * len + 2;
             spanLo = std::min(spanLo, lo);
             spanHi = std::max(spanHi, hi);
-            maxLen = std::max(maxLen, len);
         }
         RACE_HIP(dJobs.reserve(nj * sizeof(RangeJob)));
         RACE_HIP(dBatchQ.reserve(qTotal));
@@ -790,14 +796,16 @@ int GpuTraverser::traverseBatch(int dist, const std::vector<std::pair<int, int>>
         const RangeJob* dj = reinterpret_cast<const RangeJob*>(dJobs.p);
         const int stamp0 = stampNext;
         stampNext += (int)nj;
-        if (maxLen <= 4096)
-            hipLaunchKernelGGL(k_bfs_batch<256>, dim3(nj), dim3(256), 0, st, dRowPtr.p, dCol.p, dPerm.p,
+        const size_t large = nLarge > c0 ? std::min(nj, nLarge - c0) : 0;
+        if (large > 0)
+            hipLaunchKernelGGL(k_bfs_batch<1024>, dim3(large), dim3(1024), 0, st, dRowPtr.p, dCol.p, dPerm.p,
                                dInv.p, dVisit.p, dBVisit.p, dDist.p, dBatchQ.p, dLvRow.p, dLvNnz.p, dLvStart.p,
                                dTmp.p, dj, stamp0, two, dist == DIST_POWER ? 1 : 0, n, dNLev.p, dNLev.p + nj);
-        else
-            hipLaunchKernelGGL(k_bfs_batch<1024>, dim3(nj), dim3(1024), 0, st, dRowPtr.p, dCol.p, dPerm.p,
+        if (nj > large)
+            hipLaunchKernelGGL(k_bfs_batch<256>, dim3(nj - large), dim3(256), 0, st, dRowPtr.p, dCol.p, dPerm.p,
                                dInv.p, dVisit.p, dBVisit.p, dDist.p, dBatchQ.p, dLvRow.p, dLvNnz.p, dLvStart.p,
-                               dTmp.p, dj, stamp0, two, dist == DIST_POWER ? 1 : 0, n, dNLev.p, dNLev.p + nj);
+                               dTmp.p, dj + large, stamp0 + (int)large, two, dist == DIST_POWER ? 1 : 0, n,
+                               dNLev.p + large, dNLev.p + nj);
         RACE_HIP(hipGetLastError());
         hNLev.resize(nj + 1);
         RACE_HIP(hipMemcpyAsync(hNLev.data(), dNLev.p, (nj + 1) * sizeof(int), hipMemcpyDeviceToHost, st));

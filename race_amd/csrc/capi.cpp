@@ -21,6 +21,7 @@
 #include "bfs.hpp"
 #include "simdify.hpp"
 #include "engine.hpp"
+#include "parallel.hpp"
 #include "exec.hpp"
 #include "graph_cache.hpp"
 #include "schedule_io.hpp"
@@ -338,8 +339,9 @@ static void setPermAndSchedules(race_handle h) {
         h->inv.resize(h->nrow);
         for (int i = 0; i < h->nrow; ++i) h->inv[h->perm[i]] = i;
     }
-    h->fwd = flattenSchedule(*h->tree, false, h->nGraph);
-    h->rev = flattenSchedule(*h->tree, true, h->nGraph);
+    parallelRanges(2, 1, [&](int lo, int hi) {
+        for (int rev = lo; rev < hi; ++rev) (rev ? h->rev : h->fwd) = flattenSchedule(*h->tree, rev != 0, h->nGraph);
+    });
     appendSerialPhase(h, &h->fwd);
     appendSerialPhase(h, &h->rev);
 }

@@ -1,6 +1,8 @@
 // engine.cpp -- host scheduling logic of the MI355X RACE engine.
 #include "engine.hpp"
 
+#include "parallel.hpp"
+
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
@@ -315,26 +317,41 @@ void ZoneTree::updateEffRow(int p) {
     for (int q = p; q != -1; q = tree[q].parentZ) tree[q].effRowZ = keyChildEffRow(q);
 }
 
-void ZoneTree::updateNThreads(int p) {
-    for (int q = p; q != -1; q = tree[q].parentZ) {
-        const std::vector<int>& ch = tree[q].children;
-        int best = 0;
-        for (size_t sb = 0; sb < ch.size() / 2; ++sb) {
-            int nt = (ch[2 * sb + 1] - ch[2 * sb]) / bpt;
-            int sum = 0;
-            for (int i = 0; i < nt; ++i) {
-                int m = 0;
-                for (int b = 0; b < bpt; ++b) m = std::max(m, tree[ch[2 * sb] + bpt * i + b].nthreadsZ);
-                sum += m;
-            }
-            best = std::max(best, sum);
+int ZoneTree::childThreads(int q) const {
+    const std::vector<int>& ch = tree[q].children;
+    int best = 0;
+    for (size_t sb = 0; sb < ch.size() / 2; ++sb) {
+        int nt = (ch[2 * sb + 1] - ch[2 * sb]) / bpt;
+        int sum = 0;
+        for (int i = 0; i < nt; ++i) {
+            int m = 0;
+            for (int b = 0; b < bpt; ++b) m = std::max(m, tree[ch[2 * sb] + bpt * i + b].nthreadsZ);
+            sum += m;
         }
-        tree[q].nthreadsZ = best;
+        best = std::max(best, sum);
     }
+    return best;
+}
+
+void ZoneTree::updateNThreads(int p) {
+    for (int q = p; q != -1; q = tree[q].parentZ) tree[q].nthreadsZ = childThreads(q);
+}
+
+void ZoneTree::updateAll() {
+    for (int q = (int)tree.size() - 1; q >= 0; --q)
+        if (!tree[q].children.empty()) {
+            tree[q].effRowZ = keyChildEffRow(q);
+            tree[q].nthreadsZ = childThreads(q);
+        }
 }
 
 bool ZoneTree::spawnChild(int parent, int parentSub, int request, const LevelData& ld, double eff) {
-    LBResult lb = splitZones(ld, request, eff, dist, d2, lbTarget);
+    const LBResult lb = splitZones(ld, request, eff, dist, d2, lbTarget);
+    adopt(parent, parentSub, lb);
+    return lb.threads() == request;
+}
+
+void ZoneTree::attach(int parent, int parentSub, const LBResult& lb) {
     const int first = (int)tree.size();
     const int base = tree[parent].valueZ[parentSub];
     const int stage = tree[parent].stage;
@@ -354,15 +371,18 @@ bool ZoneTree::spawnChild(int parent, int parentSub, int request, const LevelDat
         }
         leaf.valueZ.push_back(subRow);
         row += lb.zoneRows[b];
-        tree.push_back(leaf);
+        tree.push_back(std::move(leaf));
     }
     (void)row;
     tree[parent].children.push_back(first + blocks);
+}
+
+void ZoneTree::adopt(int parent, int parentSub, const LBResult& lb) {
+    attach(parent, parentSub, lb);
     if (parentSub == tree[parent].totalSubBlocks - 1) {
         updateEffRow(parent);
         updateNThreads(parent);
     }
-    return lb.threads() == request;
 }
 
 // ---------------------------------------------------------------------------
@@ -388,16 +408,16 @@ int LevelRecursion::lvlThreads(int lvl) const {
     return (lvl - 1 >= 0 && lvl - 1 < (int)lvlThreadsVec.size()) ? lvlThreadsVec[lvl - 1] : -1;
 }
 
-long LevelRecursion::nnzSum(int lo, int hi) const {
+void LevelRecursion::sumNnz() {
     const std::vector<int>& p = trav->perm();
-    long s = 0;
-    for (int r = lo; r < hi; ++r) s += trav->rowLen(p[r]);
-    return s;
+    nnzBefore.resize((size_t)n + 1);
+    nnzBefore[0] = 0;
+    for (int r = 0; r < n; ++r) nnzBefore[r + 1] = nnzBefore[r] + trav->rowLen(p[r]);
 }
 
-void LevelRecursion::idealNthreads(int parent, int parentSub, int currLvl) {
-    auto& T = zt->tree;
-    const int bpt = zt->bpt;
+void LevelRecursion::idealNthreads(ZoneTree& z, int parent, int parentSub, int currLvl) {
+    auto& T = z.tree;
+    const int bpt = z.bpt;
     const int c0 = T[parent].children[2 * parentSub];
     const int nt = (T[parent].children[2 * parentSub + 1] - c0) / bpt;
     if (lvlThreads(currLvl) != -1) {
@@ -409,12 +429,12 @@ void LevelRecursion::idealNthreads(int parent, int parentSub, int currLvl) {
     const int parentThreads = T[parent].idealNthreadsZ;
     const int s = T[parent].valueZ[parentSub], e = T[parent].valueZ[parentSub + 1];
     // the reference accumulates nnz in int
-    const int total = (lbTarget == LB_NNZ) ? (int)nnzSum(s, e) : e - s;
+    const int total = (lbTarget == LB_NNZ) ? (int)(nnzBefore[e] - nnzBefore[s]) : e - s;
     std::vector<int> weights(nt);
     for (int i = 0; i < nt; ++i) {
         const int ss = T[c0 + i * bpt].valueZ.front();
         const int ee = T[c0 + bpt * (i + 1) - 1].valueZ.back();
-        weights[i] = (lbTarget == LB_NNZ) ? (int)nnzSum(ss, ee) : ee - ss;
+        weights[i] = (lbTarget == LB_NNZ) ? (int)(nnzBefore[ee] - nnzBefore[ss]) : ee - ss;
     }
     const std::vector<int> my = splitThreads(weights, total, parentThreads);
     for (int i = 0; i < nt; ++i)
@@ -444,48 +464,101 @@ std::vector<int> splitThreads(const std::vector<int>& weights, int total, int pa
     return my;
 }
 
-int LevelRecursion::recursivePartition(int parent, int parentSub, int currLvl) {
-    idealNthreads(parent, parentSub, currLvl);
-    const std::vector<int> ch = zt->tree[parent].children;
-    // The ranges traversed below are fixed here (valueZ and idealNthreadsZ
-    // of these children change no more) and disjoint, and a traversal
-    // depends only on the rows of its range, so all of them are traversed
-    // up front as one batch; the loop then consumes the results in order.
+// The recursion below the root, in two passes.  A range's traversal and split
+// depend only on the rows of the range and on its thread count, both fixed by
+// its ancestors; ranges of one depth are disjoint.  So the first pass goes
+// breadth first over a copy of the tree and traverses all ranges of a depth as
+// one batch.  Depth first, the 3600 nodes of a 72^3 mesh were 3600 small
+// batches, each a launch, five copies and two waits (27-point, 16 rows per
+// thread: 530 ms, 115 ms in one batch per depth).  The second pass gives the
+// nodes the reference's depth-first numbering from the splits that the first
+// one found.  The reference updates the threads and rows of all ancestors after
+// every split.  Where every zone is one sub-block, the last of these updates to
+// reach a node finds its children final, so one pass from the leaves up gives
+// the same values (11 ms of that mesh); otherwise they are made split by split,
+// in the reference's order.
+int LevelRecursion::splitAll(Splits* out) {
+    struct Item {
+        int parent, sub, lvl;
+    };
+    struct Task {
+        int node, sub, lvl, threads;
+    };
+    ZoneTree z = *zt;
+    std::vector<Item> front{{0, 0, 2}}, deeper;
+    std::vector<Task> tasks;
     std::vector<std::pair<int, int>> ranges;
-    for (int ci = ch[2 * parentSub]; ci < ch[2 * parentSub + 1]; ++ci) {
-        if (zt->tree[ci].idealNthreadsZ <= 1) continue;
-        const std::vector<int>& rng = zt->tree[ci].valueZ;
-        for (size_t j = 0; j + 1 < rng.size(); ++j)
-            if (rng[j + 1] > rng[j]) ranges.push_back({rng[j], rng[j + 1]});
-    }
     std::vector<LevelData> lds;
-    int berr = trav->traverseBatch(dist, ranges, &lds);
-    if (berr != OK) return berr;
-    size_t next = 0;
-    for (int ci = ch[2 * parentSub]; ci < ch[2 * parentSub + 1]; ++ci) {
+    out->node.assign(z.tree.size(), {});
+    while (!front.empty()) {
+        tasks.clear();
+        ranges.clear();
+        deeper.clear();
+        if (lbTarget == LB_NNZ) sumNnz();  // in the order that the last traversals left
+        for (const Item& it : front) {
+            idealNthreads(z, it.parent, it.sub, it.lvl);
+            const std::vector<int>& ch = z.tree[it.parent].children;
+            for (int ci = ch[2 * it.sub]; ci < ch[2 * it.sub + 1]; ++ci) {
+                const ZoneLeaf& leaf = z.tree[ci];
+                out->node[ci].threads = leaf.idealNthreadsZ;
+                if (leaf.idealNthreadsZ <= 1) continue;
+                for (size_t j = 0; j + 1 < leaf.valueZ.size(); ++j) {
+                    if (leaf.valueZ[j + 1] <= leaf.valueZ[j]) continue;
+                    tasks.push_back({ci, (int)j, it.lvl, leaf.idealNthreadsZ});
+                    ranges.push_back({leaf.valueZ[j], leaf.valueZ[j + 1]});
+                }
+            }
+        }
+        const int err = trav->traverseBatch(dist, ranges, &lds);
+        if (err != OK) return err;
+        std::vector<LBResult> lb(tasks.size());
+        parallelRanges((int)tasks.size(), 16, [&](int t0, int t1) {
+            for (int t = t0; t < t1; ++t)
+                lb[t] = splitZones(lds[t], tasks[t].threads, efficiency(tasks[t].lvl), z.dist, z.d2, z.lbTarget);
+        });
+        for (size_t t = 0; t < tasks.size(); ++t) {
+            const Task& k = tasks[t];
+            const int first = (int)z.tree.size();
+            z.attach(k.node, k.sub, lb[t]);
+            out->node.resize(z.tree.size());
+            for (int b : lb[t].numBlocks) out->subBlocks |= b != 1;
+            if (lb[t].threads() != k.threads && (int)lb[t].zoneRows.size() / z.bpt > 1)
+                deeper.push_back({k.node, k.sub, k.lvl + 1});
+            std::vector<Splits::Sub>& subs = out->node[k.node].subs;
+            subs.resize(k.sub + 1);
+            subs[k.sub] = {first, std::move(lb[t])};
+        }
+        front.swap(deeper);
+    }
+    return OK;
+}
+
+void LevelRecursion::place(const Splits& sp, int parent, int parentSub, int spFirst) {
+    // copied: the tree grows below
+    const int c0 = zt->tree[parent].children[2 * parentSub], c1 = zt->tree[parent].children[2 * parentSub + 1];
+    for (int ci = c0; ci < c1; ++ci) zt->tree[ci].idealNthreadsZ = sp.node[spFirst + (ci - c0)].threads;
+    for (int ci = c0; ci < c1; ++ci) {
         const int nt = zt->tree[ci].idealNthreadsZ;
+        const Splits::Node& node = sp.node[spFirst + (ci - c0)];
         const std::vector<int> rng = zt->tree[ci].valueZ;
         if (nt <= 1) continue;
         for (size_t j = 0; j + 1 < rng.size(); ++j) {
             if (rng[j + 1] > rng[j]) {
-                const LevelData& ld = lds[next++];
-                int err;
-                bool ok = zt->spawnChild(ci, (int)j, nt, ld, efficiency(currLvl));
-                if (!ok) {
-                    const std::vector<int>& cc = zt->tree[ci].children;
-                    int sub = (cc[2 * j + 1] - cc[2 * j]) / zt->bpt;
+                const Splits::Sub& u = node.subs[j];
+                if (sp.subBlocks)
+                    zt->adopt(ci, (int)j, u.lb);
+                else
+                    zt->attach(ci, (int)j, u.lb);
+                if (u.lb.threads() != nt) {
+                    const int sub = (int)u.lb.zoneRows.size() / zt->bpt;
                     if (sub == 1) zt->tree[ci].reachedLimit = true;
-                    if (sub > 1) {
-                        err = recursivePartition(ci, (int)j, currLvl + 1);
-                        if (err != OK) return err;
-                    }
+                    if (sub > 1) place(sp, ci, (int)j, u.first);
                 }
             } else {
                 zt->tree[ci].reachedLimit = true;
             }
         }
     }
-    return OK;
 }
 
 int LevelRecursion::levelBalancing(ZoneTree* tree) {
@@ -504,8 +577,12 @@ int LevelRecursion::levelBalancing(ZoneTree* tree) {
     int stage1 = lvlThreads(1) != -1 ? lvlThreads(1) : request;
     zt->spawnChild(0, 0, stage1, ld, efficiency(1));
     if (zt->tree[0].nthreadsZ != request) {
-        err = recursivePartition(0, 0, 2);
+        Splits sp;
+        err = splitAll(&sp);
         if (err != OK) return err;
+        zt->tree.reserve(sp.node.size());
+        place(sp, 0, 0, zt->tree[0].children[0]);
+        if (!sp.subBlocks) zt->updateAll();
     }
     availableThreads = zt->tree[0].nthreadsZ;
     return OK;

@@ -90,11 +90,18 @@ class ZoneTree {
     std::vector<ZoneLeaf> tree;
     // ZoneTree::spawnChild src/zone_tree.cpp:243-305
     bool spawnChild(int parent, int parentSub, int request, const LevelData& ld, double eff);
+    // its second half, from a split that is already known: the nodes of the
+    // split (attach), then the effective rows and threads of their ancestors
+    void adopt(int parent, int parentSub, const LBResult& lb);
+    void attach(int parent, int parentSub, const LBResult& lb);
+    // effective rows and threads of every node from its children's
+    void updateAll();
     int maxStage() const;
 
   private:
     int keyChildEffRow(int p) const;  // findKeyChild :91-155
     void updateEffRow(int p);         // :158-170
+    int childThreads(int q) const;
     void updateNThreads(int p);       // :172-206
 };
 
@@ -150,9 +157,24 @@ class LevelRecursion {
     std::vector<int> lvlThreadsVec;
     double efficiency(int lvl) const;
     int lvlThreads(int lvl) const;
-    long nnzSum(int lo, int hi) const;
-    void idealNthreads(int parent, int parentSub, int currLvl);
-    int recursivePartition(int parent, int parentSub, int currLvl);
+    std::vector<long> nnzBefore;  // graph entries of the rows before each position
+    void sumNnz();
+    // every split below the root; nodes numbered breadth first
+    struct Splits {
+        struct Sub {
+            int first = 0;  // first node of the split
+            LBResult lb;
+        };
+        struct Node {
+            int threads = 1;
+            std::vector<Sub> subs;  // per sub-block
+        };
+        std::vector<Node> node;
+        bool subBlocks = false;  // some zone has several sub-blocks
+    };
+    void idealNthreads(ZoneTree& z, int parent, int parentSub, int currLvl);
+    int splitAll(Splits* out);
+    void place(const Splits& sp, int parent, int parentSub, int spFirst);
 };
 
 // Flattened colour schedule: leaves grouped into barrier-separated phases.

@@ -23,11 +23,11 @@
 
 #include <algorithm>
 #include <cstdint>
-#include <thread>
 #include <type_traits>
 
 #include "exec.hpp"
 #include "exec_common.hpp"
+#include "parallel.hpp"
 #include "rowblock.hpp"
 #include "sell_common.hpp"
 
@@ -37,21 +37,6 @@ namespace {
 
 constexpr int kC = 64;               // rows per chunk (one wavefront)
 constexpr int kWavesPerBlock = kBlock / kC;
-
-// f(lo, hi) over [0, n) in contiguous parts on up to 8 host threads
-template <class F>
-void parallelRanges(int n, int grain, F&& f) {
-    const int want = std::min({8, (int)std::max(1u, std::thread::hardware_concurrency()), n / std::max(1, grain)});
-    if (want <= 1) {
-        f(0, n);
-        return;
-    }
-    std::vector<std::thread> ts;
-    ts.reserve(want);
-    for (int t = 0; t < want; ++t)
-        ts.emplace_back([&f, n, want, t] { f((int)((long)n * t / want), (int)((long)n * (t + 1) / want)); });
-    for (std::thread& t : ts) t.join();
-}
 
 // A block of E entries per lane of elements T: a lane reads V of them at once
 template <typename T>
