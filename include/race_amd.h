@@ -178,8 +178,12 @@ int race_register_device(race_handle h, const race_kernel_desc *desc, int *id);
  *                  256-1024-thread workgroups): the chains of all colour
  *                  phases are handed out in phase order and each waits only
  *                  for the earlier chains it conflicts with (per-chain
- *                  completion flags) instead of a launch boundary per phase
- *                  (default 0); set before registering; results identical
+ *                  completion flags) instead of a launch boundary per phase;
+ *                  calls of one function must not overlap.  0 = one launch
+ *                  per phase.  Unless set, small matrices take the one-launch
+ *                  sweep and others the phase launches (calls may overlap on
+ *                  different streams).  Set before registering; results
+ *                  identical
  * No counterpart in the reference (its executor has no layout choice). */
 int race_set_option(race_handle h, const char *key, int value);
 /* re-point a registered device function at other vectors */

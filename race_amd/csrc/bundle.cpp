@@ -436,8 +436,14 @@ long chainDeps(const BundleTable& t, long nkeys, const std::vector<long>* colBas
     // (waiting chain, chain it waits for)
     std::vector<std::pair<int, int>> edge;
     long same = 0;
-    auto add = [&](int waiter, int first) {
+    // seen[other]: the chain whose columns last gave this pair, so that the
+    // many columns two chains share make one edge
+    std::vector<int> seen(std::max(nchain, 0), -1);
+    auto add = [&](int waiter, int first, int c) {
         if (phaseOf[waiter] == phaseOf[first]) ++same;
+        int& s = seen[waiter == c ? first : waiter];
+        if (s == c) return;
+        s = c;
         edge.push_back({waiter, first});
     };
     if (t.kind != RACE_K_KACZ) {
@@ -452,9 +458,9 @@ long chainDeps(const BundleTable& t, long nkeys, const std::vector<long>* colBas
                     const int o = owner[keyOf(colBase, b, t.ext[e])];
                     if (o < 0 || o == c) continue;  // not written in the sweep, or by this chain
                     if (o < c)
-                        add(c, o);  // c reads what o wrote
+                        add(c, o, c);  // c reads what o wrote
                     else
-                        add(o, c);  // o overwrites what c read
+                        add(o, c, c);  // o overwrites what c read
                 }
     } else {
         // every column a chain touches is read and written: each chain waits
@@ -464,7 +470,7 @@ long chainDeps(const BundleTable& t, long nkeys, const std::vector<long>* colBas
             for (int b = t.chainPtr[c]; b < t.chainPtr[c + 1]; ++b)
                 for (int e = t.extPtr[b]; e < t.extPtr[b + 1]; ++e) {
                     const int o = last[keyOf(colBase, b, t.ext[e])];
-                    if (o >= 0 && o != c) add(c, o);
+                    if (o >= 0 && o != c) add(c, o, c);
                 }
             for (int b = t.chainPtr[c]; b < t.chainPtr[c + 1]; ++b)
                 for (int e = t.extPtr[b]; e < t.extPtr[b + 1]; ++e) last[keyOf(colBase, b, t.ext[e])] = c;

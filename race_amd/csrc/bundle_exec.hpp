@@ -18,6 +18,7 @@
 #include <atomic>
 #include <cstdint>
 #include <cstring>
+#include <mutex>
 #include <thread>
 #include <type_traits>
 
@@ -1260,6 +1261,9 @@ void launchPhase(int bs, int tpr, int E, int kind, int nrhs, const BundleDev<VT,
 // polls of one dependency flag or queue position before a launch gives up
 // (about seconds; a correct dependency table never gets near it)
 constexpr int kFlowPollLimit = 1 << 22;
+// and of a launch that the caller did not ask for by the option (and whose
+// aborts it will not look for): far longer than any pause of the device
+constexpr int kAutoPollLimit = 1 << 30;
 
 // a bundle's prologue, gathers and stores, in dependency waves (weight of a
 // bundle in the longest-path estimate of a readiness-driven sweep)
@@ -1271,15 +1275,21 @@ constexpr int kBundleFixedWaves = 4;
 // an arrival counter per chain and a ready queue (readiness-driven), and a
 // ticket/epoch state.
 struct FlowDev {
-    DevBuf<int> depPtr, dep, flag, ext, lo, hi;
-    DevBuf<FlowState> fs;
-    // readiness-driven sweeps (Kaczmarz): successors, roots, arrival
-    // counters and ready queues
+    DevBuf<int> depPtr, dep, ext, lo, hi;
+    // readiness-driven sweeps (Kaczmarz): successors and roots
     DevBuf<int> succPtr, succ, roots;
-    DevBuf<unsigned> arrivals;
-    DevBuf<unsigned long long> queue;
+    // what a running sweep changes; sweeps on different streams may overlap
+    // if each uses a set of its own
+    struct Live {
+        DevBuf<int> flag;
+        DevBuf<FlowState> fs;
+        // readiness-driven: arrival counters and ready queues
+        DevBuf<unsigned> arrivals;
+        DevBuf<unsigned long long> queue;
+    };
+    std::vector<std::unique_ptr<Live>> live;
     bool readyMode = false;
-    int nroots = 0;
+    int nroots = 0, pollLimit = kFlowPollLimit;
     // readiness-driven: the longest dependency path of the sweep, in
     // dependency waves plus kBundleFixedWaves per bundle
     long longestPath = 0;
@@ -1290,9 +1300,10 @@ struct FlowDev {
     // nkeys / colBase: the key space of the rows and columns (chainDeps);
     // kern: the kernel that will run it, for its occupancy
     // ready: readiness-driven (queue) instead of tickets in chain order
+    // sets: sweeps that may overlap
     template <typename VT, typename XT>
     int init(const BundleDev<VT, XT>& d, long nkeys, const std::vector<long>* colBase, int bs, int nrhs_,
-             const void* kern, bool ready) {
+             const void* kern, bool ready, int sets = 1) {
         readyMode = ready;
         std::vector<int> dp, dd;
         samePhase = chainDeps(d.h, nkeys, colBase, &dp, &dd);
@@ -1340,8 +1351,6 @@ struct FlowDev {
         if ((e = upload(hi, hhi.data(), hhi.size()))) return e;
         const std::vector<int> fx = flowExt(d.h, nkeys, colBase);
         if ((e = upload(ext, fx.data(), fx.size()))) return e;
-        const std::vector<int> zeros((size_t)std::max(nchain, 1) * nrhs, 0);
-        if ((e = upload(flag, zeros.data(), zeros.size()))) return e;
         if (ready) {
             std::vector<int> sp(nchain + 1, 0), sv(qd.size()), rv;
             for (int c = 0; c < nchain; ++c)
@@ -1358,21 +1367,28 @@ struct FlowDev {
             if ((e = upload(succPtr, sp.data(), sp.size()))) return e;
             if ((e = upload(succ, sv.data(), sv.size()))) return e;
             if ((e = upload(roots, rv.data(), rv.size()))) return e;
-            const std::vector<unsigned> az((size_t)std::max(nchain, 1) * nrhs, 0u);
-            if ((e = upload(arrivals, az.data(), az.size()))) return e;
-            // queue entries of epoch 0 never match a launch
-            const std::vector<unsigned long long> qz((size_t)std::max(nchain, 1) * nrhs, 0ull);
-            if ((e = upload(queue, qz.data(), qz.size()))) return e;
         }
-        // flags start below the first epoch
+        // flags start below the first epoch, queue entries of epoch 0 never
+        // match a launch
+        const size_t cells = (size_t)std::max(nchain, 1) * nrhs;
         FlowState f0{};
         f0.epoch = 1;
         f0.tail = nroots;
         const std::vector<FlowState> fv(nrhs, f0);
-        if ((e = upload(fs, fv.data(), fv.size()))) return e;
+        for (int k = 0; k < sets; ++k) {
+            live.push_back(std::make_unique<Live>());
+            Live& v = *live.back();
+            if ((e = upload(v.fs, fv.data(), fv.size()))) return e;
+            if (!ready) {
+                if ((e = upload(v.flag, std::vector<int>(cells, 0).data(), cells))) return e;
+                continue;
+            }
+            if ((e = upload(v.arrivals, std::vector<unsigned>(cells, 0u).data(), cells))) return e;
+            if ((e = upload(v.queue, std::vector<unsigned long long>(cells, 0ull).data(), cells))) return e;
+        }
         return OK;
     }
-    ReadyTables tables() const {
+    ReadyTables tables(int set) const {
         ReadyTables r;
         r.lo = lo.p;
         r.hi = hi.p;
@@ -1380,82 +1396,84 @@ struct FlowDev {
         r.succPtr = succPtr.p;
         r.succ = succ.p;
         r.roots = roots.p;
-        r.arrivals = arrivals.p;
-        r.queue = queue.p;
-        r.fs = fs.p;
+        r.arrivals = live[set]->arrivals.p;
+        r.queue = live[set]->queue.p;
+        r.fs = live[set]->fs.p;
         r.nchain = nchain;
         r.nroots = nroots;
-        r.pollLimit = kFlowPollLimit;
+        r.pollLimit = pollLimit;
         return r;
     }
     int aborts(int* out) const {
         *out = 0;
-        if (!fs.p) return OK;
-        std::vector<FlowState> f(nrhs);
-        RACE_HIP(hipMemcpy(f.data(), fs.p, sizeof(FlowState) * nrhs, hipMemcpyDeviceToHost));
-        for (const FlowState& q : f) *out += q.aborts;
+        for (const auto& v : live) {
+            std::vector<FlowState> f(nrhs);
+            RACE_HIP(hipMemcpy(f.data(), v->fs.p, sizeof(FlowState) * nrhs, hipMemcpyDeviceToHost));
+            for (const FlowState& q : f) *out += q.aborts;
+        }
         return OK;
     }
 };
 
 template <int TPR, int EE, typename VT, typename XT>
-int launchFlow(const BundleDev<VT, XT>& d, FlowDev& f, XT* x, const XT* b, hipStream_t st) {
+int launchFlow(const BundleDev<VT, XT>& d, FlowDev& f, int set, XT* x, const XT* b, hipStream_t st) {
     constexpr int BS = 256;
     auto kern = k_gs_flow<BS, TPR, EE, VT, XT>;
     hipLaunchKernelGGL(kern, dim3(f.grid), dim3(BS), f.lds, st, d.slot.p, d.wave.p, d.off.p, d.len.p, d.extPtr.p,
                        d.slotWave.p, d.rowId.p, d.diag.p, f.ext.p, d.sidx.p, d.sval.p, d.zero, x, b, f.lo.p, f.hi.p,
-                       f.nchain, f.depPtr.p, f.dep.p, f.flag.p, f.fs.p, kFlowPollLimit);
+                       f.nchain, f.depPtr.p, f.dep.p, f.live[set]->flag.p, f.live[set]->fs.p, f.pollLimit);
     RACE_HIP(hipGetLastError());
     return OK;
 }
 
 template <typename VT, typename XT>
-int launchFlowShape(int tpr, int E, const BundleDev<VT, XT>& d, FlowDev& f, XT* x, const XT* b, hipStream_t st) {
+int launchFlowShape(int tpr, int E, const BundleDev<VT, XT>& d, FlowDev& f, int set, XT* x, const XT* b,
+                    hipStream_t st) {
     switch (tpr * 100 + E) {
-        case 104: return launchFlow<1, 4>(d, f, x, b, st);
-        case 108: return launchFlow<1, 8>(d, f, x, b, st);
-        case 116: return launchFlow<1, 16>(d, f, x, b, st);
-        case 208: return launchFlow<2, 8>(d, f, x, b, st);
-        case 213: return launchFlow<2, 13>(d, f, x, b, st);
-        case 216: return launchFlow<2, 16>(d, f, x, b, st);
-        case 408: return launchFlow<4, 8>(d, f, x, b, st);
-        case 416: return launchFlow<4, 16>(d, f, x, b, st);
+        case 104: return launchFlow<1, 4>(d, f, set, x, b, st);
+        case 108: return launchFlow<1, 8>(d, f, set, x, b, st);
+        case 116: return launchFlow<1, 16>(d, f, set, x, b, st);
+        case 208: return launchFlow<2, 8>(d, f, set, x, b, st);
+        case 213: return launchFlow<2, 13>(d, f, set, x, b, st);
+        case 216: return launchFlow<2, 16>(d, f, set, x, b, st);
+        case 408: return launchFlow<4, 8>(d, f, set, x, b, st);
+        case 416: return launchFlow<4, 16>(d, f, set, x, b, st);
         default: return ERR_INTERNAL;
     }
 }
 
 // Kaczmarz one-launch sweep: grid (resident workgroups per side, nrhs)
 template <int BS, int TPR, int EE, typename VT, typename XT, bool BATCH>
-int launchKaczFlow(const BundleDev<VT, XT>& d, FlowDev& f, XT* x, const XT* b, int n, XT* const* bX,
+int launchKaczFlow(const BundleDev<VT, XT>& d, FlowDev& f, int set, XT* x, const XT* b, int n, XT* const* bX,
                    const XT* const* bB, const int* bN, hipStream_t st) {
     if constexpr (TPR == 0) {
         hipLaunchKernelGGL((k_kacz_flow_vl<BS, VT, XT, BATCH>), dim3(f.grid, f.nrhs), dim3(BS), f.lds, st, d.slot.p,
                            d.wave.p, d.off.p, d.len.p, d.extPtr.p, d.slotWave.p, d.rowId.p, d.rowNorm.p, f.ext.p,
                            d.sidx.p, d.sval.p, d.zero, x, b, n, f.maxLocal, f.spare, d.lanePtr.p, d.laneSlot.p, bX, bB, bN,
-                           f.tables());
+                           f.tables(set));
     } else {
         hipLaunchKernelGGL((k_kacz_flow<BS, TPR, EE, VT, XT, BATCH>), dim3(f.grid, f.nrhs), dim3(BS), f.lds, st,
                            d.slot.p, d.wave.p, d.off.p, d.len.p, d.extPtr.p, d.slotWave.p, d.rowId.p, d.rowNorm.p,
-                           f.ext.p, d.sidx.p, d.sval.p, d.zero, x, b, n, f.spare, bX, bB, bN, f.tables());
+                           f.ext.p, d.sidx.p, d.sval.p, d.zero, x, b, n, f.spare, bX, bB, bN, f.tables(set));
     }
     RACE_HIP(hipGetLastError());
     return OK;
 }
 
 template <typename VT, typename XT, bool BATCH>
-int launchKaczFlowShape(int bs, int tpr, int E, const BundleDev<VT, XT>& d, FlowDev& f, XT* x, const XT* b, int n,
-                        XT* const* bX, const XT* const* bB, const int* bN, hipStream_t st) {
+int launchKaczFlowShape(int bs, int tpr, int E, const BundleDev<VT, XT>& d, FlowDev& f, int set, XT* x, const XT* b,
+                        int n, XT* const* bX, const XT* const* bB, const int* bN, hipStream_t st) {
 #define RACE_KFLOW_CASE(BS_)                                                                                       \
     switch (tpr * 100 + E) {                                                                                       \
-        case 104: return launchKaczFlow<BS_, 1, 4, VT, XT, BATCH>(d, f, x, b, n, bX, bB, bN, st);                  \
-        case 108: return launchKaczFlow<BS_, 1, 8, VT, XT, BATCH>(d, f, x, b, n, bX, bB, bN, st);                  \
-        case 116: return launchKaczFlow<BS_, 1, 16, VT, XT, BATCH>(d, f, x, b, n, bX, bB, bN, st);                 \
-        case 208: return launchKaczFlow<BS_, 2, 8, VT, XT, BATCH>(d, f, x, b, n, bX, bB, bN, st);                  \
-        case 213: return launchKaczFlow<BS_, 2, 13, VT, XT, BATCH>(d, f, x, b, n, bX, bB, bN, st);                 \
-        case 216: return launchKaczFlow<BS_, 2, 16, VT, XT, BATCH>(d, f, x, b, n, bX, bB, bN, st);                 \
-        case 408: return launchKaczFlow<BS_, 4, 8, VT, XT, BATCH>(d, f, x, b, n, bX, bB, bN, st);                  \
-        case 416: return launchKaczFlow<BS_, 4, 16, VT, XT, BATCH>(d, f, x, b, n, bX, bB, bN, st);                 \
-        case 16: return launchKaczFlow<BS_, 0, kVarE, VT, XT, BATCH>(d, f, x, b, n, bX, bB, bN, st);               \
+        case 104: return launchKaczFlow<BS_, 1, 4, VT, XT, BATCH>(d, f, set, x, b, n, bX, bB, bN, st);                  \
+        case 108: return launchKaczFlow<BS_, 1, 8, VT, XT, BATCH>(d, f, set, x, b, n, bX, bB, bN, st);                  \
+        case 116: return launchKaczFlow<BS_, 1, 16, VT, XT, BATCH>(d, f, set, x, b, n, bX, bB, bN, st);                 \
+        case 208: return launchKaczFlow<BS_, 2, 8, VT, XT, BATCH>(d, f, set, x, b, n, bX, bB, bN, st);                  \
+        case 213: return launchKaczFlow<BS_, 2, 13, VT, XT, BATCH>(d, f, set, x, b, n, bX, bB, bN, st);                 \
+        case 216: return launchKaczFlow<BS_, 2, 16, VT, XT, BATCH>(d, f, set, x, b, n, bX, bB, bN, st);                 \
+        case 408: return launchKaczFlow<BS_, 4, 8, VT, XT, BATCH>(d, f, set, x, b, n, bX, bB, bN, st);                  \
+        case 416: return launchKaczFlow<BS_, 4, 16, VT, XT, BATCH>(d, f, set, x, b, n, bX, bB, bN, st);                 \
+        case 16: return launchKaczFlow<BS_, 0, kVarE, VT, XT, BATCH>(d, f, set, x, b, n, bX, bB, bN, st);               \
         default: return ERR_INTERNAL;                                                                              \
     }
     switch (bs) {
@@ -1541,6 +1559,42 @@ class BundleFn : public DeviceFn {
     // Kaczmarz with 256-1024-thread workgroups
     bool flow = false;
     FlowDev ff, fr;
+    // Small matrices sweep in one launch without the option.  A phase launch
+    // costs about 4.7 us however few its bundles, a level of the one-launch
+    // sweep about 3.3 us (a store, a flag, a poll and a gather through memory)
+    // while every chain finds a workgroup at once.  us per symmetric step, phase
+    // launches / one launch: Gauss-Seidel 27-point FP64 14^3 127 / 87, 40^3 141 /
+    // 108, 48^3 145 / 130 (864 chains), 52^3 147 / 155 (1100), FP32 48^3 132 / 127,
+    // 52^3 133 / 151: 896 chains, 3.5 per CU.  Kaczmarz 7-point FP64 20^3 102 / 67,
+    // 45^3 208 / 192, 64^3 266 / 219; FP32 20^3 90 / 62, 48^3 192 / 192, 50^3 194 /
+    // 205: with FP32 up to 1280 chains (48^3), with FP64 as far as measured.
+    // Long chains are left out: their coherent stores cost more than the
+    // launches (Chung-Lu graph of 20000 rows, 4 launches: 1916 / 2064).
+    // Sweeps that overlap need sets of their own, so each of the first kSets
+    // streams gets one; other streams and captured launches run the phases.
+    static constexpr int kSets = 2, kAutoBundles = 4;
+    static int autoChains(int kind) { return kind == RACE_K_GS ? 896 : sizeof(XT) == 8 ? 16384 : 1280; }
+    bool autoFlow = false;
+    std::mutex setLock;
+    std::vector<hipStream_t> setOwner;
+    // the set for a launch on st, -1 for the phase launches
+    int setFor(hipStream_t st) {
+        if (flow) return 0;
+        if (!autoFlow || st == nullptr || st == hipStreamLegacy || st == hipStreamPerThread) return -1;
+        hipStreamCaptureStatus cap;
+        if (hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) return -1;
+        std::lock_guard<std::mutex> g(setLock);
+        const auto at = std::find(setOwner.begin(), setOwner.end(), st);
+        if (at != setOwner.end()) return (int)(at - setOwner.begin());
+        if ((int)setOwner.size() == kSets) return -1;
+        setOwner.push_back(st);
+        return (int)setOwner.size() - 1;
+    }
+    static bool autoFits(const BundleTable& t) {
+        int longest = 0;
+        for (size_t c = 0; c + 1 < t.chainPtr.size(); ++c) longest = std::max(longest, t.chainPtr[c + 1] - t.chainPtr[c]);
+        return t.numPhases() >= 3 && longest <= kAutoBundles;
+    }
 
     int init(const race_kernel_desc& d, const ExecContext& ctx) {
         kind = d.kind;
@@ -1575,25 +1629,32 @@ class BundleFn : public DeviceFn {
             if (dr.lds(p, bs).bytes > kMaxLds) return fallBack();
         const bool gsFlow = kind == RACE_K_GS && nrhs == 1 && bs == 256 && tpr > 0;
         const bool kaczFlow = kind == RACE_K_KACZ && kaczFlowBs(bs);
-        if (ctx.flow && (gsFlow || kaczFlow)) {
+        const int chains = std::max((int)df.h.chainPtr.size(), (int)dr.h.chainPtr.size()) - 1;
+        const bool small =
+            ctx.flow < 0 && (long)chains * nrhs <= autoChains(kind) && autoFits(df.h) && autoFits(dr.h);
+        if ((ctx.flow > 0 || small) && (gsFlow || kaczFlow)) {
+            const int sets = small ? kSets : 1;
             const int sides = kind == RACE_K_KACZ ? nrhs : 1;
             const void* kern =
                 kind == RACE_K_KACZ ? kaczFlowKernel<VT, XT, false>(bs, tpr, E) : gsFlowKernel<VT, XT>(tpr, E);
             if (!kern) return ERR_INTERNAL;
             const bool ready = kind == RACE_K_KACZ;
-            if ((e = ff.init(df, n, nullptr, bs, sides, kern, ready)) ||
-                (e = fr.init(dr, n, nullptr, bs, sides, kern, ready)))
+            if ((e = ff.init(df, n, nullptr, bs, sides, kern, ready, sets)) ||
+                (e = fr.init(dr, n, nullptr, bs, sides, kern, ready, sets)))
                 return e;
             // conflicts inside a phase would serialise its chains, and one
             // LDS layout serves every phase: keep the phase launches if
             // either does not hold
-            flow = ff.samePhase == 0 && fr.samePhase == 0 && ff.lds <= kMaxLds && fr.lds <= kMaxLds;
+            const bool ok = ff.samePhase == 0 && fr.samePhase == 0 && ff.lds <= kMaxLds && fr.lds <= kMaxLds;
+            flow = ok && !small;
+            autoFlow = ok && small;
+            if (small) ff.pollLimit = fr.pollLimit = kAutoPollLimit;
         }
         return OK;
     }
     int flowAborts(int* out) const override {
         *out = 0;
-        if (!flow) return OK;
+        if (!flow && !autoFlow) return OK;
         int a = 0, c = 0, e;
         if ((e = ff.aborts(&a)) || (e = fr.aborts(&c))) return e;
         *out = a + c;
@@ -1607,7 +1668,7 @@ class BundleFn : public DeviceFn {
     bool graphable() const override { return fallback ? fallback->graphable() : true; }
     int launches(bool rev) const override {
         if (fallback) return fallback->launches(rev);
-        if (flow) return 1;
+        if (flow || autoFlow) return 1;
         const std::vector<int>& pc = (rev ? dr : df).h.phaseChain;
         int k = 0;
         for (size_t p = 0; p + 1 < pc.size(); ++p) k += pc[p + 1] > pc[p];
@@ -1620,10 +1681,11 @@ class BundleFn : public DeviceFn {
             return fallback->run(rev, st);
         }
         const Dev& d = rev ? dr : df;
-        if (flow && kind == RACE_K_KACZ)
-            return launchKaczFlowShape<VT, XT, false>(bs, tpr, E, d, rev ? fr : ff, (XT*)x, (const XT*)b, n, nullptr,
-                                                      nullptr, nullptr, st);
-        if (flow) return launchFlowShape<VT, XT>(tpr, E, d, rev ? fr : ff, (XT*)x, (const XT*)b, st);
+        const int set = setFor(st);
+        if (set >= 0 && kind == RACE_K_KACZ)
+            return launchKaczFlowShape<VT, XT, false>(bs, tpr, E, d, rev ? fr : ff, set, (XT*)x, (const XT*)b, n,
+                                                      nullptr, nullptr, nullptr, st);
+        if (set >= 0) return launchFlowShape<VT, XT>(tpr, E, d, rev ? fr : ff, set, (XT*)x, (const XT*)b, st);
         const std::vector<int>& pc = d.h.phaseChain;
         for (int p = 0; p + 1 < (int)pc.size(); ++p) {
             const int c0 = pc[p], nchain = pc[p + 1] - pc[p];
@@ -1824,7 +1886,7 @@ class BundleBatchFn : public DeviceFn {
                 Group& g = *groups[launchOrder[dir][q]];
                 hipStream_t s = q == 0 ? st : side[q - 1];
                 if (q > 0) RACE_HIP(hipStreamWaitEvent(s, forkEv, 0));
-                int e = launchKaczFlowShape<VT, XT, true>(bs, g.tpr, g.E, g.dev[dir], g.flow[dir], nullptr, nullptr,
+                int e = launchKaczFlowShape<VT, XT, true>(bs, g.tpr, g.E, g.dev[dir], g.flow[dir], 0, nullptr, nullptr,
                                                           0, g.bx[dir].p, g.bb[dir].p, g.bn[dir].p, s);
                 if (e) return e;
                 if (q > 0) RACE_HIP(hipEventRecord(joinEv[q - 1], s));

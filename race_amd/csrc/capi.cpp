@@ -109,7 +109,7 @@ struct race_handle_s {
     std::vector<Function> funcs;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     int optLayout = 0, optBundleRows = 128, optBundleLocal = 6144, optBundleThreads = 256, optBundleTpr = 0, optXcd = 0;
-    int optBfsBlockMax = 1 << 17, optSymmMode = 0, optGraph = 0, optFlow = 0;
+    int optBfsBlockMax = 1 << 17, optSymmMode = 0, optGraph = 0, optFlow = -1;
     ~race_handle_s() {
         if (ev0) (void)hipEventDestroy(ev0);
         if (ev1) (void)hipEventDestroy(ev1);

@@ -65,7 +65,7 @@ struct ExecContext {
     int symmMode = 0;         // SymmSpMV: 0 auto, 1 colour phases, 2 SELL atomics, 3 expanded
     int sellC = 64;           // batched SELL kernels: rows per chunk (8, 16, 32, 64)
     int sellSigma = 1;        // batched SELL kernels: row-sorting window (1 = unsorted)
-    int flow = 0;             // Gauss-Seidel: one launch per sweep with per-chain dependency flags
+    int flow = 0;             // one launch per sweep with per-chain dependencies: 1 yes, 0 no, -1 by size
 };
 
 int makeDeviceFn(const race_kernel_desc& d, const ExecContext& ctx, std::unique_ptr<DeviceFn>* out);

@@ -247,3 +247,64 @@ def test_flow_batch_async_sweeps_in_order():
     for ce, (xa, xb) in keep:
         assert np.array_equal(xa.download(), xb.download())
     assert batches[0].flowAborts() == 0 and batches[1].flowAborts() == 0
+
+
+# --- without the option: small matrices sweep in one launch by themselves
+
+@pytest.mark.parametrize("kind", [R.K_GS, R.K_KACZ])
+def test_default_sweeps_on_overlapping_streams(kind):
+    """A function called on several streams at once, each call with vectors
+    of its own: the first two streams sweep in one launch with state of their
+    own, further ones by phases; all equal the phase launches bit for bit."""
+    rp, col = M.stencil27(12) if kind == R.K_GS else M.stencil7(14)
+    val = M.gs_values(rp, col, seed=5)
+    n = len(rp) - 1
+    ce = R.Interface(n, 64, R.ONE if kind == R.K_GS else R.TWO, rp, col, symm_hint=True)
+    ce.RACEColor()
+    A = M.make_diag_first(*M.permute(rp, col, val, ce.getPerm(), ce.getInvPerm()))
+    owners = [R.Interface(n, 1, R.ONE, rp, col, symm_hint=True) for _ in range(4)]
+    streams = [o.stream() for o in owners]
+    vecs = [(R.DeviceArray.from_host(np.zeros(n)), R.DeviceArray.from_host(M.uniform_vec(n, k))) for k in range(4)]
+    refs = [R.DeviceArray.from_host(np.zeros(n)) for _ in range(4)]
+    fid = ce.registerDevice(kind, *A, *vecs[0])
+    assert ce.launchCount(fid) == 1
+    ce.setOption("flow", 0)
+    ref = ce.registerDevice(kind, *A, *vecs[0])
+    assert ce.launchCount(ref) > 1
+    for step in range(6):
+        print("case default flow", kind, step, flush=True)
+        for k, s in enumerate(streams):
+            ce.setVectors(fid, *vecs[k])
+            for rev in (False, True):
+                ce.executeAsync(fid, rev, s)
+    assert ce.flowAborts(fid) == 0  # waits for the device
+    for k in range(4):
+        ce.setVectors(ref, refs[k], vecs[k][1])
+        for step in range(6):
+            for rev in (False, True):
+                ce.executeFunction(ref, rev)
+        assert np.array_equal(vecs[k][0].download(), refs[k].download()), k
+    assert ce.flowAborts(fid) == 0
+
+
+@pytest.mark.parametrize("g,expect", [(4, None), (10, 1), (48, 1), (60, 0)])
+def test_default_sweep_by_size(g, expect):
+    """one launch up to the size line, phase launches past it, equal results"""
+    rp, col = M.stencil27(g)
+    val = M.gs_values(rp, col, seed=5)
+    n = len(rp) - 1
+    ce = R.Interface(n, max(1, n // 16), R.ONE, rp, col, symm_hint=True)
+    ce.RACEColor()
+    A = M.make_diag_first(*M.permute(rp, col, val, ce.getPerm(), ce.getInvPerm()))
+    b = R.DeviceArray.from_host(M.uniform_vec(n, 1))
+    xa, xb = R.DeviceArray.from_host(np.zeros(n)), R.DeviceArray.from_host(np.zeros(n))
+    fa = ce.registerDevice(R.K_GS, *A, xa, b)
+    ce.setOption("flow", 0)
+    fb = ce.registerDevice(R.K_GS, *A, xb, b)
+    print("case default by size", g, ce.launchCount(fa), flush=True)
+    if expect is not None:
+        assert (ce.launchCount(fa) == 1) == bool(expect)
+    for rev in (False, True, False):
+        ce.executeFunction(fa, rev)
+        ce.executeFunction(fb, rev)
+        assert np.array_equal(xa.download(), xb.download())
