@@ -1415,10 +1415,9 @@ struct FlowDev {
     }
 };
 
-template <int TPR, int EE, typename VT, typename XT>
+template <int BS, int TPR, int EE, typename VT, typename XT>
 int launchFlow(const BundleDev<VT, XT>& d, FlowDev& f, int set, XT* x, const XT* b, hipStream_t st) {
-    constexpr int BS = 256;
-    auto kern = k_gs_flow<BS, TPR, EE, VT, XT>;
+    auto kern = k_gs_flow<BS, TPR, EE, VT, XT, BS == 512 ? 4 : 6>;
     hipLaunchKernelGGL(kern, dim3(f.grid), dim3(BS), f.lds, st, d.slot.p, d.wave.p, d.off.p, d.len.p, d.extPtr.p,
                        d.slotWave.p, d.rowId.p, d.diag.p, f.ext.p, d.sidx.p, d.sval.p, d.zero, x, b, f.lo.p, f.hi.p,
                        f.nchain, f.depPtr.p, f.dep.p, f.live[set]->flag.p, f.live[set]->fs.p, f.pollLimit);
@@ -1427,17 +1426,19 @@ int launchFlow(const BundleDev<VT, XT>& d, FlowDev& f, int set, XT* x, const XT*
 }
 
 template <typename VT, typename XT>
-int launchFlowShape(int tpr, int E, const BundleDev<VT, XT>& d, FlowDev& f, int set, XT* x, const XT* b,
+int launchFlowShape(int bs, int tpr, int E, const BundleDev<VT, XT>& d, FlowDev& f, int set, XT* x, const XT* b,
                     hipStream_t st) {
+    // 512 threads: four lanes per row only (BundleFn::fourLanes)
+    if (bs == 512 && tpr == 4) return launchFlow<512, 4, 8>(d, f, set, x, b, st);
     switch (tpr * 100 + E) {
-        case 104: return launchFlow<1, 4>(d, f, set, x, b, st);
-        case 108: return launchFlow<1, 8>(d, f, set, x, b, st);
-        case 116: return launchFlow<1, 16>(d, f, set, x, b, st);
-        case 208: return launchFlow<2, 8>(d, f, set, x, b, st);
-        case 213: return launchFlow<2, 13>(d, f, set, x, b, st);
-        case 216: return launchFlow<2, 16>(d, f, set, x, b, st);
-        case 408: return launchFlow<4, 8>(d, f, set, x, b, st);
-        case 416: return launchFlow<4, 16>(d, f, set, x, b, st);
+        case 104: return launchFlow<256, 1, 4>(d, f, set, x, b, st);
+        case 108: return launchFlow<256, 1, 8>(d, f, set, x, b, st);
+        case 116: return launchFlow<256, 1, 16>(d, f, set, x, b, st);
+        case 208: return launchFlow<256, 2, 8>(d, f, set, x, b, st);
+        case 213: return launchFlow<256, 2, 13>(d, f, set, x, b, st);
+        case 216: return launchFlow<256, 2, 16>(d, f, set, x, b, st);
+        case 408: return launchFlow<256, 4, 8>(d, f, set, x, b, st);
+        case 416: return launchFlow<256, 4, 16>(d, f, set, x, b, st);
         default: return ERR_INTERNAL;
     }
 }
@@ -1489,7 +1490,8 @@ inline bool kaczFlowBs(int bs) { return bs == 256 || bs == 512 || bs == 1024; }
 
 // the kernel a one-launch sweep of this shape runs (for its occupancy)
 template <typename VT, typename XT>
-const void* gsFlowKernel(int tpr, int E) {
+const void* gsFlowKernel(int bs, int tpr, int E) {
+    if (bs == 512 && tpr == 4) return reinterpret_cast<const void*>(k_gs_flow<512, 4, 8, VT, XT, 4>);
     switch (tpr * 100 + E) {
         case 104: return reinterpret_cast<const void*>(k_gs_flow<256, 1, 4, VT, XT>);
         case 108: return reinterpret_cast<const void*>(k_gs_flow<256, 1, 8, VT, XT>);
@@ -1590,6 +1592,23 @@ class BundleFn : public DeviceFn {
         setOwner.push_back(st);
         return (int)setOwner.size() - 1;
     }
+    // Gauss-Seidel rows of 17 to 32 entries off the diagonal: four lanes per
+    // row (8 entries a lane instead of 16) and 64 rows per bundle where the
+    // chain of waves counts more than the bytes.  us per symmetric step of a
+    // 27-point grid, 128 rows x 2 lanes / 64 x 4.  One launch per sweep, FP64
+    // 14^3 87 / 82, FP32 84 / 72; 40^3 FP64 107 / 136, as twice the chains no longer
+    // find a workgroup at once: up to 256 bundles of 64 rows.  One launch per
+    // phase, past the sizes of the one-launch sweep: FP32 56^3 167 / 156, 100^3 229 /
+    // 213, 128^3 324 / 318, BF16 56^3 207 / 178; FP64 gains 2 % at 56^3 and loses 4 %
+    // at 128^3 to the outside columns that smaller bundles share less, and keeps
+    // two lanes.  By size alone, not by the flow option: the lanes of a row set
+    // the order of its sum, and both kinds of launches give the same bits.  With
+    // the option on, larger matrices take 512 threads for the same 128 rows
+    // (FP32 64^3 204 us with two lanes, 177 with 512 threads, 268 with 64 rows).
+    bool fourLanes() const {
+        if (kind != RACE_K_GS || nrhs != 1) return false;
+        return n <= 256 * 64 || (sizeof(XT) == 4 && n > 128 * autoChains(kind));
+    }
     static bool autoFits(const BundleTable& t) {
         int longest = 0;
         for (size_t c = 0; c + 1 < t.chainPtr.size(); ++c) longest = std::max(longest, t.chainPtr[c + 1] - t.chainPtr[c]);
@@ -1607,7 +1626,15 @@ class BundleFn : public DeviceFn {
         int maxLen = 0;
         for (int r = 0; r < n; ++r) maxLen = std::max(maxLen, d.rowPtr[r + 1] - d.rowPtr[r]);
         pickShape(kind, maxLen, ctx.bundleTpr, &tpr, &E);
-        const int rowsCap = rowsCapFor(ctx.bundleRows, bs, tpr);
+        int rowsCap = rowsCapFor(ctx.bundleRows, bs, tpr);
+        bool flowWide = false;
+        if (tpr == 2 && ctx.bundleTpr == 0 && ctx.bundleRows == 128 && bs == 256 && fourLanes()) {
+            tpr = 4;
+            E = pickE(4, (maxLen - 1 + 3) / 4);
+            flowWide = ctx.flow > 0 && n > 256 * 64;
+            if (flowWide) bs = 512;
+            rowsCap = rowsCapFor(ctx.bundleRows, bs, tpr);
+        }
         const bool fp64 = std::is_same<VT, double>::value && std::is_same<XT, double>::value;
         auto fallBack = [&]() -> int {
             if (ctx.layout == 2 || !fp64) return ERR_INCOMPATIBILITY;  // bundles required
@@ -1627,7 +1654,7 @@ class BundleFn : public DeviceFn {
             if (df.lds(p, bs).bytes > kMaxLds) return fallBack();
         for (int p = 0; p < dr.h.numPhases(); ++p)
             if (dr.lds(p, bs).bytes > kMaxLds) return fallBack();
-        const bool gsFlow = kind == RACE_K_GS && nrhs == 1 && bs == 256 && tpr > 0;
+        const bool gsFlow = kind == RACE_K_GS && nrhs == 1 && (bs == 256 || flowWide) && tpr > 0;
         const bool kaczFlow = kind == RACE_K_KACZ && kaczFlowBs(bs);
         const int chains = std::max((int)df.h.chainPtr.size(), (int)dr.h.chainPtr.size()) - 1;
         const bool small =
@@ -1636,7 +1663,7 @@ class BundleFn : public DeviceFn {
             const int sets = small ? kSets : 1;
             const int sides = kind == RACE_K_KACZ ? nrhs : 1;
             const void* kern =
-                kind == RACE_K_KACZ ? kaczFlowKernel<VT, XT, false>(bs, tpr, E) : gsFlowKernel<VT, XT>(tpr, E);
+                kind == RACE_K_KACZ ? kaczFlowKernel<VT, XT, false>(bs, tpr, E) : gsFlowKernel<VT, XT>(bs, tpr, E);
             if (!kern) return ERR_INTERNAL;
             const bool ready = kind == RACE_K_KACZ;
             if ((e = ff.init(df, n, nullptr, bs, sides, kern, ready, sets)) ||
@@ -1685,7 +1712,7 @@ class BundleFn : public DeviceFn {
         if (set >= 0 && kind == RACE_K_KACZ)
             return launchKaczFlowShape<VT, XT, false>(bs, tpr, E, d, rev ? fr : ff, set, (XT*)x, (const XT*)b, n,
                                                       nullptr, nullptr, nullptr, st);
-        if (set >= 0) return launchFlowShape<VT, XT>(tpr, E, d, rev ? fr : ff, set, (XT*)x, (const XT*)b, st);
+        if (set >= 0) return launchFlowShape<VT, XT>(bs, tpr, E, d, rev ? fr : ff, set, (XT*)x, (const XT*)b, st);
         const std::vector<int>& pc = d.h.phaseChain;
         for (int p = 0; p + 1 < (int)pc.size(); ++p) {
             const int c0 = pc[p], nchain = pc[p + 1] - pc[p];

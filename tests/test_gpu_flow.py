@@ -308,3 +308,26 @@ def test_default_sweep_by_size(g, expect):
         ce.executeFunction(fa, rev)
         ce.executeFunction(fb, rev)
         assert np.array_equal(xa.download(), xb.download())
+
+
+@pytest.mark.parametrize("prec", [R.FP64, R.FP32, R.BF16])
+@pytest.mark.parametrize("g", [25, 26, 50])
+def test_lanes_by_size(oracle, g, prec):
+    """27-point rows on both sides of the lines between two and four lanes per
+    row (16384 rows; 114688 rows in FP32 / BF16): RACE's order, and the same
+    bits from one launch per sweep (512 threads past the second line)."""
+    rp, col = M.stencil27(g)
+    val = M.gs_values(rp, col, seed=8)
+    n = len(rp) - 1
+    ce, A, zt = _prepared(rp, col, val, max(1, n // 16), R.ONE, oracle)
+    b = M.uniform_vec(n, 2)
+    (fa, xa), (fb, xb) = (_register(ce, *A, np.zeros(n), b, flow, prec) for flow in (0, 1))
+    xo = np.zeros(n)
+    for rev in (False, True):
+        print("case lanes", g, prec, rev, flush=True)
+        ce.executeFunction(fa, rev)
+        ce.executeFunction(fb, rev)
+        oracle.run_calls(oracle.K_GS, *A, xo, b, oracle.leaf_calls(zt, rev))
+        assert np.array_equal(xa.download(), xb.download())
+        assert relerr(xa.download(), xo) <= {R.FP64: TOL, R.FP32: 1e-6, R.BF16: 5e-3}[prec]
+    assert ce.flowAborts(fb) == 0
