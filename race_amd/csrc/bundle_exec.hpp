@@ -18,7 +18,6 @@
 #include <atomic>
 #include <cstdint>
 #include <cstring>
-#include <mutex>
 #include <thread>
 #include <type_traits>
 
@@ -1577,21 +1576,9 @@ class BundleFn : public DeviceFn {
     static constexpr int kSets = 2, kAutoBundles = 4;
     static int autoChains(int kind) { return kind == RACE_K_GS ? 896 : sizeof(XT) == 8 ? 16384 : 1280; }
     bool autoFlow = false;
-    std::mutex setLock;
-    std::vector<hipStream_t> setOwner;
+    StreamSets streamSets;
     // the set for a launch on st, -1 for the phase launches
-    int setFor(hipStream_t st) {
-        if (flow) return 0;
-        if (!autoFlow || st == nullptr || st == hipStreamLegacy || st == hipStreamPerThread) return -1;
-        hipStreamCaptureStatus cap;
-        if (hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) return -1;
-        std::lock_guard<std::mutex> g(setLock);
-        const auto at = std::find(setOwner.begin(), setOwner.end(), st);
-        if (at != setOwner.end()) return (int)(at - setOwner.begin());
-        if ((int)setOwner.size() == kSets) return -1;
-        setOwner.push_back(st);
-        return (int)setOwner.size() - 1;
-    }
+    int setFor(hipStream_t st) { return flow ? 0 : autoFlow ? streamSets.find(st, kSets) : -1; }
     // Gauss-Seidel rows of 17 to 32 entries off the diagonal: four lanes per
     // row (8 entries a lane instead of 16) and 64 rows per bundle where the
     // chain of waves counts more than the bytes.  us per symmetric step of a

@@ -2,8 +2,11 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <cstring>
+#include <mutex>
+#include <vector>
 
 #include "engine.hpp"
 #include "hip_util.hpp"
@@ -29,6 +32,30 @@ inline uint16_t toBf16(double v) {
     u += 0x7fffu + ((u >> 16) & 1u);
     return (uint16_t)(u >> 16);
 }
+
+// Which of a function's `sets` of scratch memory a launch on a stream may use:
+// launches of one function on different streams may overlap, so each of the
+// first streams gets a set of its own, for good.  -1 (run without scratch) for
+// further streams, for the streams whose handle stands for several, and while
+// the stream is captured (a graph may be replayed anywhere).
+class StreamSets {
+  public:
+    int find(hipStream_t st, int sets) {
+        if (st == nullptr || st == hipStreamLegacy || st == hipStreamPerThread) return -1;
+        hipStreamCaptureStatus cap;
+        if (hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) return -1;
+        std::lock_guard<std::mutex> g(lock);
+        const auto at = std::find(owner.begin(), owner.end(), st);
+        if (at != owner.end()) return (int)(at - owner.begin());
+        if ((int)owner.size() >= sets) return -1;
+        owner.push_back(st);
+        return (int)owner.size() - 1;
+    }
+
+  private:
+    std::mutex lock;
+    std::vector<hipStream_t> owner;
+};
 
 inline unsigned gridFor(long n, int block = kBlock) {
     long g = (n + block - 1) / block;

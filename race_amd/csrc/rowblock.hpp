@@ -69,6 +69,7 @@ struct RowBlocks {
     DevBuf<uint16_t> col16;
     DevBuf<VT> val;
     int nBlk = 0;
+    int cap = kRbEntries;  // entries of a block of several rows, set before add
 
     // rows [0, n) of one more matrix
     void add(int n, const int* R, const int* C, const double* V, int mat) {
@@ -78,10 +79,10 @@ struct RowBlocks {
         hval.reserve(hcol.capacity());
         for (int r = 0; r < n;) {
             RowBlk k{r, 0, (int)(hcol.size() / 4), 0, INT32_MAX, mat, rp0 + r, R[r]};
-            while (r < n && k.nrows < kRbRows && (k.nrows == 0 || R[r + 1] - k.p0 <= kRbEntries)) {
+            while (r < n && k.nrows < kRbRows && (k.nrows == 0 || R[r + 1] - k.p0 <= cap)) {
                 ++r;
                 ++k.nrows;
-                if (R[r] - k.p0 > kRbEntries) break;  // a long row, alone
+                if (R[r] - k.p0 > cap) break;  // a long row, alone
             }
             k.ne = R[r] - k.p0;
             int hi = 0;
@@ -233,6 +234,146 @@ __global__ void __launch_bounds__(kBlock) k_rowblk(RowBlkView<CT, VT> A, const X
             __syncthreads();
         }
     }
+}
+
+// The R values of one row of packed right-hand sides (k_pack_rhs).
+template <int R, typename XT>
+__device__ __forceinline__ void loadRow(const XT* __restrict__ p, XT (&out)[R]) {
+    constexpr int B = R * (int)sizeof(XT), V = B < 16 ? R : 16 / (int)sizeof(XT);
+    struct alignas(V * sizeof(XT)) P {
+        XT v[V];
+    };
+#pragma unroll
+    for (int s = 0; s < R / V; ++s) {
+        const P a = reinterpret_cast<const P*>(p)[s];
+#pragma unroll
+        for (int k = 0; k < V; ++k) out[s * V + k] = a.v[k];
+    }
+}
+
+// Right-hand sides q0 .. q0 + R - 1 (zeros past the last), row by row.  An
+// entry's R values of x are then R * sizeof(XT) consecutive bytes instead of R
+// separate cache lines.
+template <int R, typename XT>
+__global__ void __launch_bounds__(kBlock) k_pack_rhs(const XT* __restrict__ x, XT* __restrict__ packed, long n,
+                                                     int nrhs) {
+    const long r = (long)blockIdx.x * kBlock + threadIdx.x;
+    const int q0 = (int)blockIdx.y * R;
+    if (r >= n) return;
+    XT v[R];
+#pragma unroll
+    for (int q = 0; q < R; ++q) v[q] = q0 + q < nrhs ? x[(long)(q0 + q) * n + r] : XT(0);
+    constexpr int V = R * sizeof(XT) < 16 ? R : 16 / (int)sizeof(XT);
+    struct alignas(V * sizeof(XT)) P {
+        XT v[V];
+    };
+    P* o = reinterpret_cast<P*>(packed + ((long)blockIdx.y * n + r) * R);
+#pragma unroll
+    for (int s = 0; s < R / V; ++s) {
+        P a;
+#pragma unroll
+        for (int k = 0; k < V; ++k) a.v[k] = v[s * V + k];
+        o[s] = a;
+    }
+}
+
+// k_rowblk over packed right-hand sides, R per blockIdx.y.  Entries go to the
+// threads one by one (t, t + 256, ...), so that the products of neighbouring
+// lanes are neighbours in LDS.  Blocks of kPackedEntries leave 16 KB of products
+// (ten workgroups per CU).
+constexpr int kPackedEntries = 2 * kBlock;
+template <int R, typename CT, typename VT, typename XT>
+__global__ void __launch_bounds__(kBlock) k_rowblk_packed(RowBlkView<CT, VT> A, const XT* __restrict__ packed,
+                                                          XT* __restrict__ y, long n, int nrhs, int acc) {
+    __shared__ __align__(16) XT prod[kPackedEntries * R];
+    const int t = threadIdx.x;
+    const RowBlk k = A.blks[blockIdx.x];
+    const int q0 = (int)blockIdx.y * R, q = t % R, slot = t / R;
+    const XT* __restrict__ x = packed + ((long)blockIdx.y * n + k.base) * R;
+    const CT* __restrict__ col = A.col + (long)k.e0 * 4;
+    const VT* __restrict__ val = A.val + (long)k.e0 * 4;
+    const int ne = k.ne;
+    auto put = [&](int at, const XT (&v)[R]) {
+#pragma unroll
+        for (int u = 0; u < R; ++u) prod[at * R + u] = v[u];
+    };
+    if (ne <= kPackedEntries) {
+        // entries past the block's last read its first and are not summed
+        constexpr int N = kPackedEntries / kBlock;
+        CT c[N];
+        VT v[N];
+#pragma unroll
+        for (int u = 0; u < N; ++u) {
+            const int j = t + u * kBlock < ne ? t + u * kBlock : 0;
+            c[u] = col[j];
+            v[u] = val[j];
+        }
+        XT g[N][R];
+#pragma unroll
+        for (int u = 0; u < N; ++u) loadRow<R>(x + (long)(unsigned)c[u] * R, g[u]);
+#pragma unroll
+        for (int u = 0; u < N; ++u) {
+#pragma unroll
+            for (int p = 0; p < R; ++p) g[u][p] *= fromStorage<XT>(v[u]);
+            put(t + u * kBlock, g[u]);
+        }
+        __syncthreads();
+        // slots of R lanes; as many slots per row as the rows leave, inside
+        // one wavefront
+        constexpr int S = kBlock / R, W = 64 / R;
+        const int lg = min(31 - __clz(max(1, S / k.nrows)), 31 - __clz(W));
+        const int l = slot & ((1 << lg) - 1);
+        for (int r0 = 0; r0 < k.nrows; r0 += S >> lg) {
+            const int r = r0 + (slot >> lg);
+            const bool live = r < k.nrows;
+            const int lo = live ? A.rp[k.rp0 + r] - k.p0 : 0, hi = live ? A.rp[k.rp0 + r + 1] - k.p0 : 0;
+            const long at = (long)(q0 + q) * n + k.row0 + r;
+            const bool store = live && l == 0 && q0 + q < nrhs;
+            const XT old = acc && store ? y[at] : XT(0);
+            // four products in flight
+            XT s = XT(0);
+            const int step = R << lg;
+            int i = (lo + l) * R + q;
+            const int end = hi * R;
+            for (; i + 3 * step < end; i += 4 * step) {
+                const XT a = prod[i], b = prod[i + step], c2 = prod[i + 2 * step], d = prod[i + 3 * step];
+                s += (a + b) + (c2 + d);
+            }
+            for (; i < end; i += step) s += prod[i];
+            for (int o = (1 << lg) / 2; o > 0; o >>= 1) s += __shfl_xor(s, o * R);
+            if (store) y[at] = old + s;
+        }
+    } else {
+        XT s[R] = {};
+        for (int j = t; j < ne; j += kBlock) {
+            XT g[R];
+            loadRow<R>(x + (long)(unsigned)col[j] * R, g);
+            const XT v = fromStorage<XT>(val[j]);
+#pragma unroll
+            for (int u = 0; u < R; ++u) s[u] += v * g[u];
+        }
+        put(t, s);
+        __syncthreads();
+        for (int o = kBlock / 2; o > 0; o >>= 1) {
+            for (int i = t; i < o * R; i += kBlock) prod[i] += prod[i + o * R];
+            __syncthreads();
+        }
+        if (t < R && q0 + t < nrhs) {
+            const long at = (long)(q0 + t) * n + k.row0;
+            y[at] = acc ? y[at] + prod[t] : prod[t];
+        }
+    }
+}
+
+template <int R, typename VT, typename XT>
+void launchRowBlkPacked(const RowBlocks<VT>& A, const XT* packed, XT* y, long n, int nrhs, bool acc, hipStream_t st) {
+    const dim3 grid(A.nBlk, (nrhs + R - 1) / R);
+    if (A.narrowIds)
+        hipLaunchKernelGGL((k_rowblk_packed<R, uint16_t, VT, XT>), grid, dim3(kBlock), 0, st,
+                           A.template view<uint16_t>(nullptr), packed, y, n, nrhs, (int)acc);
+    else
+        hipLaunchKernelGGL((k_rowblk_packed<R, int, VT, XT>), grid, dim3(kBlock), 0, st, A.template view<int>(nullptr),
+                           packed, y, n, nrhs, (int)acc);
 }
 
 // one launch over all blocks.  Right-hand sides share a pass over the entries

@@ -412,12 +412,65 @@ struct Product {
     RowBlocks<VT> blocks;
     int n = 0;
     bool useBlocks = false;
+    // Several right-hand sides over row blocks may be packed row by row first
+    // (k_pack_rhs, one more launch and pass over x), into scratch of the
+    // launch's stream (StreamSets).  Then an entry takes one cache line of x
+    // for all of them instead of one each, and one or two trips through the
+    // address unit instead of nrhs.  It pays where columns are scattered over
+    // x, so that every gather is a line of its own; where lines are shared
+    // (kScattered) only with many entries.  us, separate columns / packed:
+    // Chung-Lu graph 150000 rows, 3.0M entries FP32 2 / 3 / 8 sides 37 / 23, 71 / 27,
+    // 162 / 40, FP64 8 sides 224 / 62; 20000 rows, 0.4M, FP32 2 / 8 sides 13.0 / 8.1,
+    // 50 / 12; random band of 200000 rows, 7.9M FP32 2 / 3 / 8 sides 32 / 33, 55 /
+    // 41, 104 / 55; 90001 rows, 1.9M FP32 3 / 8 sides 13.0 / 12.9, 26 / 20; 200000
+    // rows, 1.2M, FP32 8 sides 20 / 23.  Chunks of stencils gather coalesced lines
+    // as they are (27-point 96^3 FP64 8 sides 135 / 158).
+    static constexpr int kSets = 2;
+    static constexpr double kScattered = 0.4;
+    DevBuf<XT> packed[kSets];
+    StreamSets streamSets;
+    int rhs = 1, R = 0;  // R: right-hand sides of a packed row, 0: not packed
     int build(const race_kernel_desc& d) {
         n = d.nrow;
+        rhs = d.kind == RACE_K_MPK || d.kind == RACE_K_MPK_HIGHEST ? 1 : std::max(1, d.nrhs);
         useBlocks = ragged(d);
+        if (rhs > 1) {
+            const int w = rhs == 2 ? 2 : rhs <= 4 || sizeof(XT) == 8 ? 4 : 8, planes = (rhs + w - 1) / w;
+            const long nnz = d.rowPtr[n];
+            const bool scattered = nnz * (rhs - 1) >= 200000 && linesPerEntry(d) > kScattered;
+            if (scattered || (useBlocks && nnz * (rhs - planes) >= 10000000)) {
+                useBlocks = true;
+                R = w;
+                blocks.cap = kPackedEntries;
+                for (DevBuf<XT>& b : packed) RACE_HIP(b.reserve((size_t)n * planes * R));
+            }
+        }
         if (!useBlocks) return sell.build(d);
         blocks.add(n, d.rowPtr, d.col, d.val, 0);
         return blocks.finish();
+    }
+    // distinct 128-byte lines of x per entry, in runs of kPackedEntries entries
+    // (up to 2000 runs, spread over the matrix)
+    static double linesPerEntry(const race_kernel_desc& d) {
+        const long nnz = d.rowPtr[d.nrow], run = kPackedEntries;
+        if (nnz < run) return 0.0;
+        const long runs = nnz / run, step = std::max(1l, runs / 2000);
+        constexpr int perLine = 128 / (int)sizeof(XT);
+        std::vector<int> seen((size_t)d.nrow / perLine + 1, -1);
+        long lines = 0, entries = 0;
+        for (long k = 0; k < runs; k += step, entries += run)
+            for (long j = k * run; j < (k + 1) * run; ++j) {
+                int& s = seen[d.col[j] / perLine];
+                lines += s != (int)k;
+                s = (int)k;
+            }
+        return (double)lines / (double)entries;
+    }
+    template <int RR>
+    void runPacked(const XT* x, XT* y, XT* buf, bool acc, hipStream_t st) const {
+        hipLaunchKernelGGL((k_pack_rhs<RR, XT>), dim3(gridFor(n), (rhs + RR - 1) / RR), dim3(kBlock), 0, st, x, buf,
+                           (long)n, rhs);
+        launchRowBlkPacked<RR, VT, XT>(blocks, buf, y, n, rhs, acc, st);
     }
     static bool ragged(const race_kernel_desc& d) {
         long slots = 0;
@@ -429,7 +482,14 @@ struct Product {
         return slots * kC * 4 > (long)d.rowPtr[d.nrow] * 5;
     }
     // y = A x (acc: y += A x)
-    void run(const void* x, void* y, int nrhs, bool acc, hipStream_t st) const {
+    void run(const void* x, void* y, int nrhs, bool acc, hipStream_t st) {
+        const int set = R && nrhs == rhs ? streamSets.find(st, kSets) : -1;
+        if (set >= 0) {
+            XT* buf = packed[set].p;
+            if (R == 2) return runPacked<2>((const XT*)x, (XT*)y, buf, acc, st);
+            if (R == 4) return runPacked<4>((const XT*)x, (XT*)y, buf, acc, st);
+            if constexpr (sizeof(XT) == 4) return runPacked<8>((const XT*)x, (XT*)y, buf, acc, st);
+        }
         if (useBlocks)
             launchRowBlk<false, VT, XT>(blocks, nullptr, x, y, n, nrhs, acc, st);
         else
@@ -442,6 +502,7 @@ template <typename VT, typename XT>
 class SellSpmvFn : public DeviceFn {
   public:
     Product<VT, XT> A;
+    int launches(bool) const override { return A.R ? 2 : 1; }
     int nrhs = 1;
     int init(const race_kernel_desc& d) {
         kind = d.kind;
@@ -466,6 +527,7 @@ template <typename VT, typename XT>
 class SymmSellFn : public DeviceFn {
   public:
     Product<VT, XT> A;
+    int launches(bool) const override { return A.R ? 2 : 1; }
     int mode = 2, nrhs = 1;
     int init(const race_kernel_desc& d, int mode_) {
         kind = d.kind;
@@ -610,6 +672,7 @@ template <typename VT, typename XT>
 class SpmtvFn : public DeviceFn {
   public:
     Product<VT, XT> A;
+    int launches(bool) const override { return A.R ? 2 : 1; }
     int nrhs = 1;
     int init(const race_kernel_desc& d) {
         kind = d.kind;

@@ -160,3 +160,42 @@ def test_row_blocks_wide_ids():
     col = rng.integers(0, n, rp[-1]).astype(np.int32)
     for prec, nrhs in ((R.FP64, 1), (R.FP32, 4)):
         _check(rp, col, rng.uniform(-1, 1, len(col)), R.K_SPMV, prec, nrhs)
+
+
+@pytest.mark.parametrize("kind", [R.K_SPMV, R.K_SPMTV])
+@pytest.mark.parametrize("nrhs", [2, 3, 4, 5, 8, 9])
+def test_packed_right_hand_sides(nrhs, kind):
+    """scattered columns: right-hand sides packed row by row, full and partly
+    filled blocks of them; rows of 0, 512, 513 and 3000 entries"""
+    n = 6000
+    lengths = [int(k) for k in np.random.default_rng(3).integers(0, 60, n)]
+    lengths[5], lengths[6], lengths[7], lengths[4000], lengths[-1] = 512, 513, 1024, 3000, 0
+    for prec in (R.FP64, R.FP32, R.BF16):
+        print("case packed", nrhs, kind, prec, flush=True)
+        rp, col, val = _random(n, lengths, 7)
+        _check(rp, col, val, kind, prec, nrhs)
+
+
+def test_packed_on_overlapping_streams():
+    """one function on four streams at once, each call with vectors of its
+    own: two streams with packing scratch, the others without"""
+    n, nrhs = 20000, 4
+    rng = np.random.default_rng(1)
+    lengths = rng.integers(0, 40, n)
+    rp = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int32)
+    col = rng.integers(0, n, rp[-1]).astype(np.int32)
+    val = rng.uniform(-1, 1, len(col))
+    owners = [R.Interface(n, 1, R.ONE, rp, col, symm_hint=False) for _ in range(4)]
+    xs = [M.uniform_vec(n, k, nrhs=nrhs) for k in range(4)]
+    vecs = [(R.DeviceArray.from_host(x), R.DeviceArray.from_host(np.zeros(n * nrhs))) for x in xs]
+    fid = owners[0].registerDevice(R.K_SPMV, rp, col, val, *vecs[0], nrhs=nrhs)
+    assert owners[0].launchCount(fid) == 2
+    for step in range(20):
+        for k, o in enumerate(owners):
+            owners[0].setVectors(fid, *vecs[k])
+            owners[0].executeAsync(fid, stream=o.stream())
+    assert owners[0].flowAborts(fid) == 0  # waits for the device
+    A = M.to_scipy(rp, col, val)
+    for k in range(4):
+        ref = (A @ xs[k].reshape(nrhs, n).T).T
+        assert np.max(np.abs(vecs[k][1].download().reshape(nrhs, n) - ref)) <= 60 * 2.0 ** -53 * 60
