@@ -138,6 +138,8 @@ RAGGED = {
     "all_empty": [0] * 700,
     # a block that ends by its row count, and hub rows among short ones
     "short_rows": [1, 0, 2] * 200 + [900] + [3] * 50,
+    # the longest row a lane or its lanes sum alone, and one entry more; as many hubs as a block holds
+    "hub_edges": [1] * 100 + [16] + [1] * 150 + [17] * 70 + [64, 65, 128, 129] + [0] * 250 + [33] * 9 + [1] * 240,
 }
 
 
