@@ -411,6 +411,50 @@ BundleTable concatBundles(const std::vector<const BundleTable*>& tabs, std::vect
     return t;
 }
 
+int residentChains(BundleTable& t, int minBundles, int maxCols) {
+    maxCols = std::min(maxCols, 65535);  // 16-bit local columns
+    const int nb = (int)t.slot.size() - 1;
+    std::vector<int> ext, extPtr(1, 0), cols;
+    std::vector<uint16_t> place;
+    int made = 0;
+    for (int p = 0; p < t.numPhases(); ++p)
+        for (int c = t.phaseChain[p]; c < t.phaseChain[p + 1]; ++c) {
+            const int b0 = t.chainPtr[c], b1 = t.chainPtr[c + 1];
+            cols.assign(t.ext.begin() + t.extPtr[b0], t.ext.begin() + t.extPtr[b1]);
+            if (b1 - b0 >= minBundles) {
+                std::sort(cols.begin(), cols.end());
+                cols.erase(std::unique(cols.begin(), cols.end()), cols.end());
+            }
+            if (b1 - b0 < minBundles || cols.empty() || (int)cols.size() > maxCols) {
+                for (int b = b0; b < b1; ++b) {
+                    ext.insert(ext.end(), t.ext.begin() + t.extPtr[b], t.ext.begin() + t.extPtr[b + 1]);
+                    extPtr.push_back((int)ext.size());
+                }
+                continue;
+            }
+            for (int b = b0; b < b1; ++b) {
+                // both lists ascend
+                place.clear();
+                for (int e = t.extPtr[b], q = 0; e < t.extPtr[b + 1]; ++e) {
+                    while (cols[q] != t.ext[e]) ++q;
+                    place.push_back((uint16_t)q);
+                }
+                const long end = b + 1 < nb ? t.off[b + 1] : (long)t.sidx.size();
+                if (!place.empty())  // else no entries
+                    for (long e = t.off[b]; e < end; ++e) t.sidx[e] = place[t.sidx[e]];
+                if (b == b0) ext.insert(ext.end(), cols.begin(), cols.end());
+                extPtr.push_back((int)ext.size());
+            }
+            t.phLocal[p] = std::max(t.phLocal[p], (int)cols.size());
+            ++made;
+        }
+    if (made > 0) {
+        t.ext = std::move(ext);
+        t.extPtr = std::move(extPtr);
+    }
+    return made;
+}
+
 }  // namespace race
 
 namespace race {

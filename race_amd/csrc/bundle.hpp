@@ -39,7 +39,8 @@ struct BundleTable {
     std::vector<int> len;           // bundle -> register entries per lane
     std::vector<int> extPtr;        // bundle -> first entry in ext
     std::vector<int> ext;           // global columns of the local column space
-                                    // (GS: outside columns; KACZ: all columns)
+                                    // (GS: outside columns; KACZ: all columns,
+                                    // or all of the chain, see residentChains)
     std::vector<int> rowId;         // slot -> matrix row
     std::vector<double> diag;       // slot -> diagonal value (GS)
     std::vector<double> rowNorm;    // slot -> sum of squares of the row (KACZ)
@@ -76,6 +77,12 @@ BundleTable buildBundles(const Schedule& s, int kind, int n, const int* rowPtr, 
 // ids and column ids stay those of their own matrix (each bundle of a batch
 // carries its own vectors).  bundleTable[k] = table of fused bundle k.
 BundleTable concatBundles(const std::vector<const BundleTable*>& tabs, std::vector<int>* bundleTable);
+
+// Kaczmarz: one local column space for all bundles of a chain where the chain
+// has at least minBundles bundles and touches at most maxCols columns.  Its
+// first bundle lists the chain's columns, the others none.  Returns the number
+// of such chains.
+int residentChains(BundleTable& t, int minBundles, int maxCols);
 
 // Dependencies between the chains of one sweep, for a launch that runs all
 // of them in chain order (phase order) with a completion flag per chain

@@ -542,7 +542,18 @@ __device__ __forceinline__ void placeCols(const XT* x, const int* __restrict__ e
 #pragma unroll
     for (int k = 0; k < kColSlots; ++k)
         if (t + k * BS < ne) xl[t + k * BS] = g[k];
-    for (int c = t + kColSlots * BS; c < ne; c += BS) xl[c] = ldX<FLOW>(x, (unsigned)ext[e0 + c]);
+    // a chain's columns (residentChains): the batches after the first
+    for (int c0 = t + kColSlots * BS; c0 < ne; c0 += kColSlots * BS) {
+        unsigned id[kColSlots];
+        XT v[kColSlots];
+#pragma unroll
+        for (int k = 0; k < kColSlots; ++k) id[k] = (unsigned)ext[e0 + (c0 + k * BS < ne ? c0 + k * BS : c0)];
+#pragma unroll
+        for (int k = 0; k < kColSlots; ++k) v[k] = ldX<FLOW>(x, id[k]);
+#pragma unroll
+        for (int k = 0; k < kColSlots; ++k)
+            if (c0 + k * BS < ne) xl[c0 + k * BS] = v[k];
+    }
 }
 template <int BS, bool FLOW, typename XT>
 __device__ __forceinline__ void storeCols(XT* x, const int* __restrict__ ext, int e0, int ne,
@@ -551,7 +562,14 @@ __device__ __forceinline__ void storeCols(XT* x, const int* __restrict__ ext, in
 #pragma unroll
     for (int k = 0; k < kColSlots; ++k)
         if (t + k * BS < ne) stX<FLOW>(x, ex[k], xl[t + k * BS]);
-    for (int c = t + kColSlots * BS; c < ne; c += BS) stX<FLOW>(x, (unsigned)ext[e0 + c], xl[c]);
+    for (int c0 = t + kColSlots * BS; c0 < ne; c0 += kColSlots * BS) {
+        unsigned id[kColSlots];
+#pragma unroll
+        for (int k = 0; k < kColSlots; ++k) id[k] = (unsigned)ext[e0 + (c0 + k * BS < ne ? c0 + k * BS : c0)];
+#pragma unroll
+        for (int k = 0; k < kColSlots; ++k)
+            if (c0 + k * BS < ne) stX<FLOW>(x, id[k], xl[c0 + k * BS]);
+    }
 }
 
 // The quotient d / rn by the row norm of which inv is the reciprocal: a
@@ -946,7 +964,9 @@ __global__ void __launch_bounds__(BS) k_gs_bundle_vl(
 }
 
 // Variable lanes per row, Kaczmarz (see kaczChain).  part: BS partial
-// sums, rl0: the first lane of every row of the bundle.
+// sums, rl0: the first lane of every row of the bundle.  A bundle without
+// columns of its own works in those of the bundle before it (residentChains);
+// they are stored before the next bundle that has columns and after the last.
 template <int BS, typename VT, typename XT, bool BATCH, bool FLOW>
 __device__ __forceinline__ void kaczChainVL(
     const int cLo, const int cHi, const int k, XT* xl, const int spare, XT* part, int* rl0,
@@ -970,6 +990,7 @@ __device__ __forceinline__ void kaczChainVL(
     unsigned ex[kColSlots];
     loadCols<BS>(ext, e0, ne, ex);
     int i = (int)laneSlot[t < nl ? lp + t : 0];  // used by active lanes only
+    bool load = true;
     for (int bnd = cLo;;) {
         const int nb = bSlot[bnd + 1] - s0;
         const long off = bOff[bnd];
@@ -990,9 +1011,9 @@ __device__ __forceinline__ void kaczChainVL(
             lv[u] = sval[e];
         }
         XT g[kColSlots];
-        gatherCols<BS, FLOW>(x, ne, ex, g);
+        if (load) gatherCols<BS, FLOW>(x, ne, ex, g);
         const XT br = b[active ? row : 0u];
-        placeCols<BS, FLOW>(x, ext, e0, ne, g, xl);
+        if (load) placeCols<BS, FLOW>(x, ext, e0, ne, g, xl);
         // behind the gathers, as in kaczChain
         setSpans(spans, active, myWave);
         if (active && (t == 0 || iPrev != i)) rl0[i] = t;
@@ -1010,7 +1031,7 @@ __device__ __forceinline__ void kaczChainVL(
             s0n = bSlot[bnd + 1];
             e0n = bExt[bnd + 1], nen = bExt[bnd + 2] - e0n;
             lpn = lanePtr[bnd + 1], nln = lanePtr[bnd + 2] - lpn;
-            loadCols<BS>(ext, e0n, nen, exn);
+            if (nen > 0) loadCols<BS>(ext, e0n, nen, exn);
             in = (int)laneSlot[t < nln ? lpn + t : 0];
         }
         runWaves(spans, nw, [&](int w, bool spread) {
@@ -1036,13 +1057,17 @@ __device__ __forceinline__ void kaczChainVL(
                 for (int u = 0; u < E; ++u) xl[lw[u]] = cur[u] - scale * valOf<XT>(lv[u]);
             }
         });
-        storeCols<BS, FLOW>(x, ext, e0, ne, ex, xl);
+        load = nen > 0;
+        if (load || !more) storeCols<BS, FLOW>(x, ext, e0, ne, ex, xl);
         __syncthreads();
         if (!more) break;
         ++bnd;
-        s0 = s0n, e0 = e0n, ne = nen, lp = lpn, nl = nln, i = in;
+        s0 = s0n, lp = lpn, nl = nln, i = in;
+        if (load) {
+            e0 = e0n, ne = nen;
 #pragma unroll
-        for (int q = 0; q < kColSlots; ++q) ex[q] = exn[q];
+            for (int q = 0; q < kColSlots; ++q) ex[q] = exn[q];
+        }
     }
 }
 
@@ -1108,12 +1133,55 @@ struct LdsPlan {
     size_t bytes;
     int spare;
 };
+// beside the local columns: with variable lanes a partial sum per lane and the
+// first lane of every row
 template <typename XT>
-LdsPlan ldsPlan(int local, int rows, int tpr, int bs) {
-    const size_t var = tpr == 0 ? (size_t)bs * sizeof(XT) + (size_t)(rows + 1) * sizeof(int) : 0;
-    const size_t need = (size_t)local * sizeof(XT) + var;
-    const int spare = need + 64 * sizeof(XT) <= kMaxLds ? 64 : 32 / (int)sizeof(XT);
+size_t ldsBeside(int rows, int tpr, int bs) {
+    return tpr == 0 ? (size_t)bs * sizeof(XT) + (size_t)(rows + 1) * sizeof(int) : 0;
+}
+template <typename XT>
+LdsPlan ldsPlan(int local, int rows, int tpr, int bs, size_t limit) {
+    const size_t need = (size_t)local * sizeof(XT) + ldsBeside<XT>(rows, tpr, bs);
+    const int spare = need + 64 * sizeof(XT) <= limit ? 64 : 32 / (int)sizeof(XT);
     return {need + spare * sizeof(XT), spare};
+}
+
+// a bundle's prologue, gathers and stores, in dependency waves (weight of a
+// bundle in the longest-path estimate of a readiness-driven sweep)
+constexpr int kBundleFixedWaves = 4;
+
+// Long Kaczmarz chains whose columns fit the LDS of a whole CU keep them there
+// from the first bundle to the last instead of gathering and storing some 5000
+// scattered columns per bundle (the graph of WaveSpans: 4.34 -> 3.65 ms a sweep;
+// a batch with eight such graphs and eight right-hand sides, both sweeps and a
+// symmetric product: 10.2 -> 7.6 ms).  Loading the next bundle's entries and row
+// data behind the current waves as well gave nothing (3.71 ms).
+// A workgroup then has its CU to itself, so only where one workgroup per CU
+// gets through all other chains in the time of the longest one.  Short chains
+// gain nothing.
+constexpr int kResidentBundles = 8;
+constexpr size_t kStaticLds = 1024;  // spans, tickets: less than this
+// most columns of a chain to keep, 0 for none; limit: LDS of a workgroup then
+template <typename XT>
+int residentCols(const BundleTable& t, int nrhs, int bs, size_t* limit, int* cols) {
+    *cols = 0;
+    long all = 0, longest = 0;
+    for (size_t c = 0; c + 1 < t.chainPtr.size(); ++c) {
+        const int b0 = t.chainPtr[c], b1 = t.chainPtr[c + 1];
+        const long cost = t.wave[b1] - t.wave[b0] + (long)kBundleFixedWaves * (b1 - b0);
+        all += cost;
+        longest = std::max(longest, cost);
+    }
+    int dev = 0, cus = 0, lds = 0, rows = 0;
+    RACE_HIP(hipGetDevice(&dev));
+    RACE_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+    RACE_HIP(hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
+    for (int r : t.phRows) rows = std::max(rows, r);
+    *limit = (size_t)std::max(0, lds) > kStaticLds ? (size_t)lds - kStaticLds : 0;
+    const size_t beside = ldsBeside<XT>(rows, t.tpr, bs) + 64 * sizeof(XT);
+    if (all * nrhs <= longest * cus && *limit > std::max(beside, kMaxLds))
+        *cols = (int)((*limit - beside) / sizeof(XT));
+    return OK;
 }
 
 template <typename VT, typename XT>
@@ -1127,9 +1195,23 @@ struct BundleDev {
     long zero = 0;  // index of the zero entry in sidx / sval
     DevBuf<XT> diag;
     DevBuf<double> rowNorm;
-    int load(BundleTable&& t) {
+    size_t maxLds = kMaxLds;
+    // LDS a workgroup of bs threads needs, at most maxLds: false if a phase
+    // needs more
+    bool fits(int bs) const {
+        for (int p = 0; p < h.numPhases(); ++p)
+            if (lds(p, bs).bytes > maxLds) return false;
+        return true;
+    }
+    int load(BundleTable&& t, int bs, int nrhs) {
         h = std::move(t);
         int e;
+        if (h.kind == RACE_K_KACZ && h.tpr == 0 && fits(bs)) {
+            size_t limit = 0;
+            int cols = 0;
+            if ((e = residentCols<XT>(h, nrhs, bs, &limit, &cols))) return e;
+            if (residentChains(h, kResidentBundles, cols)) maxLds = limit;
+        }
         if ((e = upload(slot, h.slot.data(), h.slot.size()))) return e;
         if ((e = upload(wave, h.wave.data(), h.wave.size()))) return e;
         if ((e = upload(len, h.len.data(), h.len.size()))) return e;
@@ -1179,7 +1261,7 @@ struct BundleDev {
     // LDS bytes of phase p for workgroups of bs threads: the local column
     // space, the spare places behind it and, with variable lanes, a partial
     // sum per lane and the first lane of every row
-    LdsPlan lds(int p, int bs) const { return ldsPlan<XT>(h.phLocal[p], h.phRows[p], h.tpr, bs); }
+    LdsPlan lds(int p, int bs) const { return ldsPlan<XT>(h.phLocal[p], h.phRows[p], h.tpr, bs, maxLds); }
 };
 
 // one fused or plain launch of the chains [c0, c0 + nchain) of phase p
@@ -1264,10 +1346,6 @@ constexpr int kFlowPollLimit = 1 << 22;
 // aborts it will not look for): far longer than any pause of the device
 constexpr int kAutoPollLimit = 1 << 30;
 
-// a bundle's prologue, gathers and stores, in dependency waves (weight of a
-// bundle in the longest-path estimate of a readiness-driven sweep)
-constexpr int kBundleFixedWaves = 4;
-
 // Device state of the one-launch sweep of one direction: the bundle range
 // and the dependencies of every chain, column ids with the coherent-read
 // bit, and per right-hand side a flag per chain (tickets in chain order) or
@@ -1294,6 +1372,7 @@ struct FlowDev {
     long longestPath = 0;
     int nchain = 0, grid = 0, nrhs = 1, maxLocal = 0, maxRows = 0, spare = 64;
     size_t lds = 0;
+    bool fits = false;
     // chains whose conflicts lie inside one phase (0 for a valid colouring)
     long samePhase = 0;
     // nkeys / colBase: the key space of the rows and columns (chainDeps);
@@ -1314,10 +1393,10 @@ struct FlowDev {
         }
         // one layout for every phase: the largest local column space, then
         // (variable lanes) the partial sums and the first lane of every row
-        const LdsPlan plan = ldsPlan<XT>(maxLocal, maxRows, d.h.tpr, bs);
+        const LdsPlan plan = ldsPlan<XT>(maxLocal, maxRows, d.h.tpr, bs, d.maxLds);
         lds = plan.bytes;
         spare = plan.spare;
-        if (lds > kMaxLds) return OK;  // not used (the caller checks lds)
+        if (!(fits = lds <= d.maxLds)) return OK;  // not used
         // as many workgroups per right-hand side as are resident at once,
         // all sides together (more would only find the tickets gone)
         int per = 0, dev = 0, cus = 0;
@@ -1635,12 +1714,9 @@ class BundleFn : public DeviceFn {
                                       ctx.bundleLocal, tpr, bs);
         if (!tr.ok) return fallBack();
         int e;
-        if ((e = df.load(std::move(tf)))) return e;
-        if ((e = dr.load(std::move(tr)))) return e;
-        for (int p = 0; p < df.h.numPhases(); ++p)
-            if (df.lds(p, bs).bytes > kMaxLds) return fallBack();
-        for (int p = 0; p < dr.h.numPhases(); ++p)
-            if (dr.lds(p, bs).bytes > kMaxLds) return fallBack();
+        if ((e = df.load(std::move(tf), bs, nrhs))) return e;
+        if ((e = dr.load(std::move(tr), bs, nrhs))) return e;
+        if (!df.fits(bs) || !dr.fits(bs)) return fallBack();
         const bool gsFlow = kind == RACE_K_GS && nrhs == 1 && (bs == 256 || flowWide) && tpr > 0;
         const bool kaczFlow = kind == RACE_K_KACZ && kaczFlowBs(bs);
         const int chains = std::max((int)df.h.chainPtr.size(), (int)dr.h.chainPtr.size()) - 1;
@@ -1659,7 +1735,7 @@ class BundleFn : public DeviceFn {
             // conflicts inside a phase would serialise its chains, and one
             // LDS layout serves every phase: keep the phase launches if
             // either does not hold
-            const bool ok = ff.samePhase == 0 && fr.samePhase == 0 && ff.lds <= kMaxLds && fr.lds <= kMaxLds;
+            const bool ok = ff.samePhase == 0 && fr.samePhase == 0 && ff.fits && fr.fits;
             flow = ok && !small;
             autoFlow = ok && small;
             if (small) ff.pollLimit = fr.pollLimit = kAutoPollLimit;
@@ -1822,9 +1898,8 @@ class BundleBatchFn : public DeviceFn {
                 if ((e = upload(grp->bx[dir], hx.data(), hx.size()))) return e;
                 if ((e = upload(grp->bb[dir], hb.data(), hb.size()))) return e;
                 if ((e = upload(grp->bn[dir], hn.data(), hn.size()))) return e;
-                if ((e = grp->dev[dir].load(std::move(fused)))) return e;
-                for (int p = 0; p < grp->dev[dir].h.numPhases(); ++p)
-                    if (grp->dev[dir].lds(p, bs).bytes > kMaxLds) return ERR_INCOMPATIBILITY;
+                if ((e = grp->dev[dir].load(std::move(fused), bs, nrhs))) return e;
+                if (!grp->dev[dir].fits(bs)) return ERR_INCOMPATIBILITY;
                 maxPhases[dir] = std::max(maxPhases[dir], grp->dev[dir].h.numPhases());
                 if (ctx.flow && kind == RACE_K_KACZ && kaczFlowBs(bs)) {
                     // every matrix its own range of row / column keys
@@ -1838,7 +1913,7 @@ class BundleBatchFn : public DeviceFn {
                         return e;
                     // conflicts inside a phase, or one LDS layout for all
                     // phases too large: the fused phase launches then
-                    if (grp->flow[dir].samePhase != 0 || grp->flow[dir].lds > kMaxLds) flowOk = false;
+                    if (grp->flow[dir].samePhase != 0 || !grp->flow[dir].fits) flowOk = false;
                 }
             }
             groups.push_back(std::move(grp));

@@ -14,7 +14,7 @@
 namespace race {
 
 constexpr int kBlock = 256;
-constexpr size_t kMaxLds = 64 * 1024;  // LDS bytes one workgroup may allocate
+constexpr size_t kMaxLds = 64 * 1024;  // LDS bytes of a workgroup that shares its CU
 
 template <int W>
 __device__ __forceinline__ double groupSum(double v) {

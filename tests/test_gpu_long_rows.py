@@ -85,3 +85,36 @@ def test_kaczmarz_row_of_infinite_right_hand_side():
     got = dx.download()
     assert got[10] == np.inf and np.all(np.isfinite(np.delete(got, 10)))
     assert relerr(np.delete(got, 10), 1.0 / np.delete(pval, 10)) <= TOL
+
+
+# Columns of one chain that just fit a CU's LDS beside 256 partial sums and 129
+# row starts, and one more.  FP32: a row's sum of up to 16 products a lane and
+# ten additions over lanes errs by less than 30 * 2^-24, and a column is written
+# by at most ten rows.
+@pytest.mark.parametrize("prec,n,tol", [(R.FP64, 19000, TOL), (R.FP64, 19967, TOL), (R.FP64, 19968, TOL),
+                                        (R.FP32, 40255, 2e-5), (R.FP32, 40256, 2e-5)])
+def test_chain_columns_held_in_lds(oracle, prec, n, tol):
+    """a single leaf of over a hundred bundles, one and three right-hand sides,
+    phase launches and one launch per sweep"""
+    rp, col, val = _hubs(n, [(5, 200), (77, 2500), (n - 1, 70)], 3)
+    ce = R.Interface(n, 1, R.TWO, rp, col, symm_hint=True)
+    ce.RACEColor()
+    zt = oracle.level_recursion(oracle.Graph(rp, col, symm_hint=True), 1, oracle.TWO)
+    prp, pcol, pval = M.make_diag_first(*M.permute(rp, col, val, ce.getPerm(), ce.getInvPerm()))
+    dt = np.float64 if prec == R.FP64 else np.float32
+    ce.setOption("bundle_threads", 256)
+    for nrhs in (1, 3):
+        b = M.uniform_vec(n, 4, nrhs=nrhs).astype(dt)
+        for flow in (0, 1):
+            ce.setOption("flow", flow)
+            dx, db = R.DeviceArray.from_host(np.zeros(n * nrhs, dt)), R.DeviceArray.from_host(b)
+            fid = ce.registerDevice(R.K_KACZ, prp, pcol, pval, dx, db, nrhs=nrhs, val_precision=prec,
+                                    vec_precision=prec)
+            xo = np.zeros(n * nrhs)
+            for rev in (False, True):
+                print("case chain columns", n, prec, nrhs, flow, rev, flush=True)
+                ce.executeFunction(fid, rev)
+                oracle.run_calls(oracle.K_KACZ, prp, pcol, pval, xo, b.astype(np.float64).ravel(),
+                                 oracle.leaf_calls(zt, rev), nrhs=nrhs)
+                assert relerr(dx.download().ravel(), xo) <= tol
+            assert ce.flowAborts(fid) == 0
