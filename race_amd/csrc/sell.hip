@@ -230,7 +230,7 @@ __device__ __forceinline__ void sellBlock(const CT (&c)[E], const VT (&v)[E], co
 // row's entries, as the CRS row order.  The entries of the last blocks are
 // requested first, those of each full block while the x entries of the one
 // before it arrive.
-template <int NR, bool NT, typename CT, typename VT, typename XT>
+template <int NR, bool NT, bool SHORT, typename CT, typename VT, typename XT>
 __device__ __forceinline__ void sellRow(const SellView<CT, VT>& A, int c, int lane, const XT* const (&x)[NR],
                                         XT (&t)[NR]) {
     int W = A.W;
@@ -245,7 +245,7 @@ __device__ __forceinline__ void sellRow(const SellView<CT, VT>& A, int c, int la
     const CT* __restrict__ col = A.col + s0 * kC;
     const VT* __restrict__ val = A.val + s0 * kC;
     const int* __restrict__ base = A.base + (sizeof(CT) == 2 ? s0 : 0);
-    const int full = W & ~7, at2 = full + (W & 4), at1 = at2 + (W & 2);
+    const int full = SHORT ? 0 : W & ~7, at2 = full + (W & 4), at1 = at2 + (W & 2);
     CT c4[4], c2[2], c1[1];
     VT v4[4], v2[2], v1[1];
     if (W & 4) {
@@ -287,7 +287,7 @@ __device__ __forceinline__ void sellRow(const SellView<CT, VT>& A, int c, int la
 
 // y = A x (acc: y += A x) for nrhs right-hand sides (vectors column-major,
 // v[r + k n]), NR at a time: the entries are read once for NR of them.
-template <int NR, bool NT, typename CT, typename VT, typename XT>
+template <int NR, bool NT, bool SHORT, typename CT, typename VT, typename XT>
 __global__ void __launch_bounds__(kBlock) k_sell(SellView<CT, VT> A, const XT* __restrict__ x, XT* __restrict__ y,
                                                  int nrhs, int acc, int perXcd) {
     // the chunk is uniform over its wavefront: its tables load through the scalar unit
@@ -306,7 +306,7 @@ __global__ void __launch_bounds__(kBlock) k_sell(SellView<CT, VT> A, const XT* _
             t[q] = XT(0);
             old[q] = acc && r < A.n ? y[vo + r] : XT(0);
         }
-        sellRow<NR, NT>(A, c, lane, xq, t);
+        sellRow<NR, NT, SHORT>(A, c, lane, xq, t);
         if (r < A.n)
 #pragma unroll
             for (int q = 0; q < NR; ++q)
@@ -364,6 +364,11 @@ __global__ void __launch_bounds__(kBlock) k_sell_symm_atomic(SellView<CT, double
 // mapping only unbalances a short launch (7-point 64^3 5.2 -> 6.1).
 constexpr long kL2Bytes = 32l << 20, kInfinityCacheBytes = 256l << 20;
 
+// Matrices whose chunks all have the same width below 8 (SHORT) run without the
+// loop over full blocks, whose double buffer costs 94 registers instead of 42
+// in FP64 and so 5 waves per SIMD instead of 8: 7-point 256^3 FP64 321 -> 288
+// us, 224^3 214 -> 190, 192^3 119 -> 106, 96^3 16.4 -> 13.6, 64^3 the same.
+//
 // one launch of y = A x or y += A x.  Right-hand sides are taken 1, 2, 4 or 8
 // at a time, the smallest block that covers them (8 for 5 to 8, blocks of 4
 // otherwise): a pass over the entries costs more than idle columns of a block.
@@ -373,12 +378,15 @@ void launchSellNr(const SellMatrix<VT>& A, const void* x, void* y, int nrhs, boo
     const long all = A.bytes + 2l * nrhs * A.n * (long)sizeof(XT);
     const int perXcd = A.bytes <= kInfinityCacheBytes && all > kL2Bytes ? (g + 7) / 8 : 0;
     const dim3 grid(perXcd ? 8 * perXcd : g);
-    if (A.bytes > kInfinityCacheBytes)
-        hipLaunchKernelGGL((k_sell<NR, true, CT, VT, XT>), grid, dim3(kBlock), 0, st, A.template view<CT>(),
-                           (const XT*)x, (XT*)y, nrhs, (int)acc, perXcd);
+    const bool nt = A.bytes > kInfinityCacheBytes;
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, dim3(kBlock), 0, st, A.template view<CT>(), (const XT*)x, (XT*)y, nrhs,
+                           (int)acc, perXcd);
+    };
+    if (A.uniformW >= 0 && A.uniformW < 8)
+        nt ? launch(k_sell<NR, true, true, CT, VT, XT>) : launch(k_sell<NR, false, true, CT, VT, XT>);
     else
-        hipLaunchKernelGGL((k_sell<NR, false, CT, VT, XT>), grid, dim3(kBlock), 0, st, A.template view<CT>(),
-                           (const XT*)x, (XT*)y, nrhs, (int)acc, perXcd);
+        nt ? launch(k_sell<NR, true, false, CT, VT, XT>) : launch(k_sell<NR, false, false, CT, VT, XT>);
 }
 template <typename CT, typename VT, typename XT>
 void launchSellIds(const SellMatrix<VT>& A, const void* x, void* y, int nrhs, bool acc, hipStream_t st) {
@@ -597,8 +605,8 @@ class SymmSellFn : public DeviceFn {
 // the products and their order are the same, only the launches differ.  A
 // slope-2 wavefront over the groups (power q on group L - 2 (q - 1) in launch
 // L) was measured on 7-point 192^3, k = 8, 256 MB blocking, FP64: 100 launches,
-// 1.23 ms, against 1.02 ms for 8 launches over the same SELL layout (0.95 ms
-// with packed entries); 27-point 33^3, k = 5, 4 MB, FP32: 31 launches,
+// 1.23 ms, against 1.02 ms for 8 launches over the same SELL layout (0.84 ms
+// with packed entries and the SHORT kernels); 27-point 33^3, k = 5, 4 MB, FP32: 31 launches,
 // 139.7 us, against 19.3 us.  The 256 MB Infinity Cache serves a
 // gathering SpMV little faster than HBM, so the reuse does not pay for the
 // extra launches (3-5 us each) at any size.
@@ -722,7 +730,7 @@ __global__ void __launch_bounds__(kBlock) k_sell_residual(SellView<CT, double> A
             const double* const xq[1] = {x + vo};
             double t[1] = {0.0};
             const double bv = b[vo + (live ? row : 0)];
-            sellRow<1, NT>(A, c, lane, xq, t);
+            sellRow<1, NT, false>(A, c, lane, xq, t);
             if (!live) continue;
             const double rv = bv - t[0];
             r[vo + row] = (RT)rv;
@@ -860,7 +868,7 @@ static void expandUpper(const race_kernel_desc& d, std::vector<int>& rp, std::ve
 // store more than 5 slots for 4 entries (Product's rule) or be wider than 64
 // entries: with 8 right-hand sides a chunk holding a hub row runs its up to
 // 400 steps once per right-hand side.  16 matrices of 2000 to 40000 rows, FP32,
-// 8 right-hand sides: 864 us in chunks alone, 176 us.
+// 8 right-hand sides: 864 us in chunks alone, 167 us.
 template <typename XT>
 class SellBatchFn : public DeviceFn {
   public:
