@@ -167,7 +167,7 @@ int race_register_device(race_handle h, const race_kernel_desc *desc, int *id);
  *                  2 = one launch over a SELL-C upper triangle, FP64 atomics,
  *                  3 = one launch over the expanded full matrix (default, 0)
  *   "graph"        1 = executeFunction replays the function's launch sequence
- *                  (one kernel per colour phase or wavefront step) as a HIP
+ *                  (one kernel per colour phase or matrix power) as a HIP
  *                  graph, captured once per sweep direction, vectors and
  *                  power (default 0)
  *   "bfs_block_max" ranges of at most this many rows are traversed one
@@ -315,7 +315,7 @@ int race_schedule_info(const void *buf, size_t size, int *nrow, int *dist, int *
 /* dependency waves of a registered GS/KACZ function (critical path length) */
 int race_get_wave_count(race_handle h, int id, int rev, int *waves);
 /* kernel launches one execution of a registered device function issues
- * (colour phases, MPK wavefront steps) */
+ * (colour phases, MPK powers) */
 int race_get_launch_count(race_handle h, int id, int rev, int *launches);
 /* one-launch ("flow") sweeps of a device function whose dependency waits gave
  * up after their poll budget (always 0 for a consistent schedule; a nonzero

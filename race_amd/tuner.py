@@ -10,7 +10,8 @@ the smallest predicted value.
 
 For the matrix powers (kind "mpk", k = 4) the candidates are the cache
 budgets MPK_CACHE_MB handed to RACEColor(4, budget): the MPK block depth
-(level groups per wavefront step), which sets the number of launches.
+(level groups).  The budget sets the permutation and the order of the host
+callbacks; the device runs one launch per power whatever it is.
 For RACE's own preprocessing (kind "race") the candidates are the rows per
 RACE thread RACE_ROWS_PER_THREAD of a distance-1 colouring for a symmetric
 Gauss-Seidel step: the thread count sets the recursion depth (stages,
