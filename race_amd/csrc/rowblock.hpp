@@ -99,8 +99,11 @@ struct RowBlocks {
             narrowIds &= hi - k.base <= 65535;
             hcol.insert(hcol.end(), C + k.p0, C + R[r]);
             for (int j = k.p0; j < R[r]; ++j) hval.push_back(toStorage<VT>(V[j]));
-            // the last thread's four entries: the block's smallest column, value 0
-            while (hcol.size() % 4) {
+            // the last thread's four entries: the block's smallest column,
+            // value 0.  A block of empty rows has four of its own too (column
+            // 0): its threads load them, and gather x of its own matrix, which
+            // the entries of the next block need not (batches).
+            for (int q = 0; (k.ne == 0 && q < 4) || hcol.size() % 4; ++q) {
                 hcol.push_back(k.base);
                 hval.push_back(VT(0));
             }
@@ -112,9 +115,6 @@ struct RowBlocks {
         nBlk = (int)hb.size();
         int e;
         if (!fits()) return ERR_INVALID_ARG;
-        // a block without entries still loads four from its place
-        hcol.resize(hcol.size() + 4, 0);
-        hval.resize(hval.size() + 4, VT(0));
         if (narrowIds) {
             std::vector<uint16_t> h(hcol.size(), 0);
             for (const RowBlk& k : hb)
@@ -143,6 +143,12 @@ struct RowBlocks {
         return RowBlkView<CT, VT>{blks.p, rp.p, c, val.p, vecs};
     }
 };
+
+// Where thread t of a block of ne entries reads its four in k_rowblk, and its
+// entry j in k_rowblk_packed: past the block's last the first again, which are
+// not summed.
+__host__ __device__ inline int firstOf4(int t, int ne) { return 4 * t < ne ? 4 * t : 0; }
+__host__ __device__ inline int entryAt(int j, int ne) { return j < ne ? j : 0; }
 
 // four consecutive entries, aligned to their size
 template <typename T>
@@ -174,11 +180,10 @@ __global__ void __launch_bounds__(kBlock) k_rowblk(RowBlkView<CT, VT> A, const X
     const CT* __restrict__ col = A.col + (long)k.e0 * 4;
     const VT* __restrict__ val = A.val + (long)k.e0 * 4;
     const int ne = k.ne;
-    // entries past the block's last four read its first four and are not summed
     CT c[4];
     VT v[4];
-    load4(col + (4 * t < ne ? 4 * t : 0), c);
-    load4(val + (4 * t < ne ? 4 * t : 0), v);
+    load4(col + firstOf4(t, ne), c);
+    load4(val + firstOf4(t, ne), v);
     if (ne <= kRbEntries) {
         // lanes per row: the largest power of two the rows leave room for, at
         // most a wavefront
@@ -322,13 +327,12 @@ __global__ void __launch_bounds__(kBlock) k_rowblk_packed(RowBlkView<CT, VT> A, 
         for (int u = 0; u < R; ++u) prod[at * R + u] = v[u];
     };
     if (ne <= kPackedEntries) {
-        // entries past the block's last read its first and are not summed
         constexpr int N = kPackedEntries / kBlock;
         CT c[N];
         VT v[N];
 #pragma unroll
         for (int u = 0; u < N; ++u) {
-            const int j = t + u * kBlock < ne ? t + u * kBlock : 0;
+            const int j = entryAt(t + u * kBlock, ne);
             c[u] = col[j];
             v[u] = val[j];
         }
