@@ -8,6 +8,10 @@
 //     thread may load lies in the table, names a column of the block's own
 //     matrix, and is one of the block's entries or has the value 0; every row
 //     of every matrix is in one block with its own entries.
+//   rowblock_table growth
+//     matrices added one by one: entries are moved to new memory a number of
+//     times that grows with the logarithm of their count, and one matrix alone
+//     not at all.
 // Prints "ok" and exits 0 on success.
 #include <cstdio>
 #include <cstring>
@@ -88,12 +92,32 @@ int check(int cap) {
     return bad;
 }
 
+int growth() {
+    const Crs m = matrix(20000, 7, 300, [](int) { return false; });
+    int bad = 0;
+    for (int count : {1, 16, 64, 256}) {
+        RowBlocks<float> rb;
+        int moves = 0, log2 = 0;
+        const int* at = nullptr;
+        for (int k = 0; k < count; ++k) {
+            rb.add(m.n, m.rp.data(), m.col.data(), m.val.data(), k);
+            moves += at != nullptr && at != rb.hcol.data();
+            at = rb.hcol.data();
+        }
+        while (1 << log2 < count) ++log2;
+        if (moves > log2 + 1) std::printf("%d matrices: %d moves\n", count, moves), ++bad;
+    }
+    return bad;
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
     int bad = 1;
     if (argc == 2 && !std::strcmp(argv[1], "columns"))
         bad = check<double>(kRbEntries) + check<float>(kPackedEntries) + check<uint16_t>(kRbEntries);
+    else if (argc == 2 && !std::strcmp(argv[1], "growth"))
+        bad = growth();
     if (bad == 0) std::puts("ok");
     return bad != 0;
 }

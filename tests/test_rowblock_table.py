@@ -30,3 +30,8 @@ def test_loaded_columns_lie_in_their_own_matrix(program):
     """Empty rows at the start, in the middle and at the end of a matrix of a
     batch: no thread of a block reads x past its own matrix."""
     run(program, "columns")
+
+
+def test_growing_batch_moves_its_entries_seldom(program):
+    """Adding matrix after matrix takes time in proportion to their entries."""
+    run(program, "growth")
