@@ -413,25 +413,46 @@ BundleTable concatBundles(const std::vector<const BundleTable*>& tabs, std::vect
 
 int residentChains(BundleTable& t, int minBundles, int maxCols) {
     maxCols = std::min(maxCols, 65535);  // 16-bit local columns
+    // the chains to keep, before any table is touched: most sweeps have none
+    std::vector<int> keep;               // chain
+    std::vector<std::vector<int>> kept;  // its columns, ascending
+    std::vector<int> seen;               // per column: the chain that counted it last, plus 1
+    const int nchain = (int)t.chainPtr.size() - 1;
+    for (int c = 0; c < nchain && maxCols > 0; ++c) {
+        const int b0 = t.chainPtr[c], b1 = t.chainPtr[c + 1];
+        if (b1 - b0 < minBundles || t.extPtr[b1] == t.extPtr[b0]) continue;
+        int widest = 0;
+        for (int b = b0; b < b1; ++b) widest = std::max(widest, t.extPtr[b + 1] - t.extPtr[b]);
+        if (widest > maxCols) continue;
+        if (seen.empty()) seen.assign((size_t)*std::max_element(t.ext.begin(), t.ext.end()) + 1, 0);
+        std::vector<int> cols;
+        for (int e = t.extPtr[b0]; e < t.extPtr[b1] && (int)cols.size() <= maxCols; ++e) {
+            int& s = seen[t.ext[e]];
+            if (s == c + 1) continue;
+            s = c + 1;
+            cols.push_back(t.ext[e]);
+        }
+        if ((int)cols.size() > maxCols) continue;
+        std::sort(cols.begin(), cols.end());
+        keep.push_back(c);
+        kept.push_back(std::move(cols));
+    }
+    if (keep.empty()) return 0;
     const int nb = (int)t.slot.size() - 1;
-    std::vector<int> ext, extPtr(1, 0), cols;
+    std::vector<int> ext, extPtr(1, 0);
     std::vector<uint16_t> place;
-    int made = 0;
+    size_t next = 0;
     for (int p = 0; p < t.numPhases(); ++p)
         for (int c = t.phaseChain[p]; c < t.phaseChain[p + 1]; ++c) {
             const int b0 = t.chainPtr[c], b1 = t.chainPtr[c + 1];
-            cols.assign(t.ext.begin() + t.extPtr[b0], t.ext.begin() + t.extPtr[b1]);
-            if (b1 - b0 >= minBundles) {
-                std::sort(cols.begin(), cols.end());
-                cols.erase(std::unique(cols.begin(), cols.end()), cols.end());
-            }
-            if (b1 - b0 < minBundles || cols.empty() || (int)cols.size() > maxCols) {
+            if (next == keep.size() || keep[next] != c) {
                 for (int b = b0; b < b1; ++b) {
                     ext.insert(ext.end(), t.ext.begin() + t.extPtr[b], t.ext.begin() + t.extPtr[b + 1]);
                     extPtr.push_back((int)ext.size());
                 }
                 continue;
             }
+            const std::vector<int>& cols = kept[next++];
             for (int b = b0; b < b1; ++b) {
                 // both lists ascend
                 place.clear();
@@ -446,13 +467,10 @@ int residentChains(BundleTable& t, int minBundles, int maxCols) {
                 extPtr.push_back((int)ext.size());
             }
             t.phLocal[p] = std::max(t.phLocal[p], (int)cols.size());
-            ++made;
         }
-    if (made > 0) {
-        t.ext = std::move(ext);
-        t.extPtr = std::move(extPtr);
-    }
-    return made;
+    t.ext = std::move(ext);
+    t.extPtr = std::move(extPtr);
+    return (int)keep.size();
 }
 
 }  // namespace race

@@ -1210,7 +1210,7 @@ struct BundleDev {
             size_t limit = 0;
             int cols = 0;
             if ((e = residentCols<XT>(h, nrhs, bs, &limit, &cols))) return e;
-            if (residentChains(h, kResidentBundles, cols)) maxLds = limit;
+            if (cols > 0 && residentChains(h, kResidentBundles, cols)) maxLds = limit;
         }
         if ((e = upload(slot, h.slot.data(), h.slot.size()))) return e;
         if ((e = upload(wave, h.wave.data(), h.wave.size()))) return e;
