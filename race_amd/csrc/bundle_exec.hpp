@@ -510,19 +510,37 @@ __device__ __forceinline__ void stX(XT* x, unsigned id, XT v) {
 // column per thread and round cost two dependent memory round trips per round,
 // and the bundles of a long leaf have 4000 to 6000 columns
 // (the graph of WaveSpans: 6.02 -> 5.60 ms).
-constexpr int kColSlots = 8;
-template <int BS>
-__device__ __forceinline__ void loadCols(const int* __restrict__ ext, int e0, int ne, unsigned (&ex)[kColSlots]) {
+//
+// The ids that a thread holds over the waves of a bundle cost registers, so the
+// kernels come with K of them; columns past K per thread are taken in further
+// rounds.
+//   kColSlots   where the time of a chain counts
+//   kFewSlots   no bundle has more columns than that: the same loads with 16 to
+//               24 registers less (256 threads, 8 entries a lane, FP64: 4 workgroups
+//               per CU with kColSlots, 5 with kFewSlots), for sweeps with more
+//               chains than find a place at once.  us per symmetric step, phase
+//               launches, kColSlots / kFewSlots: 7-point 96^3 FP64 8 right-hand
+//               sides 1292 / 1099, 128^3 3185 / 2625, FP32 2242 / 1504, one side 484
+//               / 385; 27-point 112^3 8 sides FP64 5707 / 5581, FP32 3972 / 3390.
+//               Larger bundles lose by it (band of 154560 rows, 1500 columns a
+//               bundle of 256 threads 2246 / 2398).
+//   kLeanSlots  batches that keep every place of the chip busy for several times
+//               the longest chain path: also without the second index array of
+//               an update, so that three workgroups of 512 threads share a CU
+//               instead of two (BundleBatchFn::leanBatch)
+constexpr int kColSlots = 8, kFewSlots = 4, kLeanSlots = 2;
+template <int BS, int K>
+__device__ __forceinline__ void loadCols(const int* __restrict__ ext, int e0, int ne, unsigned (&ex)[K]) {
     const int t = threadIdx.x;
 #pragma unroll
     for (int k = 0; k < 2; ++k) ex[k] = (unsigned)ext[t + k * BS < ne ? e0 + t + k * BS : 0];
-    if (ne > 2 * BS)
+    if (K > 2 && ne > 2 * BS)
 #pragma unroll
-        for (int k = 2; k < kColSlots; ++k) ex[k] = (unsigned)ext[t + k * BS < ne ? e0 + t + k * BS : 0];
+        for (int k = 2; k < K; ++k) ex[k] = (unsigned)ext[t + k * BS < ne ? e0 + t + k * BS : 0];
 }
 // x of the columns: to g first (issued together), then to LDS
-template <int BS, bool FLOW, typename XT>
-__device__ __forceinline__ void gatherCols(const XT* x, int ne, const unsigned (&ex)[kColSlots], XT (&g)[kColSlots]) {
+template <int BS, bool FLOW, int K, typename XT>
+__device__ __forceinline__ void gatherCols(const XT* x, int ne, const unsigned (&ex)[K], XT (&g)[K]) {
     const int t = threadIdx.x;
     auto slots = [&](auto k0, auto k1) {
 #pragma unroll
@@ -533,41 +551,46 @@ __device__ __forceinline__ void gatherCols(const XT* x, int ne, const unsigned (
                 if (t + k * BS < ne && ex[k] >> 31) g[k] = ldCoh(&x[ex[k] & 0x7fffffffu]);
     };
     slots(std::integral_constant<int, 0>{}, std::integral_constant<int, 2>{});
-    if (ne > 2 * BS) slots(std::integral_constant<int, 2>{}, std::integral_constant<int, kColSlots>{});
+    if constexpr (K > 2)
+        if (ne > 2 * BS) slots(std::integral_constant<int, 2>{}, std::integral_constant<int, K>{});
 }
-template <int BS, bool FLOW, typename XT>
-__device__ __forceinline__ void placeCols(const XT* x, const int* __restrict__ ext, int e0, int ne,
-                                          const XT (&g)[kColSlots], XT* xl) {
+// columns of a round after the first
+template <int K>
+constexpr int kRound = K < 4 ? 4 : K;
+template <int BS, bool FLOW, int K, typename XT>
+__device__ __forceinline__ void placeCols(const XT* x, const int* __restrict__ ext, int e0, int ne, const XT (&g)[K],
+                                          XT* xl) {
+    constexpr int N = kRound<K>;
     const int t = threadIdx.x;
 #pragma unroll
-    for (int k = 0; k < kColSlots; ++k)
+    for (int k = 0; k < K; ++k)
         if (t + k * BS < ne) xl[t + k * BS] = g[k];
-    // a chain's columns (residentChains): the batches after the first
-    for (int c0 = t + kColSlots * BS; c0 < ne; c0 += kColSlots * BS) {
-        unsigned id[kColSlots];
-        XT v[kColSlots];
+    for (int c0 = t + K * BS; c0 < ne; c0 += N * BS) {
+        unsigned id[N];
+        XT v[N];
 #pragma unroll
-        for (int k = 0; k < kColSlots; ++k) id[k] = (unsigned)ext[e0 + (c0 + k * BS < ne ? c0 + k * BS : c0)];
+        for (int k = 0; k < N; ++k) id[k] = (unsigned)ext[e0 + (c0 + k * BS < ne ? c0 + k * BS : c0)];
 #pragma unroll
-        for (int k = 0; k < kColSlots; ++k) v[k] = ldX<FLOW>(x, id[k]);
+        for (int k = 0; k < N; ++k) v[k] = ldX<FLOW>(x, id[k]);
 #pragma unroll
-        for (int k = 0; k < kColSlots; ++k)
+        for (int k = 0; k < N; ++k)
             if (c0 + k * BS < ne) xl[c0 + k * BS] = v[k];
     }
 }
-template <int BS, bool FLOW, typename XT>
-__device__ __forceinline__ void storeCols(XT* x, const int* __restrict__ ext, int e0, int ne,
-                                          const unsigned (&ex)[kColSlots], const XT* xl) {
+template <int BS, bool FLOW, int K, typename XT>
+__device__ __forceinline__ void storeCols(XT* x, const int* __restrict__ ext, int e0, int ne, const unsigned (&ex)[K],
+                                          const XT* xl) {
+    constexpr int N = kRound<K>;
     const int t = threadIdx.x;
 #pragma unroll
-    for (int k = 0; k < kColSlots; ++k)
+    for (int k = 0; k < K; ++k)
         if (t + k * BS < ne) stX<FLOW>(x, ex[k], xl[t + k * BS]);
-    for (int c0 = t + kColSlots * BS; c0 < ne; c0 += kColSlots * BS) {
-        unsigned id[kColSlots];
+    for (int c0 = t + K * BS; c0 < ne; c0 += N * BS) {
+        unsigned id[N];
 #pragma unroll
-        for (int k = 0; k < kColSlots; ++k) id[k] = (unsigned)ext[e0 + (c0 + k * BS < ne ? c0 + k * BS : c0)];
+        for (int k = 0; k < N; ++k) id[k] = (unsigned)ext[e0 + (c0 + k * BS < ne ? c0 + k * BS : c0)];
 #pragma unroll
-        for (int k = 0; k < kColSlots; ++k)
+        for (int k = 0; k < N; ++k)
             if (c0 + k * BS < ne) stX<FLOW>(x, id[k], xl[c0 + k * BS]);
     }
 }
@@ -591,7 +614,7 @@ __device__ __forceinline__ XT rowScale(double d, double rn, double inv) {
 // row norms stay FP64.  The next bundle's offsets, column ids and row ids are
 // requested before the current one's waves run, so that a bundle starts with
 // the gathers of x and the entries.
-template <int BS, int TPR, int E, typename VT, typename XT, bool BATCH, bool FLOW>
+template <int BS, int TPR, int E, typename VT, typename XT, bool BATCH, bool FLOW, int K>
 __device__ __forceinline__ void kaczChain(
     const int cLo, const int cHi, const int k, XT* xl, const int spare, const int* __restrict__ bSlot,
     const int* __restrict__ bWave, const long* __restrict__ bOff, const int* __restrict__ bLen,
@@ -599,6 +622,7 @@ __device__ __forceinline__ void kaczChain(
     const double* __restrict__ rowNorm, const int* __restrict__ ext, const uint16_t* __restrict__ sidx,
     const VT* __restrict__ sval, long zero, XT* x0, const XT* __restrict__ b0, int n0, XT* const* __restrict__ bX,
     const XT* const* __restrict__ bB, const int* __restrict__ bN) {
+    constexpr bool LEAN = K == kLeanSlots;
     if (cLo >= cHi) return;
     const BundleVec<BATCH, XT> vec(x0, b0, n0, bX, bB, bN, cLo);
     const size_t vo = (size_t)k * vec.n;
@@ -608,7 +632,7 @@ __device__ __forceinline__ void kaczChain(
 
     int s0 = bSlot[cLo], nb = bSlot[cLo + 1] - s0;
     int e0 = bExt[cLo], ne = bExt[cLo + 1] - e0;
-    unsigned ex[kColSlots], row = (unsigned)rowId[i < nb ? s0 + i : 0];
+    unsigned ex[K], row = (unsigned)rowId[i < nb ? s0 + i : 0];
     loadCols<BS>(ext, e0, ne, ex);
     for (int bnd = cLo;;) {
         const long off = bOff[bnd];
@@ -628,7 +652,7 @@ __device__ __forceinline__ void kaczChain(
         }
         const double rn = rowNorm[sr];
         const int myWave = (int)slotWave[sr];
-        XT g[kColSlots];
+        XT g[K];
         gatherCols<BS, FLOW>(x, ne, ex, g);
         const XT br = b[active ? row : 0u];
         placeCols<BS, FLOW>(x, ext, e0, ne, g, xl);
@@ -636,14 +660,15 @@ __device__ __forceinline__ void kaczChain(
         const double rnInv = 1.0 / rn;
         // where an entry's update goes: an entry of value 0 (a padding entry
         // may name a column another row updates) to a spare place behind the
-        // columns
-        int lw[E];
+        // columns, or, LEAN, nowhere
+        int lw[LEAN ? 1 : E];
+        if constexpr (!LEAN)
 #pragma unroll
-        for (int u = 0; u < E; ++u) lw[u] = valOf<XT>(lv[u]) != XT(0) ? li[u] : ne + (t & (spare - 1));
+            for (int u = 0; u < E; ++u) lw[u] = valOf<XT>(lv[u]) != XT(0) ? li[u] : ne + (t & (spare - 1));
         __syncthreads();
         const bool more = bnd + 1 < cHi;
         int s0n = 0, nbn = 0, e0n = 0, nen = 0;
-        unsigned exn[kColSlots] = {}, rown = 0;
+        unsigned exn[K] = {}, rown = 0;
         if (more) {
             s0n = bSlot[bnd + 1], nbn = bSlot[bnd + 2] - s0n;
             e0n = bExt[bnd + 1], nen = bExt[bnd + 2] - e0n;
@@ -668,7 +693,13 @@ __device__ __forceinline__ void kaczChain(
                 const XT dot = laneSum<TPR>(sa + sb);
                 const XT scale = rowScale<XT>((double)dot - (double)br, rn, rnInv);
 #pragma unroll
-                for (int u = 0; u < E; ++u) xl[lw[u]] = cur[u] - scale * valOf<XT>(lv[u]);
+                for (int u = 0; u < E; ++u) {
+                    const XT a = valOf<XT>(lv[u]);
+                    if constexpr (!LEAN)
+                        xl[lw[u]] = cur[u] - scale * a;
+                    else if (a != XT(0))
+                        xl[li[u]] = cur[u] - scale * a;
+                }
             }
             __syncthreads();
         }
@@ -678,11 +709,11 @@ __device__ __forceinline__ void kaczChain(
         ++bnd;
         s0 = s0n, nb = nbn, e0 = e0n, ne = nen, row = rown;
 #pragma unroll
-        for (int q = 0; q < kColSlots; ++q) ex[q] = exn[q];
+        for (int q = 0; q < K; ++q) ex[q] = exn[q];
     }
 }
 
-template <int BS, int TPR, int E, typename VT, typename XT, bool BATCH>
+template <int BS, int TPR, int E, typename VT, typename XT, bool BATCH, int K>
 __global__ void __launch_bounds__(BS) k_kacz_bundle(
     const int* __restrict__ bSlot, const int* __restrict__ bWave, const long* __restrict__ bOff,
     const int* __restrict__ bLen, const int* __restrict__ bExt, const uint16_t* __restrict__ slotWave,
@@ -699,7 +730,7 @@ __global__ void __launch_bounds__(BS) k_kacz_bundle(
     // run in order (each segment reads what the previous one wrote)
     const int cLo = chainPtr[chain0 + q], cHi = chainPtr[chain0 + q + 1];
     // right-hand sides are independent: one per grid.y
-    kaczChain<BS, TPR, E, VT, XT, BATCH, false>(cLo, cHi, (int)blockIdx.y, xl, spare, bSlot, bWave, bOff, bLen, bExt,
+    kaczChain<BS, TPR, E, VT, XT, BATCH, false, K>(cLo, cHi, (int)blockIdx.y, xl, spare, bSlot, bWave, bOff, bLen, bExt,
                                                 slotWave, rowId, rowNorm, ext, sidx, sval, zero, x0, b0, n0, bX, bB, bN);
 }
 
@@ -789,7 +820,7 @@ __device__ __forceinline__ void readyLoop(const ReadyTables& r, Body&& body) {
 
 // Kaczmarz, all phases of a sweep in one readiness-driven launch; grid.y =
 // right-hand sides.
-template <int BS, int TPR, int E, typename VT, typename XT, bool BATCH>
+template <int BS, int TPR, int E, typename VT, typename XT, bool BATCH, int K>
 __global__ void __launch_bounds__(BS) k_kacz_flow(
     const int* __restrict__ bSlot, const int* __restrict__ bWave, const long* __restrict__ bOff,
     const int* __restrict__ bLen, const int* __restrict__ bExt, const uint16_t* __restrict__ slotWave,
@@ -801,7 +832,7 @@ __global__ void __launch_bounds__(BS) k_kacz_flow(
     XT* xl = reinterpret_cast<XT*>(smem);
     const int k = (int)blockIdx.y;
     readyLoop<BS>(rt, [&](int cLo, int cHi) {
-        kaczChain<BS, TPR, E, VT, XT, BATCH, true>(cLo, cHi, k, xl, spare, bSlot, bWave, bOff, bLen, bExt, slotWave,
+        kaczChain<BS, TPR, E, VT, XT, BATCH, true, K>(cLo, cHi, k, xl, spare, bSlot, bWave, bOff, bLen, bExt, slotWave,
                                                    rowId, rowNorm, ext, sidx, sval, zero, x0, b0, n0, bX, bB, bN);
     });
 }
@@ -967,7 +998,7 @@ __global__ void __launch_bounds__(BS) k_gs_bundle_vl(
 // sums, rl0: the first lane of every row of the bundle.  A bundle without
 // columns of its own works in those of the bundle before it (residentChains);
 // they are stored before the next bundle that has columns and after the last.
-template <int BS, typename VT, typename XT, bool BATCH, bool FLOW>
+template <int BS, typename VT, typename XT, bool BATCH, bool FLOW, int K>
 __device__ __forceinline__ void kaczChainVL(
     const int cLo, const int cHi, const int k, XT* xl, const int spare, XT* part, int* rl0,
     const int* __restrict__ bSlot, const int* __restrict__ bWave, const long* __restrict__ bOff,
@@ -978,6 +1009,7 @@ __device__ __forceinline__ void kaczChainVL(
     const XT* const* __restrict__ bB, const int* __restrict__ bN) {
     constexpr int E = kVarE;
     __shared__ WaveSpans<BS / 64> spans;
+    constexpr bool LEAN = K == kLeanSlots;
     if (cLo >= cHi) return;
     const BundleVec<BATCH, XT> vec(x0, b0, n0, bX, bB, bN, cLo);
     const size_t vo = (size_t)k * vec.n;
@@ -987,7 +1019,7 @@ __device__ __forceinline__ void kaczChainVL(
 
     int s0 = bSlot[cLo], e0 = bExt[cLo], ne = bExt[cLo + 1] - e0;
     int lp = lanePtr[cLo], nl = lanePtr[cLo + 1] - lp;
-    unsigned ex[kColSlots];
+    unsigned ex[K];
     loadCols<BS>(ext, e0, ne, ex);
     int i = (int)laneSlot[t < nl ? lp + t : 0];  // used by active lanes only
     bool load = true;
@@ -1010,7 +1042,7 @@ __device__ __forceinline__ void kaczChainVL(
             li[u] = (int)sidx[e];
             lv[u] = sval[e];
         }
-        XT g[kColSlots];
+        XT g[K];
         if (load) gatherCols<BS, FLOW>(x, ne, ex, g);
         const XT br = b[active ? row : 0u];
         if (load) placeCols<BS, FLOW>(x, ext, e0, ne, g, xl);
@@ -1019,19 +1051,20 @@ __device__ __forceinline__ void kaczChainVL(
         if (active && (t == 0 || iPrev != i)) rl0[i] = t;
         if (t == 0) rl0[nb] = nl;
         const double rnInv = 1.0 / rn;
-        int lw[E];
+        int lw[LEAN ? 1 : E];
+        if constexpr (!LEAN)
 #pragma unroll
-        for (int u = 0; u < E; ++u) lw[u] = valOf<XT>(lv[u]) != XT(0) ? li[u] : ne + (t & (spare - 1));
+            for (int u = 0; u < E; ++u) lw[u] = valOf<XT>(lv[u]) != XT(0) ? li[u] : ne + (t & (spare - 1));
         __syncthreads();
         const int rowL0 = active ? rl0[i] : 0, rowL1 = active ? rl0[i + 1] : 0;
         const bool more = bnd + 1 < cHi;
         int s0n = 0, e0n = 0, nen = 0, lpn = 0, nln = 0, in = 0;
-        unsigned exn[kColSlots] = {};
+        unsigned exn[K] = {};
         if (more) {
             s0n = bSlot[bnd + 1];
             e0n = bExt[bnd + 1], nen = bExt[bnd + 2] - e0n;
             lpn = lanePtr[bnd + 1], nln = lanePtr[bnd + 2] - lpn;
-            if (nen > 0) loadCols<BS>(ext, e0n, nen, exn);
+            if (LEAN || nen > 0) loadCols<BS>(ext, e0n, nen, exn);
             in = (int)laneSlot[t < nln ? lpn + t : 0];
         }
         runWaves(spans, nw, [&](int w, bool spread) {
@@ -1054,10 +1087,16 @@ __device__ __forceinline__ void kaczChainVL(
             if (mine) {
                 const XT scale = rowScale<XT>((double)rowDot - (double)br, rn, rnInv);
 #pragma unroll
-                for (int u = 0; u < E; ++u) xl[lw[u]] = cur[u] - scale * valOf<XT>(lv[u]);
+                for (int u = 0; u < E; ++u) {
+                    const XT a = valOf<XT>(lv[u]);
+                    if constexpr (!LEAN)
+                        xl[lw[u]] = cur[u] - scale * a;
+                    else if (a != XT(0))
+                        xl[li[u]] = cur[u] - scale * a;
+                }
             }
         });
-        load = nen > 0;
+        load = LEAN || nen > 0;
         if (load || !more) storeCols<BS, FLOW>(x, ext, e0, ne, ex, xl);
         __syncthreads();
         if (!more) break;
@@ -1066,12 +1105,12 @@ __device__ __forceinline__ void kaczChainVL(
         if (load) {
             e0 = e0n, ne = nen;
 #pragma unroll
-            for (int q = 0; q < kColSlots; ++q) ex[q] = exn[q];
+            for (int q = 0; q < K; ++q) ex[q] = exn[q];
         }
     }
 }
 
-template <int BS, typename VT, typename XT, bool BATCH>
+template <int BS, typename VT, typename XT, bool BATCH, int K>
 __global__ void __launch_bounds__(BS) k_kacz_bundle_vl(
     const int* __restrict__ bSlot, const int* __restrict__ bWave, const long* __restrict__ bOff,
     const int* __restrict__ bLen, const int* __restrict__ bExt, const uint16_t* __restrict__ slotWave,
@@ -1088,14 +1127,14 @@ __global__ void __launch_bounds__(BS) k_kacz_bundle_vl(
     const int q = bundleOfBlock(nchain, xcd);
     if (q < 0) return;
     const int cLo = chainPtr[chain0 + q], cHi = chainPtr[chain0 + q + 1];
-    kaczChainVL<BS, VT, XT, BATCH, false>(cLo, cHi, (int)blockIdx.y, xl, spare, part, rl0, bSlot, bWave, bOff, bLen,
+    kaczChainVL<BS, VT, XT, BATCH, false, K>(cLo, cHi, (int)blockIdx.y, xl, spare, part, rl0, bSlot, bWave, bOff, bLen,
                                           bExt, slotWave, rowId, rowNorm, ext, sidx, sval, zero, x0, b0, n0, lanePtr,
                                           laneSlot, bX, bB, bN);
 }
 
 // Kaczmarz with variable lanes per row, all phases of a sweep in one launch.
-template <int BS, typename VT, typename XT, bool BATCH>
-__global__ void __launch_bounds__(BS) k_kacz_flow_vl(
+template <int BS, typename VT, typename XT, bool BATCH, int K>
+__global__ void __launch_bounds__(BS, K == kLeanSlots ? 4 : 1) k_kacz_flow_vl(
     const int* __restrict__ bSlot, const int* __restrict__ bWave, const long* __restrict__ bOff,
     const int* __restrict__ bLen, const int* __restrict__ bExt, const uint16_t* __restrict__ slotWave,
     const int* __restrict__ rowId, const double* __restrict__ rowNorm, const int* __restrict__ ext,
@@ -1109,7 +1148,7 @@ __global__ void __launch_bounds__(BS) k_kacz_flow_vl(
     int* rl0 = reinterpret_cast<int*>(part + BS);
     const int k = (int)blockIdx.y;
     readyLoop<BS>(rt, [&](int cLo, int cHi) {
-        kaczChainVL<BS, VT, XT, BATCH, true>(cLo, cHi, k, xl, spare, part, rl0, bSlot, bWave, bOff, bLen, bExt, slotWave,
+        kaczChainVL<BS, VT, XT, BATCH, true, K>(cLo, cHi, k, xl, spare, part, rl0, bSlot, bWave, bOff, bLen, bExt, slotWave,
                                              rowId, rowNorm, ext, sidx, sval, zero, x0, b0, n0, lanePtr, laneSlot, bX,
                                              bB, bN);
     });
@@ -1150,6 +1189,25 @@ LdsPlan ldsPlan(int local, int rows, int tpr, int bs, size_t limit) {
 // bundle in the longest-path estimate of a readiness-driven sweep)
 constexpr int kBundleFixedWaves = 4;
 
+// A sweep in dependency waves plus kBundleFixedWaves per bundle: all its
+// chains, the longest of them, and the longest of every phase added up
+struct SweepCost {
+    long all = 0, longest = 0, phases = 0;
+    explicit SweepCost(const BundleTable& t) {
+        for (int p = 0; p < t.numPhases(); ++p) {
+            long most = 0;
+            for (int c = t.phaseChain[p]; c < t.phaseChain[p + 1]; ++c) {
+                const int b0 = t.chainPtr[c], b1 = t.chainPtr[c + 1];
+                const long cost = t.wave[b1] - t.wave[b0] + (long)kBundleFixedWaves * (b1 - b0);
+                all += cost;
+                most = std::max(most, cost);
+            }
+            longest = std::max(longest, most);
+            phases += most;
+        }
+    }
+};
+
 // Long Kaczmarz chains whose columns fit the LDS of a whole CU keep them there
 // from the first bundle to the last instead of gathering and storing some 5000
 // scattered columns per bundle (the graph of WaveSpans: 4.34 -> 3.65 ms a sweep;
@@ -1165,13 +1223,7 @@ constexpr size_t kStaticLds = 1024;  // spans, tickets: less than this
 template <typename XT>
 int residentCols(const BundleTable& t, int nrhs, int bs, size_t* limit, int* cols) {
     *cols = 0;
-    long all = 0, longest = 0;
-    for (size_t c = 0; c + 1 < t.chainPtr.size(); ++c) {
-        const int b0 = t.chainPtr[c], b1 = t.chainPtr[c + 1];
-        const long cost = t.wave[b1] - t.wave[b0] + (long)kBundleFixedWaves * (b1 - b0);
-        all += cost;
-        longest = std::max(longest, cost);
-    }
+    const SweepCost sweep(t);
     int dev = 0, cus = 0, lds = 0, rows = 0;
     RACE_HIP(hipGetDevice(&dev));
     RACE_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
@@ -1179,7 +1231,7 @@ int residentCols(const BundleTable& t, int nrhs, int bs, size_t* limit, int* col
     for (int r : t.phRows) rows = std::max(rows, r);
     *limit = (size_t)std::max(0, lds) > kStaticLds ? (size_t)lds - kStaticLds : 0;
     const size_t beside = ldsBeside<XT>(rows, t.tpr, bs) + 64 * sizeof(XT);
-    if (all * nrhs <= longest * cus && *limit > std::max(beside, kMaxLds))
+    if (sweep.all * nrhs <= sweep.longest * cus && *limit > std::max(beside, kMaxLds))
         *cols = (int)((*limit - beside) / sizeof(XT));
     return OK;
 }
@@ -1196,6 +1248,7 @@ struct BundleDev {
     DevBuf<XT> diag;
     DevBuf<double> rowNorm;
     size_t maxLds = kMaxLds;
+    bool fewCols = false;  // Kaczmarz, uniform lanes: kernels with kFewSlots hold the columns of every bundle
     // LDS a workgroup of bs threads needs, at most maxLds: false if a phase
     // needs more
     bool fits(int bs) const {
@@ -1211,6 +1264,11 @@ struct BundleDev {
             int cols = 0;
             if ((e = residentCols<XT>(h, nrhs, bs, &limit, &cols))) return e;
             if (cols > 0 && residentChains(h, kResidentBundles, cols)) maxLds = limit;
+        }
+        if (h.kind == RACE_K_KACZ && h.tpr > 0) {
+            int widest = 0;
+            for (size_t b = 0; b + 1 < h.extPtr.size(); ++b) widest = std::max(widest, h.extPtr[b + 1] - h.extPtr[b]);
+            fewCols = widest <= kFewSlots * bs;
         }
         if ((e = upload(slot, h.slot.data(), h.slot.size()))) return e;
         if ((e = upload(wave, h.wave.data(), h.wave.size()))) return e;
@@ -1272,12 +1330,17 @@ void launchBundles(int kind, int nrhs, const BundleDev<VT, XT>& d, int c0, int n
     // chains of one bundle each: the kernel indexes bundles directly
     const std::vector<int>& cp = d.h.chainPtr;
     const int bundle0 = cp[c0 + nchain] - cp[c0] == nchain ? cp[c0] : -1;
-    if (kind == RACE_K_KACZ)
-        hipLaunchKernelGGL((k_kacz_bundle<BS, TPR, EE, VT, XT, BATCH>), grid, dim3(BS), d.lds(p, BS).bytes, st,
-                           d.slot.p, d.wave.p, d.off.p, d.len.p, d.extPtr.p, d.slotWave.p, d.rowId.p,
-                           d.rowNorm.p, d.ext.p, d.sidx.p, d.sval.p, d.zero, x, b, n, nrhs, d.chainPtr.p, c0, nchain, xcd,
-                           d.lds(p, BS).spare, bX, bB, bN);
-    else if (nrhs == 1 && (BS == 256 || BS == 512) && !BATCH && d.h.phExt[p] > 2 * BS)
+    if (kind == RACE_K_KACZ) {
+        auto launch = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, grid, dim3(BS), d.lds(p, BS).bytes, st, d.slot.p, d.wave.p, d.off.p, d.len.p,
+                               d.extPtr.p, d.slotWave.p, d.rowId.p, d.rowNorm.p, d.ext.p, d.sidx.p, d.sval.p, d.zero, x,
+                               b, n, nrhs, d.chainPtr.p, c0, nchain, xcd, d.lds(p, BS).spare, bX, bB, bN);
+        };
+        if (d.fewCols)
+            launch(k_kacz_bundle<BS, TPR, EE, VT, XT, BATCH, kFewSlots>);
+        else
+            launch(k_kacz_bundle<BS, TPR, EE, VT, XT, BATCH, kColSlots>);
+    } else if (nrhs == 1 && (BS == 256 || BS == 512) && !BATCH && d.h.phExt[p] > 2 * BS)
         // many outside columns: gather up to 1536 (256 threads) or 2048
         // (512 threads) of them in one batch
         hipLaunchKernelGGL((k_gs_bundle<BS, TPR, EE, VT, XT, true, BATCH, (BS == 256 ? 6 : 4)>), dim3(grid.x), dim3(BS),
@@ -1302,7 +1365,7 @@ void launchBundlesVL(int kind, int nrhs, const BundleDev<VT, XT>& d, int c0, int
                      const XT* b, int n, XT* const* bX, const XT* const* bB, const int* bN, hipStream_t st) {
     const dim3 grid(xcd ? 8u * (unsigned)((nchain + 7) / 8) : (unsigned)nchain, (unsigned)std::max(1, nrhs));
     if (kind == RACE_K_KACZ)
-        hipLaunchKernelGGL((k_kacz_bundle_vl<BS, VT, XT, BATCH>), grid, dim3(BS), d.lds(p, BS).bytes, st, d.slot.p, d.wave.p,
+        hipLaunchKernelGGL((k_kacz_bundle_vl<BS, VT, XT, BATCH, kColSlots>), grid, dim3(BS), d.lds(p, BS).bytes, st, d.slot.p, d.wave.p,
                            d.off.p, d.len.p, d.extPtr.p, d.slotWave.p, d.rowId.p, d.rowNorm.p, d.ext.p, d.sidx.p,
                            d.sval.p, d.zero, x, b, n, nrhs, d.chainPtr.p, c0, nchain, xcd, d.h.phLocal[p], d.lds(p, BS).spare,
                            d.lanePtr.p, d.laneSlot.p, bX, bB, bN);
@@ -1375,13 +1438,13 @@ struct FlowDev {
     bool fits = false;
     // chains whose conflicts lie inside one phase (0 for a valid colouring)
     long samePhase = 0;
-    // nkeys / colBase: the key space of the rows and columns (chainDeps);
-    // kern: the kernel that will run it, for its occupancy
+    int held = kColSlots;  // Kaczmarz: column ids a thread holds, which kernel
+    // nkeys / colBase: the key space of the rows and columns (chainDeps)
     // ready: readiness-driven (queue) instead of tickets in chain order
     // sets: sweeps that may overlap
     template <typename VT, typename XT>
     int init(const BundleDev<VT, XT>& d, long nkeys, const std::vector<long>* colBase, int bs, int nrhs_,
-             const void* kern, bool ready, int sets = 1) {
+             bool ready, int sets = 1) {
         readyMode = ready;
         std::vector<int> dp, dd;
         samePhase = chainDeps(d.h, nkeys, colBase, &dp, &dd);
@@ -1397,14 +1460,6 @@ struct FlowDev {
         lds = plan.bytes;
         spare = plan.spare;
         if (!(fits = lds <= d.maxLds)) return OK;  // not used
-        // as many workgroups per right-hand side as are resident at once,
-        // all sides together (more would only find the tickets gone)
-        int per = 0, dev = 0, cus = 0;
-        RACE_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kern, bs, lds));
-        RACE_HIP(hipGetDevice(&dev));
-        RACE_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-        const int slots = std::max(1, std::max(per, 1) * cus / nrhs);
-        grid = std::max(1, std::min(nchain, slots));
         // tickets in chain order (phase order); tables indexed by ticket
         // position
         std::vector<int> order(nchain);
@@ -1464,6 +1519,19 @@ struct FlowDev {
             if ((e = upload(v.arrivals, std::vector<unsigned>(cells, 0u).data(), cells))) return e;
             if ((e = upload(v.queue, std::vector<unsigned long long>(cells, 0ull).data(), cells))) return e;
         }
+        return OK;
+    }
+    // as many workgroups per right-hand side of the kernel that will run it as
+    // are resident at once, at most `most` per CU, all sides together (more would
+    // only find the tickets gone)
+    int occupy(const void* kern, int bs, int most = INT32_MAX) {
+        if (!kern) return ERR_INTERNAL;
+        int per = 0, dev = 0, cus = 0;
+        RACE_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kern, bs, lds));
+        RACE_HIP(hipGetDevice(&dev));
+        RACE_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+        const int slots = std::max(1, std::max(std::min(per, most), 1) * cus / nrhs);
+        grid = std::max(1, std::min(nchain, slots));
         return OK;
     }
     ReadyTables tables(int set) const {
@@ -1526,14 +1594,34 @@ template <int BS, int TPR, int EE, typename VT, typename XT, bool BATCH>
 int launchKaczFlow(const BundleDev<VT, XT>& d, FlowDev& f, int set, XT* x, const XT* b, int n, XT* const* bX,
                    const XT* const* bB, const int* bN, hipStream_t st) {
     if constexpr (TPR == 0) {
-        hipLaunchKernelGGL((k_kacz_flow_vl<BS, VT, XT, BATCH>), dim3(f.grid, f.nrhs), dim3(BS), f.lds, st, d.slot.p,
-                           d.wave.p, d.off.p, d.len.p, d.extPtr.p, d.slotWave.p, d.rowId.p, d.rowNorm.p, f.ext.p,
-                           d.sidx.p, d.sval.p, d.zero, x, b, n, f.maxLocal, f.spare, d.lanePtr.p, d.laneSlot.p, bX, bB, bN,
-                           f.tables(set));
+        auto launch = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3(f.grid, f.nrhs), dim3(BS), f.lds, st, d.slot.p, d.wave.p, d.off.p, d.len.p,
+                               d.extPtr.p, d.slotWave.p, d.rowId.p, d.rowNorm.p, f.ext.p, d.sidx.p, d.sval.p, d.zero, x,
+                               b, n, f.maxLocal, f.spare, d.lanePtr.p, d.laneSlot.p, bX, bB, bN, f.tables(set));
+        };
+        if constexpr (BATCH)
+            if (f.held == kLeanSlots) {
+                launch(k_kacz_flow_vl<BS, VT, XT, BATCH, kLeanSlots>);
+                RACE_HIP(hipGetLastError());
+                return OK;
+            }
+        launch(k_kacz_flow_vl<BS, VT, XT, BATCH, kColSlots>);
     } else {
-        hipLaunchKernelGGL((k_kacz_flow<BS, TPR, EE, VT, XT, BATCH>), dim3(f.grid, f.nrhs), dim3(BS), f.lds, st,
-                           d.slot.p, d.wave.p, d.off.p, d.len.p, d.extPtr.p, d.slotWave.p, d.rowId.p, d.rowNorm.p,
-                           f.ext.p, d.sidx.p, d.sval.p, d.zero, x, b, n, f.spare, bX, bB, bN, f.tables(set));
+        auto launch = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3(f.grid, f.nrhs), dim3(BS), f.lds, st, d.slot.p, d.wave.p, d.off.p, d.len.p,
+                               d.extPtr.p, d.slotWave.p, d.rowId.p, d.rowNorm.p, f.ext.p, d.sidx.p, d.sval.p, d.zero, x,
+                               b, n, f.spare, bX, bB, bN, f.tables(set));
+        };
+        if constexpr (BATCH)
+            if (f.held == kLeanSlots) {
+                launch(k_kacz_flow<BS, TPR, EE, VT, XT, BATCH, kLeanSlots>);
+                RACE_HIP(hipGetLastError());
+                return OK;
+            }
+        if (f.held == kFewSlots)
+            launch(k_kacz_flow<BS, TPR, EE, VT, XT, BATCH, kFewSlots>);
+        else
+            launch(k_kacz_flow<BS, TPR, EE, VT, XT, BATCH, kColSlots>);
     }
     RACE_HIP(hipGetLastError());
     return OK;
@@ -1582,27 +1670,36 @@ const void* gsFlowKernel(int bs, int tpr, int E) {
         default: return nullptr;
     }
 }
-template <int BS, typename VT, typename XT, bool BATCH>
-const void* kaczFlowKernelBs(int tpr, int E) {
+template <int BS, int K, typename VT, typename XT, bool BATCH>
+const void* kaczFlowKernelOf(int tpr, int E) {
     switch (tpr * 100 + E) {
-        case 104: return reinterpret_cast<const void*>(k_kacz_flow<BS, 1, 4, VT, XT, BATCH>);
-        case 108: return reinterpret_cast<const void*>(k_kacz_flow<BS, 1, 8, VT, XT, BATCH>);
-        case 116: return reinterpret_cast<const void*>(k_kacz_flow<BS, 1, 16, VT, XT, BATCH>);
-        case 208: return reinterpret_cast<const void*>(k_kacz_flow<BS, 2, 8, VT, XT, BATCH>);
-        case 213: return reinterpret_cast<const void*>(k_kacz_flow<BS, 2, 13, VT, XT, BATCH>);
-        case 216: return reinterpret_cast<const void*>(k_kacz_flow<BS, 2, 16, VT, XT, BATCH>);
-        case 408: return reinterpret_cast<const void*>(k_kacz_flow<BS, 4, 8, VT, XT, BATCH>);
-        case 416: return reinterpret_cast<const void*>(k_kacz_flow<BS, 4, 16, VT, XT, BATCH>);
-        case 16: return reinterpret_cast<const void*>(k_kacz_flow_vl<BS, VT, XT, BATCH>);
-        default: return nullptr;
+        case 104: return reinterpret_cast<const void*>(k_kacz_flow<BS, 1, 4, VT, XT, BATCH, K>);
+        case 108: return reinterpret_cast<const void*>(k_kacz_flow<BS, 1, 8, VT, XT, BATCH, K>);
+        case 116: return reinterpret_cast<const void*>(k_kacz_flow<BS, 1, 16, VT, XT, BATCH, K>);
+        case 208: return reinterpret_cast<const void*>(k_kacz_flow<BS, 2, 8, VT, XT, BATCH, K>);
+        case 213: return reinterpret_cast<const void*>(k_kacz_flow<BS, 2, 13, VT, XT, BATCH, K>);
+        case 216: return reinterpret_cast<const void*>(k_kacz_flow<BS, 2, 16, VT, XT, BATCH, K>);
+        case 408: return reinterpret_cast<const void*>(k_kacz_flow<BS, 4, 8, VT, XT, BATCH, K>);
+        case 416: return reinterpret_cast<const void*>(k_kacz_flow<BS, 4, 16, VT, XT, BATCH, K>);
     }
+    if constexpr (K != kFewSlots)
+        if (tpr == 0) return reinterpret_cast<const void*>(k_kacz_flow_vl<BS, VT, XT, BATCH, K>);
+    return nullptr;
 }
+template <int BS, typename VT, typename XT, bool BATCH>
+const void* kaczFlowKernelBs(int held, int tpr, int E) {
+    if constexpr (BATCH)
+        if (held == kLeanSlots) return kaczFlowKernelOf<BS, kLeanSlots, VT, XT, BATCH>(tpr, E);
+    return held == kFewSlots ? kaczFlowKernelOf<BS, kFewSlots, VT, XT, BATCH>(tpr, E)
+                             : kaczFlowKernelOf<BS, kColSlots, VT, XT, BATCH>(tpr, E);
+}
+// held: column ids a thread holds (kLeanSlots: batches only)
 template <typename VT, typename XT, bool BATCH>
-const void* kaczFlowKernel(int bs, int tpr, int E) {
+const void* kaczFlowKernel(int held, int bs, int tpr, int E) {
     switch (bs) {
-        case 256: return kaczFlowKernelBs<256, VT, XT, BATCH>(tpr, E);
-        case 512: return kaczFlowKernelBs<512, VT, XT, BATCH>(tpr, E);
-        case 1024: return kaczFlowKernelBs<1024, VT, XT, BATCH>(tpr, E);
+        case 256: return kaczFlowKernelBs<256, VT, XT, BATCH>(held, tpr, E);
+        case 512: return kaczFlowKernelBs<512, VT, XT, BATCH>(held, tpr, E);
+        case 1024: return kaczFlowKernelBs<1024, VT, XT, BATCH>(held, tpr, E);
         default: return nullptr;
     }
 }
@@ -1675,6 +1772,22 @@ class BundleFn : public DeviceFn {
         if (kind != RACE_K_GS || nrhs != 1) return false;
         return n <= 256 * 64 || (sizeof(XT) == 4 && n > 128 * autoChains(kind));
     }
+    // Kaczmarz in one launch: kFewSlots where more chains could run at once than
+    // 1536 threads per CU hold, on a grid of as many.  Below, more workgroups than
+    // kColSlots leaves room for only wait for chains (7-point 64^3 FP64, one side:
+    // 166 chains at once 217 us, with kFewSlots 242).  Eight sides, kColSlots /
+    // kFewSlots: 7-point 64^3 FP32 (1325 at once) 377 / 389, 27-point 80^3 FP32
+    // (2001) 1150 / 970, FP64 1643 / 1619, 7-point 96^3 FP64 (3197) 1309 / 1138.
+    int occupyKacz(FlowDev& f, const Dev& d) const {
+        constexpr int kThreads = 1536;
+        int dev = 0, cus = 0;
+        RACE_HIP(hipGetDevice(&dev));
+        RACE_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+        const SweepCost sweep(d.h);
+        const bool few = d.fewCols && sweep.all * nrhs * bs > sweep.phases * cus * kThreads;
+        f.held = few ? kFewSlots : kColSlots;
+        return f.occupy(kaczFlowKernel<VT, XT, false>(f.held, bs, tpr, E), bs, few ? kThreads / bs : INT32_MAX);
+    }
     static bool autoFits(const BundleTable& t) {
         int longest = 0;
         for (size_t c = 0; c + 1 < t.chainPtr.size(); ++c) longest = std::max(longest, t.chainPtr[c + 1] - t.chainPtr[c]);
@@ -1725,12 +1838,12 @@ class BundleFn : public DeviceFn {
         if ((ctx.flow > 0 || small) && (gsFlow || kaczFlow)) {
             const int sets = small ? kSets : 1;
             const int sides = kind == RACE_K_KACZ ? nrhs : 1;
-            const void* kern =
-                kind == RACE_K_KACZ ? kaczFlowKernel<VT, XT, false>(bs, tpr, E) : gsFlowKernel<VT, XT>(bs, tpr, E);
-            if (!kern) return ERR_INTERNAL;
             const bool ready = kind == RACE_K_KACZ;
-            if ((e = ff.init(df, n, nullptr, bs, sides, kern, ready, sets)) ||
-                (e = fr.init(dr, n, nullptr, bs, sides, kern, ready, sets)))
+            if ((e = ff.init(df, n, nullptr, bs, sides, ready, sets)) ||
+                (e = fr.init(dr, n, nullptr, bs, sides, ready, sets)))
+                return e;
+            if ((e = ready ? occupyKacz(ff, df) : ff.occupy(gsFlowKernel<VT, XT>(bs, tpr, E), bs)) ||
+                (e = ready ? occupyKacz(fr, dr) : fr.occupy(gsFlowKernel<VT, XT>(bs, tpr, E), bs)))
                 return e;
             // conflicts inside a phase would serialise its chains, and one
             // LDS layout serves every phase: keep the phase launches if
@@ -1907,10 +2020,7 @@ class BundleBatchFn : public DeviceFn {
                     for (size_t q = 0; q < members.size(); ++q) base[q + 1] = base[q] + items[members[q]].d.nrow;
                     std::vector<long> colBase(owner.size());
                     for (size_t k = 0; k < owner.size(); ++k) colBase[k] = base[owner[k]];
-                    const void* kern = kaczFlowKernel<VT, XT, true>(bs, grp->tpr, grp->E);
-                    if (!kern) return ERR_INTERNAL;
-                    if ((e = grp->flow[dir].init(grp->dev[dir], base.back(), &colBase, bs, nrhs, kern, true)))
-                        return e;
+                    if ((e = grp->flow[dir].init(grp->dev[dir], base.back(), &colBase, bs, nrhs, true))) return e;
                     // conflicts inside a phase, or one LDS layout for all
                     // phases too large: the fused phase launches then
                     if (grp->flow[dir].samePhase != 0 || !grp->flow[dir].fits) flowOk = false;
@@ -1919,6 +2029,17 @@ class BundleBatchFn : public DeviceFn {
             groups.push_back(std::move(grp));
         }
         flow = flowOk && ctx.flow && kind == RACE_K_KACZ && kaczFlowBs(bs);
+        for (int dir = 0; dir < 2 && flow; ++dir) {
+            int e;
+            bool lean = false;
+            if ((e = leanBatch(dir, &lean))) return e;
+            for (const auto& g : groups) {
+                FlowDev& f = g->flow[dir];
+                f.held = lean ? kLeanSlots : kColSlots;
+                const int most = lean && g->tpr == 0 && groups.size() > 1 ? 1 : INT32_MAX;
+                if ((e = f.occupy(kaczFlowKernel<VT, XT, true>(f.held, bs, g->tpr, g->E), bs, most))) return e;
+            }
+        }
         for (int dir = 0; dir < 2; ++dir) {
             launchOrder[dir].resize(groups.size());
             for (size_t g = 0; g < groups.size(); ++g) launchOrder[dir][g] = (int)g;
@@ -1944,6 +2065,38 @@ class BundleBatchFn : public DeviceFn {
                     if (p < g->dev[dir].h.numPhases()) w = std::max(w, g->dev[dir].h.phWaves[p]);
                 critical[dir] += w;
             }
+        return OK;
+    }
+    // One-launch sweeps: kLeanSlots where the work of all matrices keeps the
+    // places of the chip (the workgroups per CU that the group with the most work
+    // has with kColSlots) busy for more than three times the longest dependency
+    // path.  Chains are slower then, but three workgroups of 512 threads share a
+    // CU.  ms per forward / backward sweep of eight right-hand sides, half banded
+    // matrices and half Chung-Lu graphs of 2000 to 200000 rows, 512 threads x 256
+    // rows x 4 lanes, kColSlots / kLeanSlots: FP32 384 matrices (ratio 2.7) 49.1 49.2
+    // / 54.3 50.4, 512 (3.5) 68.7 66.1 / 66.6 62.8, the banded ones of them (18.8)
+    // 48.5 48.4 / 42.2 42.1; FP64 128 (2.0) 37.5 38.4 / 38.8 39.3, 256 (3.9) 62.9 65.5
+    // / 52.3 52.4.  Groups run at once, and the longest path's, mostly that of the
+    // graphs (variable lanes), starts first: it gets one workgroup per CU, as more
+    // leave the other groups no place until it ends (the 512 and 256 matrices 78.3
+    // 80.3 and 60.1 67.0).
+    static constexpr int kLeanRatio = 3;
+    int leanBatch(int dir, bool* lean) const {
+        int dev = 0, cus = 0, per = 0;
+        RACE_HIP(hipGetDevice(&dev));
+        RACE_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+        long all = 0, most = -1, path = 1;
+        for (const auto& g : groups) {
+            if (g->dev[dir].maxLds != kMaxLds) return OK;  // lean kernels know no chains kept in LDS
+            const long cost = SweepCost(g->dev[dir].h).all;
+            all += cost;
+            path = std::max(path, g->flow[dir].longestPath);
+            if (cost <= most) continue;
+            most = cost;
+            RACE_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(
+                &per, kaczFlowKernel<VT, XT, true>(kColSlots, bs, g->tpr, g->E), bs, g->flow[dir].lds));
+        }
+        *lean = (double)all * nrhs > (double)kLeanRatio * path * cus * std::max(per, 1);
         return OK;
     }
     int waves(bool rev) const override { return (int)critical[rev ? 1 : 0]; }
