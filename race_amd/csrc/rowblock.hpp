@@ -1,8 +1,11 @@
 // rowblock.hpp -- products over blocks of whole rows with up to 1024 entries.
 //
 // A workgroup loads its block's entries in CRS order, four per thread,
-// gathers x, leaves the products in LDS and sums each row with as many lanes
-// as the block's row count leaves (a power of two).  Rows of more than
+// gathers x, leaves values and x in LDS and sums each row with as many lanes as
+// the block's row count leaves (a power of two).  Values and x, not their
+// products: a row summed by one lane is then the same chain of fused multiply-
+// adds as in a SELL chunk, with one rounding per entry.  With products rounded
+// before the sum, rows of 5 to 7 entries had up to 18 % more error.  Rows of more than
 // kLaneEntries entries a lane are summed by a whole wavefront afterwards, so
 // that no lane walks a hub row alone (a graph of 200000 rows and 1.2M entries,
 // hubs of 400 entries: 19.6 us without this, 11.3 us with it).  No entry is
@@ -170,7 +173,8 @@ __device__ __forceinline__ void load4(const T* __restrict__ p, T (&out)[4]) {
 template <int NR, bool BATCH, typename CT, typename VT, typename XT>
 __global__ void __launch_bounds__(kBlock) k_rowblk(RowBlkView<CT, VT> A, const XT* __restrict__ x0,
                                                    XT* __restrict__ y0, long n0, int nrhs, int acc) {
-    __shared__ __align__(16) XT prod[NR][kRbEntries];
+    __shared__ __align__(16) XT gx[NR][kRbEntries];
+    __shared__ __align__(16) VT gv[kRbEntries];
     __shared__ int nHub, hub[kRbEntries / kLaneEntries];
     const int t = threadIdx.x;
     const RowBlk k = A.blks[blockIdx.x];
@@ -200,6 +204,8 @@ __global__ void __launch_bounds__(kBlock) k_rowblk(RowBlkView<CT, VT> A, const X
         const bool isHub = hi - lo > kLaneEntries << lg;
         const bool hubs = k.longest > kLaneEntries << lg;
         if (hubs && t == 0) nHub = 0;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) gv[4 * t + u] = v[u];
         for (int q0 = 0; q0 < nrhs; q0 += NR) {
             XT old[NR];
 #pragma unroll
@@ -211,19 +217,23 @@ __global__ void __launch_bounds__(kBlock) k_rowblk(RowBlkView<CT, VT> A, const X
                 for (int u = 0; u < 4; ++u) g[u] = xq[(unsigned)k.base + (unsigned)c[u]];
                 old[q] = acc && live && l == 0 ? y[vo + k.row0 + r] : XT(0);
 #pragma unroll
-                for (int u = 0; u < 4; ++u) prod[q][4 * t + u] = fromStorage<XT>(v[u]) * g[u];
+                for (int u = 0; u < 4; ++u) gx[q][4 * t + u] = g[u];
             }
             __syncthreads();
             // the hubs' rows, once; each takes more than kLaneEntries of the
             // block's entries, so the list holds them all
             if (q0 == 0 && isHub && l == 0) hub[atomicAdd(&nHub, 1)] = r;
+            XT s[NR] = {};
+            if (!isHub)
+                for (int i = lo + l; i < hi; i += 1 << lg) {
+                    const XT a = fromStorage<XT>(gv[i]);
+#pragma unroll
+                    for (int q = 0; q < NR; ++q) s[q] += a * gx[q][i];
+                }
 #pragma unroll
             for (int q = 0; q < NR; ++q) {
-                XT s = XT(0);
-                if (!isHub)
-                    for (int i = lo + l; i < hi; i += 1 << lg) s += prod[q][i];
-                for (int o = (1 << lg) / 2; o > 0; o >>= 1) s += __shfl_xor(s, o);
-                if (live && !isHub && l == 0 && q0 + q < nrhs) y[(long)(q0 + q) * n + k.row0 + r] = old[q] + s;
+                for (int o = (1 << lg) / 2; o > 0; o >>= 1) s[q] += __shfl_xor(s[q], o);
+                if (live && !isHub && l == 0 && q0 + q < nrhs) y[(long)(q0 + q) * n + k.row0 + r] = old[q] + s[q];
             }
             if (hubs || q0 + NR < nrhs) __syncthreads();
             if (hubs) {
@@ -232,7 +242,7 @@ __global__ void __launch_bounds__(kBlock) k_rowblk(RowBlkView<CT, VT> A, const X
 #pragma unroll
                     for (int q = 0; q < NR; ++q) {
                         XT s = XT(0);
-                        for (int i = h0 + (t & 63); i < h1; i += 64) s += prod[q][i];
+                        for (int i = h0 + (t & 63); i < h1; i += 64) s += fromStorage<XT>(gv[i]) * gx[q][i];
                         for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
                         if ((t & 63) == 0 && q0 + q < nrhs) {
                             const long at = (long)(q0 + q) * n + k.row0 + hr;
@@ -257,10 +267,10 @@ __global__ void __launch_bounds__(kBlock) k_rowblk(RowBlkView<CT, VT> A, const X
                     if (j + u < ne) s += fromStorage<XT>(vv[u]) * xq[(unsigned)k.base + (unsigned)cc[u]];
             }
             for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
-            if ((t & 63) == 0) prod[0][t >> 6] = s;
+            if ((t & 63) == 0) gx[0][t >> 6] = s;
             __syncthreads();
             if (t == 0) {
-                for (int w = 1; w < kBlock / 64; ++w) s += prod[0][w];
+                for (int w = 1; w < kBlock / 64; ++w) s += gx[0][w];
                 const long at = (long)q * n + k.row0;
                 y[at] = acc ? y[at] + s : s;
             }
@@ -268,6 +278,9 @@ __global__ void __launch_bounds__(kBlock) k_rowblk(RowBlkView<CT, VT> A, const X
         }
     }
 }
+
+__device__ __forceinline__ float fmaOf(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ __forceinline__ double fmaOf(double a, double b, double c) { return __builtin_fma(a, b, c); }
 
 // The R values of one row of packed right-hand sides (k_pack_rhs).
 template <int R, typename XT>
@@ -311,15 +324,15 @@ __global__ void __launch_bounds__(kBlock) k_pack_rhs(const XT* __restrict__ x, X
 }
 
 // k_rowblk over packed right-hand sides, R per blockIdx.y.  Entries go to the
-// threads one by one (t, t + 256, ...), so that the products of neighbouring
-// lanes are neighbours in LDS.  Blocks of kPackedEntries leave 16 KB of products
-// (ten workgroups per CU).
+// threads one by one (t, t + 256, ...), so that the rows of x of neighbouring
+// lanes are neighbours in LDS.  Blocks of kPackedEntries take 20 KB of LDS at most.
 constexpr int kPackedEntries = 2 * kBlock;
-constexpr int kPackedLaneEntries = 64;  // with fewer lanes per row than k_rowblk, and four products in flight
+constexpr int kPackedLaneEntries = 64;  // with fewer lanes per row than k_rowblk, and up to eight entries in flight
 template <int R, typename CT, typename VT, typename XT>
 __global__ void __launch_bounds__(kBlock) k_rowblk_packed(RowBlkView<CT, VT> A, const XT* __restrict__ packed,
                                                           XT* __restrict__ y, long n, int nrhs, int acc) {
-    __shared__ __align__(16) XT prod[kPackedEntries * R];
+    __shared__ __align__(16) XT gx[kPackedEntries * R];
+    __shared__ __align__(16) VT gv[kPackedEntries];
     __shared__ int nHub, hub[kPackedEntries / kPackedLaneEntries];
     const int t = threadIdx.x;
     const RowBlk k = A.blks[blockIdx.x];
@@ -330,7 +343,7 @@ __global__ void __launch_bounds__(kBlock) k_rowblk_packed(RowBlkView<CT, VT> A, 
     const int ne = k.ne;
     auto put = [&](int at, const XT (&v)[R]) {
 #pragma unroll
-        for (int u = 0; u < R; ++u) prod[at * R + u] = v[u];
+        for (int u = 0; u < R; ++u) gx[at * R + u] = v[u];
     };
     if (ne <= kPackedEntries) {
         constexpr int N = kPackedEntries / kBlock;
@@ -347,8 +360,7 @@ __global__ void __launch_bounds__(kBlock) k_rowblk_packed(RowBlkView<CT, VT> A, 
         for (int u = 0; u < N; ++u) loadRow<R>(x + (long)(unsigned)c[u] * R, g[u]);
 #pragma unroll
         for (int u = 0; u < N; ++u) {
-#pragma unroll
-            for (int p = 0; p < R; ++p) g[u][p] *= fromStorage<XT>(v[u]);
+            gv[t + u * kBlock] = v[u];
             put(t + u * kBlock, g[u]);
         }
         if (t == 0) nHub = 0;
@@ -367,16 +379,40 @@ __global__ void __launch_bounds__(kBlock) k_rowblk_packed(RowBlkView<CT, VT> A, 
             const long at = (long)(q0 + q) * n + k.row0 + r;
             const bool store = live && !isHub && l == 0 && q0 + q < nrhs;
             const XT old = acc && store ? y[at] : XT(0);
-            // four products in flight
+            // Rows of less than 8 entries a lane are one chain of fused
+            // multiply-adds, longer ones sums of pairs, which err less (rows of
+            // 17 entries on average in FP32: 1.2e-7 as one chain, 7.8e-8 so).
             XT s = XT(0);
-            const int step = R << lg;
-            int i = (lo + l) * R + q;
-            const int end = isHub ? 0 : hi * R;
-            for (; i + 3 * step < end; i += 4 * step) {
-                const XT a = prod[i], b = prod[i + step], c2 = prod[i + 2 * step], d = prod[i + 3 * step];
-                s += (a + b) + (c2 + d);
+            const int step = 1 << lg, end = isHub ? 0 : hi;
+            int i = lo + l;
+            auto pairs = [&](const XT* a, const XT* c4) {
+                return fmaOf(a[1], c4[1], a[0] * c4[0]) + fmaOf(a[3], c4[3], a[2] * c4[2]);
+            };
+            auto load = [&](auto& a, auto& c4) {
+                constexpr int N = sizeof(a) / sizeof(XT);
+#pragma unroll
+                for (int u = 0; u < N; ++u) {
+                    a[u] = fromStorage<XT>(gv[i + u * step]);
+                    c4[u] = gx[(i + u * step) * R + q];
+                }
+                i += N * step;
+            };
+            const bool deep = i + 7 * step < end;
+            while (i + 7 * step < end) {
+                XT a[8], c4[8];
+                load(a, c4);
+                s += pairs(a, c4) + pairs(a + 4, c4 + 4);
             }
-            for (; i < end; i += step) s += prod[i];
+            if (i + 3 * step < end) {
+                XT a[4], c4[4];
+                load(a, c4);
+                if (deep)
+                    s += pairs(a, c4);
+                else
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) s = fmaOf(a[u], c4[u], s);
+            }
+            for (; i < end; i += step) s = fmaOf(fromStorage<XT>(gv[i]), gx[i * R + q], s);
             for (int o = (1 << lg) / 2; o > 0; o >>= 1) s += __shfl_xor(s, o * R);
             if (store) y[at] = old + s;
         }
@@ -385,7 +421,7 @@ __global__ void __launch_bounds__(kBlock) k_rowblk_packed(RowBlkView<CT, VT> A, 
         for (int h = t >> 6; h < nHub; h += kBlock / 64) {
             const int hr = hub[h], h0 = A.rp[k.rp0 + hr] - k.p0, h1 = A.rp[k.rp0 + hr + 1] - k.p0;
             XT s = XT(0);
-            for (int i = h0 * R + (t & 63); i < h1 * R; i += 64) s += prod[i];
+            for (int i = h0 + (t & 63) / R; i < h1; i += W) s += fromStorage<XT>(gv[i]) * gx[i * R + q];
             for (int o = W / 2; o > 0; o >>= 1) s += __shfl_xor(s, o * R);
             if ((t & 63) < R && q0 + q < nrhs) {
                 const long at = (long)(q0 + q) * n + k.row0 + hr;
@@ -404,12 +440,12 @@ __global__ void __launch_bounds__(kBlock) k_rowblk_packed(RowBlkView<CT, VT> A, 
         put(t, s);
         __syncthreads();
         for (int o = kBlock / 2; o > 0; o >>= 1) {
-            for (int i = t; i < o * R; i += kBlock) prod[i] += prod[i + o * R];
+            for (int i = t; i < o * R; i += kBlock) gx[i] += gx[i + o * R];
             __syncthreads();
         }
         if (t < R && q0 + t < nrhs) {
             const long at = (long)(q0 + t) * n + k.row0;
-            y[at] = acc ? y[at] + prod[t] : prod[t];
+            y[at] = acc ? y[at] + gx[t] : gx[t];
         }
     }
 }
