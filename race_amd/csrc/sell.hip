@@ -407,13 +407,19 @@ void launchSell(const SellMatrix<VT>& A, const void* x, void* y, int nrhs, bool 
         launchSellIds<int, VT, XT>(A, x, y, nrhs, acc, st);
 }
 
-// A matrix that is multiplied with vectors, in the layout its rows ask for:
-// row blocks where the chunks would store more than 5 slots for 4 entries,
-// otherwise SELL chunks.  Both measured on both sides of the line (us, SELL
-// chunks / row blocks, FP64): Chung-Lu graphs (2 to 5 slots an entry) of 150000
-// rows 111 / 22.8, 20000 rows 41.4 / 8.1; random banded (1.25 to 1.35) of 90001
-// rows, 21 entries a row 7.4 / 6.5, of 200000 rows, 40 entries 25.9 / 26.2;
-// 27-point grids (1.0 to 1.1) 64^3 13.6 / 18.7, 96^3 37.5 / 49.6.
+// Whether rows whose chunks store `slots` slots for nnz entries go to row blocks:
+// more than 11 slots for 8 entries with one right-hand side, more than 5 for 4
+// with several, which the row blocks read in fewer passes.  Both sides measured
+// (us, SELL chunks / row blocks, FP64, FP32): rows of 12 +- 4 entries (1.33 slots an
+// entry) 9.0 10.5, 6.3 7.1, +- 6 (1.50) 11.7 10.6, 7.2 7.1; random bands of 200000
+// rows, 40 entries a row (1.27) 25.3 25.5, 17.7 19.4, of 90001 rows, 21 entries
+// (1.39) 6.9 6.3, 5.4 5.2; three sides: the band of 1.27 64.9 51.8, 46.8 37.9, rows of
+// 1.33 30.6 25.7, 20.1 19.0; 27-point grids (1.0 to 1.1) one side 64^3 13.1 18.8,
+// three 23.2 37.1; Chung-Lu graphs (2 to 5) of 150000 rows 103 19, 20000 rows 35.5 5.5.
+inline bool raggedSlots(long slots, long nnz, int nrhs) { return nrhs > 1 ? slots * 4 > nnz * 5 : slots * 8 > nnz * 11; }
+
+// A matrix that is multiplied with vectors, in the layout its rows ask for: SELL
+// chunks or row blocks (raggedSlots).
 template <typename VT, typename XT>
 struct Product {
     SellMatrix<VT> sell;
@@ -426,12 +432,13 @@ struct Product {
     // for all of them instead of one each, and one or two trips through the
     // address unit instead of nrhs.  It pays where columns are scattered over
     // x, so that every gather is a line of its own; where lines are shared
-    // (kScattered) only with many entries.  us, separate columns / packed:
-    // Chung-Lu graph 150000 rows, 3.0M entries FP32 2 / 3 / 8 sides 37 / 23, 71 / 27,
-    // 162 / 40, FP64 8 sides 224 / 62; 20000 rows, 0.4M, FP32 2 / 8 sides 13.0 / 8.1,
-    // 50 / 12; random band of 200000 rows, 7.9M FP32 2 / 3 / 8 sides 32 / 33, 55 /
-    // 41, 104 / 55; 90001 rows, 1.9M FP32 3 / 8 sides 13.0 / 12.9, 26 / 20; 200000
-    // rows, 1.2M, FP32 8 sides 20 / 23.  Chunks of stencils gather coalesced lines
+    // (kScattered) only with many entries.  us, separate columns / packed, with
+    // products summed from LDS: Chung-Lu graph 150000 rows, 3.0M entries FP32 2 / 3 /
+    // 8 sides 37 / 23, 71 / 27, 162 / 40, FP64 8 sides 224 / 62; 20000 rows, 0.4M, FP32
+    // 2 / 8 sides 13.0 / 8.1, 50 / 12; random band of 200000 rows, 7.9M FP32 2 / 3 / 8
+    // sides 32 / 33, 55 / 41, 104 / 55; 90001 rows, 1.9M FP32 3 / 8 sides 13.0 / 12.9,
+    // 26 / 20; 200000 rows, 1.2M, FP32 8 sides 20 / 23.  With values and x there the
+    // packed side takes 23, 26 and 39 us on the first, separate columns 17 on the last.  Chunks of stencils gather coalesced lines
     // as they are (27-point 96^3 FP64 8 sides 135 / 158).
     static constexpr int kSets = 2;
     static constexpr double kScattered = 0.4;
@@ -441,7 +448,7 @@ struct Product {
     int build(const race_kernel_desc& d) {
         n = d.nrow;
         rhs = d.kind == RACE_K_MPK || d.kind == RACE_K_MPK_HIGHEST ? 1 : std::max(1, d.nrhs);
-        useBlocks = ragged(d);
+        useBlocks = ragged(d, rhs);
         if (rhs > 1) {
             const int w = rhs == 2 ? 2 : rhs <= 4 || sizeof(XT) == 8 ? 4 : 8, planes = (rhs + w - 1) / w;
             const long nnz = d.rowPtr[n];
@@ -480,14 +487,14 @@ struct Product {
                            (long)n, rhs);
         launchRowBlkPacked<RR, VT, XT>(blocks, buf, y, n, rhs, acc, st);
     }
-    static bool ragged(const race_kernel_desc& d) {
+    static bool ragged(const race_kernel_desc& d, int rhs) {
         long slots = 0;
         for (int r0 = 0; r0 < d.nrow; r0 += kC) {
             int w = 0;
             for (int r = r0; r < std::min(d.nrow, r0 + kC); ++r) w = std::max(w, d.rowPtr[r + 1] - d.rowPtr[r]);
             slots += w;
         }
-        return slots * kC * 4 > (long)d.rowPtr[d.nrow] * 5;
+        return raggedSlots(slots * kC, d.rowPtr[d.nrow], rhs);
     }
     // y = A x (acc: y += A x)
     void run(const void* x, void* y, int nrhs, bool acc, hipStream_t st) {
@@ -865,8 +872,7 @@ static void expandUpper(const race_kernel_desc& d, std::vector<int>& rp, std::ve
 // SpMV (b = A x) or SymmSpMV (b += A x, expanded from the upper triangle)
 // on a batch of matrices: one launch over the SELL chunks of all matrices
 // that fit the layout, one over the row blocks of those whose chunks would
-// store more than 5 slots for 4 entries (Product's rule) or be wider than 64
-// entries: with 8 right-hand sides a chunk holding a hub row runs its up to
+// store too many slots (raggedSlots) or be wider than 64 entries: with 8 right-hand sides a chunk holding a hub row runs its up to
 // 400 steps once per right-hand side.  16 matrices of 2000 to 40000 rows, FP32,
 // 8 right-hand sides: 864 us in chunks alone, 167 us.
 template <typename XT>
@@ -930,7 +936,7 @@ class SellBatchFn : public DeviceFn {
             hy.push_back((XT*)d.b);
             hn.push_back(n);
             hv.push_back(RowBlkVecs{d.x, d.b, n});
-            if (widest > 64 || slots * 4 > (long)R[n] * 5) {
+            if (widest > 64 || raggedSlots(slots, R[n], nrhs)) {
                 blocks.add(n, R, Cc, V, (int)m);
                 continue;
             }
