@@ -419,7 +419,8 @@ void launchSell(const SellMatrix<VT>& A, const void* x, void* y, int nrhs, bool 
 inline bool raggedSlots(long slots, long nnz, int nrhs) { return nrhs > 1 ? slots * 4 > nnz * 5 : slots * 8 > nnz * 11; }
 
 // A matrix that is multiplied with vectors, in the layout its rows ask for: SELL
-// chunks or row blocks (raggedSlots).
+// chunks or row blocks (raggedSlots).  Regular rows whose right-hand sides are
+// packed have both: launches without scratch run over the chunks.
 template <typename VT, typename XT>
 struct Product {
     SellMatrix<VT> sell;
@@ -445,6 +446,7 @@ struct Product {
     DevBuf<XT> packed[kSets];
     StreamSets streamSets;
     int rhs = 1, R = 0;  // R: right-hand sides of a packed row, 0: not packed
+    int sets = 0;        // scratch there was memory for
     int build(const race_kernel_desc& d) {
         n = d.nrow;
         rhs = d.kind == RACE_K_MPK || d.kind == RACE_K_MPK_HIGHEST ? 1 : std::max(1, d.nrhs);
@@ -454,15 +456,22 @@ struct Product {
             const long nnz = d.rowPtr[n];
             const bool scattered = nnz * (rhs - 1) >= 200000 && linesPerEntry(d) > kScattered;
             if (scattered || (useBlocks && nnz * (rhs - planes) >= 10000000)) {
-                useBlocks = true;
-                R = w;
-                blocks.cap = kPackedEntries;
-                for (DevBuf<XT>& b : packed) RACE_HIP(b.reserve((size_t)n * planes * R));
+                reserveSets((size_t)n * planes * w);
+                if (sets > 0) R = w;
             }
         }
-        if (!useBlocks) return sell.build(d);
+        if (!useBlocks)
+            if (int e = sell.build(d)) return e;
+        if (!useBlocks && R == 0) return OK;
+        if (R) blocks.cap = kPackedEntries;
         blocks.add(n, d.rowPtr, d.col, d.val, 0);
         return blocks.finish();
+    }
+    // as many sets as there is memory for: none is no error, the product then
+    // runs without packing
+    void reserveSets(size_t count) {
+        while (sets < kSets && packed[sets].reserve(count) == hipSuccess) ++sets;
+        if (sets < kSets) (void)hipGetLastError();
     }
     // distinct 128-byte lines of x per entry, in runs of kPackedEntries entries
     // (up to 2000 runs, spread over the matrix)
@@ -498,7 +507,7 @@ struct Product {
     }
     // y = A x (acc: y += A x)
     void run(const void* x, void* y, int nrhs, bool acc, hipStream_t st) {
-        const int set = R && nrhs == rhs ? streamSets.find(st, kSets) : -1;
+        const int set = R && nrhs == rhs ? streamSets.find(st, sets) : -1;
         if (set >= 0) {
             XT* buf = packed[set].p;
             if (R == 2) return runPacked<2>((const XT*)x, (XT*)y, buf, acc, st);
