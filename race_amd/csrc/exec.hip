@@ -176,6 +176,24 @@ __global__ void __launch_bounds__(kBlock) k_symmspmv_chunks(
     }
 }
 
+// b = A x for nrhs right-hand sides (column-major), TPR lanes per row
+template <int TPR>
+__global__ void __launch_bounds__(kBlock) k_spmv(const int* __restrict__ rp, const int* __restrict__ col,
+                                                 const double* __restrict__ val, const double* __restrict__ x,
+                                                 double* __restrict__ b, int n, int nrhs) {
+    const int lane = threadIdx.x % TPR;
+    const int row = (int)((blockIdx.x * (long)blockDim.x + threadIdx.x) / TPR);
+    if (row >= n) return;
+    const int s = rp[row], e = rp[row + 1];
+    for (int k = 0; k < nrhs; ++k) {
+        const size_t off = (size_t)k * n;
+        double t = 0.0;
+        for (int j = s + lane; j < e; j += TPR) t += val[j] * x[off + col[j]];
+        t = groupSum<TPR>(t);
+        if (lane == 0) b[off + row] = t;
+    }
+}
+
 // device CRS copy of a caller matrix
 struct DevCrs {
     int n = 0;
@@ -312,6 +330,40 @@ class SymmSpmvFn : public DeviceFn {
     }
 };
 
+// SpMV of a small matrix with several right-hand sides, FP64 (spmvByLanes):
+// several lanes per row.  One lane per row leaves most of the chip idle there, and
+// its chain of dependent loads bounds the call.
+class SpmvFn : public DeviceFn {
+  public:
+    DevCrs A;
+    int nrhs = 1, tpr = 8;
+    int init(const race_kernel_desc& d) {
+        kind = d.kind;
+        nrhs = d.nrhs > 0 ? d.nrhs : 1;
+        x = d.x;
+        b = d.b;
+        int e;
+        if ((e = A.load(d))) return e;
+        tpr = pickTpr(A.nnz, A.n);
+        return OK;
+    }
+    template <int TPR>
+    void launch(hipStream_t st) {
+        hipLaunchKernelGGL(k_spmv<TPR>, dim3(gridFor((long)A.n * TPR)), dim3(kBlock), 0, st, A.rp.p, A.col.p, A.val.p,
+                           (const double*)x, (double*)b, A.n, nrhs);
+    }
+    int run(bool, hipStream_t st) override {
+        switch (tpr) {
+            case 4: launch<4>(st); break;
+            case 8: launch<8>(st); break;
+            case 16: launch<16>(st); break;
+            default: launch<32>(st); break;
+        }
+        RACE_HIP(hipGetLastError());
+        return OK;
+    }
+};
+
 }  // namespace
 
 int makeWaveFn(const race_kernel_desc& d, const ExecContext& ctx, std::unique_ptr<DeviceFn>* out) {
@@ -377,9 +429,16 @@ int makeDeviceFn(const race_kernel_desc& d, const ExecContext& ctx, std::unique_
             *out = std::move(f);
             break;
         }
-        case RACE_K_SPMV:
-            e = makeSellSpmvFn(d, out);
+        case RACE_K_SPMV: {
+            if (!spmvByLanes(d)) {
+                e = makeSellSpmvFn(d, out);
+                break;
+            }
+            auto f = std::make_unique<SpmvFn>();
+            e = f->init(d);
+            *out = std::move(f);
             break;
+        }
         case RACE_K_SPMTV:
             e = makeSpmtvFn(d, out);
             break;

@@ -95,7 +95,17 @@ int refineSolveStatic(DeviceFn* f, double tol, int maxOuter, hipStream_t st, int
 size_t refineStaticScratchBytes();
 // Gauss-Seidel / Kaczmarz with one workgroup per leaf (exec.hip)
 int makeWaveFn(const race_kernel_desc& d, const ExecContext& ctx, std::unique_ptr<DeviceFn>* out);
-// SELL-C SpMV (one right-hand side) and level-blocked matrix powers (sell.hip)
+// SpMV, FP64, several right-hand sides: whether several lanes per row beat the
+// layouts of sell.hip, which need many rows.  Both measured, us, lanes / chunks or
+// row blocks: 27-point 20^3 (195000 entries) 2 / 3 / 8 sides 3.5 / 4.4, 3.9 / 6.7, 6.5 / 9.4,
+// 23^3 (303000) 8 sides 8.4 / 9.3, 26^3 (441000) 3 / 4 / 8 sides 5.5 / 6.6, 6.8 / 6.8, 11.7 / 9.4,
+// 30^3 (681000) 2 sides 5.4 / 4.5; bands of 20000 rows, 20 entries (400000, row blocks)
+// 2 / 3 / 4 sides 3.8 / 4.2, 4.7 / 5.5, 5.7 / 5.6; 20 random columns in 20000 rows (packed)
+// 3 / 4 sides 7.0 / 7.9, 8.6 / 8.0; 7-point 24^3 2 / 8 sides 3.6 / 3.3, 4.8 / 4.3, ragged rows of
+// Poisson(6) entries 20000 rows 2 / 8 sides 4.0 / 4.9, 11.1 / 9.0.  Hub rows keep their row
+// blocks.
+bool spmvByLanes(const race_kernel_desc& d);
+// SpMV and matrix powers over SELL chunks or row blocks (sell.hip)
 int makeSellSpmvFn(const race_kernel_desc& d, std::unique_ptr<DeviceFn>* out);
 int makeMpkFn(const race_kernel_desc& d, const ExecContext& ctx, std::unique_ptr<DeviceFn>* out);
 // r = b - A x in FP64 with the sums of r^2 and b^2 added to norms[0..1]

@@ -89,6 +89,7 @@ struct SellMatrix {
     int n = 0, nChunk = 0;
     int uniformW = -1;          // >= 0: every chunk has this width, chunk c at c * 64 * width
     bool narrowIds = false;     // 16-bit column ids
+    int perPass = 8;            // right-hand sides per pass, at most
     long bytes = 0;             // stored entries
     DevBuf<SellChunk> chunks;
     DevBuf<int> base, rowPtr;
@@ -371,7 +372,8 @@ constexpr long kL2Bytes = 32l << 20, kInfinityCacheBytes = 256l << 20;
 //
 // one launch of y = A x or y += A x.  Right-hand sides are taken 1, 2, 4 or 8
 // at a time, the smallest block that covers them (8 for 5 to 8, blocks of 4
-// otherwise): a pass over the entries costs more than idle columns of a block.
+// otherwise): a pass over the entries costs more than idle columns of a block,
+// but for scattered columns (Product::Plan).
 template <int NR, typename CT, typename VT, typename XT>
 void launchSellNr(const SellMatrix<VT>& A, const void* x, void* y, int nrhs, bool acc, hipStream_t st) {
     const int g = std::max(1, (A.nChunk + kWavesPerBlock - 1) / kWavesPerBlock);
@@ -390,7 +392,7 @@ void launchSellNr(const SellMatrix<VT>& A, const void* x, void* y, int nrhs, boo
 }
 template <typename CT, typename VT, typename XT>
 void launchSellIds(const SellMatrix<VT>& A, const void* x, void* y, int nrhs, bool acc, hipStream_t st) {
-    if (nrhs == 1)
+    if (nrhs == 1 || A.perPass == 1)
         launchSellNr<1, CT, VT, XT>(A, x, y, nrhs, acc, st);
     else if (nrhs == 2)
         launchSellNr<2, CT, VT, XT>(A, x, y, nrhs, acc, st);
@@ -433,35 +435,60 @@ struct Product {
     // for all of them instead of one each, and one or two trips through the
     // address unit instead of nrhs.  It pays where columns are scattered over
     // x, so that every gather is a line of its own; where lines are shared
-    // (kScattered) only with many entries.  us, separate columns / packed, with
-    // products summed from LDS: Chung-Lu graph 150000 rows, 3.0M entries FP32 2 / 3 /
-    // 8 sides 37 / 23, 71 / 27, 162 / 40, FP64 8 sides 224 / 62; 20000 rows, 0.4M, FP32
-    // 2 / 8 sides 13.0 / 8.1, 50 / 12; random band of 200000 rows, 7.9M FP32 2 / 3 / 8
-    // sides 32 / 33, 55 / 41, 104 / 55; 90001 rows, 1.9M FP32 3 / 8 sides 13.0 / 12.9,
-    // 26 / 20; 200000 rows, 1.2M, FP32 8 sides 20 / 23.  With values and x there the
-    // packed side takes 23, 26 and 39 us on the first, separate columns 17 on the last.  Chunks of stencils gather coalesced lines
-    // as they are (27-point 96^3 FP64 8 sides 135 / 158).
+    // only with many entries, and for regular rows, whose chunks gather
+    // coalesced lines of one side at a time, only with enough entries and sides
+    // (Plan).  us, separate columns / packed, ragged rows: Chung-Lu graph of
+    // 150000 rows, 3.0M entries FP32 2 / 3 / 8 sides 37 / 23, 71 / 26, 162 / 39, FP64 8 sides
+    // 224 / 63; 20000 rows, 0.4M, FP32 2 / 8 sides 13.0 / 7.3, 50 / 10.7.  Regular rows of
+    // random columns, chunks / packed: FP32 40000 rows of 20 entries 2 sides 8.7 /
+    // 8.3, 10000 rows 2 / 3 sides 5.1 / 5.7, 7.4 / 6.0; 50000 rows of 6 3 / 8 sides 5.9 /
+    // 7.9, 11.9 / 10.6; 100000 rows of 24 within 4000 columns (0.42 lines an entry) 2 / 3
+    // / 4 sides 10.4 / 13.8, 15.0 / 16.8, 19.9 / 17.0, 200000 rows of 12 within 8000 (0.61)
+    // 15.5 / 16.4, 22.9 / 20.4, 30.6 / 20.7; 27-point 96^3 FP64 8 sides 135 / 158.  Two sides
+    // of ragged rows: Poisson(12) 20000 rows FP32 4.3 / 6.5, 50000 rows 7.4 / 7.8;
+    // with hub rows, Chung-Lu 60000 rows of 6 FP32 9.6 / 8.7.
     static constexpr int kSets = 2;
-    static constexpr double kScattered = 0.4;
     DevBuf<XT> packed[kSets];
     StreamSets streamSets;
     int rhs = 1, R = 0;  // R: right-hand sides of a packed row, 0: not packed
     int sets = 0;        // scratch there was memory for
+    // how the rows of a matrix and their columns are laid out
+    struct Plan {
+        bool ragged = false, packed = false;
+        long slots = 0;
+        int longest = 0;
+        int perPass = 8;  // right-hand sides per pass over the chunks, at most
+        int width = 1;    // right-hand sides of a packed row
+        Plan(const race_kernel_desc& d, int rhs) {
+            ragged = Product::ragged(d, rhs, &slots, &longest);
+            if (rhs == 1) return;
+            width = rhs == 2 ? 2 : rhs <= 4 || sizeof(XT) == 8 ? 4 : 8;
+            const long nnz = d.rowPtr[d.nrow], planes = (rhs + width - 1) / width;
+            const double lines = linesPerEntry(d);
+            if (ragged)
+                packed = (nnz * (rhs - 1) >= (rhs > 2 ? 200000 : longest > 64 ? 350000 : 700000) && lines > 0.4) ||
+                         nnz * (rhs - planes) >= 10000000;
+            else
+                packed = nnz * (rhs - 1) > 300000 + 3l * d.nrow * rhs && lines > (rhs == 2 ? 0.65 : rhs == 3 ? 0.45 : 0.4);
+            // Columns that share few lines: two or three sides one after the
+            // other, where each side's part of x stays in the caches.  us,
+            // sides together / one after the other: the rows of 0.42 lines an
+            // entry FP32 2 / 3 sides 12.8 / 10.4, 18.6 / 15.0; of 0.24 FP64 3 sides
+            // 19.8 / 17.3, 8 sides 35.5 / 42.6.
+            if (rhs <= 3 && lines > (rhs == 2 ? 0.4 : 0.1)) perPass = 1;
+        }
+    };
     int build(const race_kernel_desc& d) {
         n = d.nrow;
         rhs = d.kind == RACE_K_MPK || d.kind == RACE_K_MPK_HIGHEST ? 1 : std::max(1, d.nrhs);
-        useBlocks = ragged(d, rhs);
-        if (rhs > 1) {
-            const int w = rhs == 2 ? 2 : rhs <= 4 || sizeof(XT) == 8 ? 4 : 8, planes = (rhs + w - 1) / w;
-            const long nnz = d.rowPtr[n];
-            const bool scattered = nnz * (rhs - 1) >= 200000 && linesPerEntry(d) > kScattered;
-            if (scattered || (useBlocks && nnz * (rhs - planes) >= 10000000)) {
-                reserveSets((size_t)n * planes * w);
-                if (sets > 0) R = w;
-            }
-        }
-        if (!useBlocks)
+        const Plan plan(d, rhs);
+        useBlocks = plan.ragged;
+        if (plan.packed) reserveSets((size_t)n * ((rhs + plan.width - 1) / plan.width) * plan.width);
+        if (sets > 0) R = plan.width;
+        if (!useBlocks) {
+            sell.perPass = plan.perPass;
             if (int e = sell.build(d)) return e;
+        }
         if (!useBlocks && R == 0) return OK;
         if (R) blocks.cap = kPackedEntries;
         blocks.add(n, d.rowPtr, d.col, d.val, 0);
@@ -496,14 +523,22 @@ struct Product {
                            (long)n, rhs);
         launchRowBlkPacked<RR, VT, XT>(blocks, buf, y, n, rhs, acc, st);
     }
-    static bool ragged(const race_kernel_desc& d, int rhs) {
+    static bool ragged(const race_kernel_desc& d, int rhs, long* stored, int* longest) {
         long slots = 0;
+        *longest = 0;
         for (int r0 = 0; r0 < d.nrow; r0 += kC) {
             int w = 0;
             for (int r = r0; r < std::min(d.nrow, r0 + kC); ++r) w = std::max(w, d.rowPtr[r + 1] - d.rowPtr[r]);
             slots += w;
+            *longest = std::max(*longest, w);
         }
-        return raggedSlots(slots * kC, d.rowPtr[d.nrow], rhs);
+        // the steps of few short rows take less time than a block's way through
+        // LDS: rows of Poisson(6) entries, us, chunks / row blocks, one side FP64, FP32:
+        // 20000 rows 3.3 3.8, 3.1 3.7, 100000 rows 5.3 6.0, 5.0 5.6, 200000 rows 11.5 8.6, 8.7
+        // 7.9; three sides FP32 50000 rows 7.4 9.3, 5000 rows 5.4 4.2
+        *stored = slots * kC;
+        const bool few = *longest <= 22 && d.nrow <= 100000 && (rhs == 1 || (rhs <= 3 && d.nrow > 10000));
+        return !few && raggedSlots(*stored, d.rowPtr[d.nrow], rhs);
     }
     // y = A x (acc: y += A x)
     void run(const void* x, void* y, int nrhs, bool acc, hipStream_t st) {
@@ -1070,6 +1105,17 @@ int makeSellResidual(const race_kernel_desc& d, std::unique_ptr<ResidualOp>* out
     int e = f->init(d);
     *out = std::move(f);
     return e;
+}
+
+bool spmvByLanes(const race_kernel_desc& d) {
+    const long n = d.nrow, nnz = d.rowPtr[d.nrow];
+    if (d.val_precision != RACE_FP64 || d.vec_precision != RACE_FP64 || d.nrhs <= 1) return false;
+    if (nnz > 450000 || nnz <= 4 * n || nnz * d.nrhs > 2500000) return false;
+    for (int r = 0; r < d.nrow; ++r)
+        if (d.rowPtr[r + 1] - d.rowPtr[r] > 64) return false;
+    const Product<double, double>::Plan plan(d, d.nrhs);
+    if (nnz <= 8 * n && (d.nrhs > 3 || !raggedSlots(plan.slots, nnz, 1))) return false;
+    return nnz * d.nrhs <= 1200000 || (!plan.ragged && !plan.packed);
 }
 
 int makeSellSpmvFn(const race_kernel_desc& d, std::unique_ptr<DeviceFn>* out) {

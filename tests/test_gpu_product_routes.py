@@ -1,5 +1,5 @@
-"""Which kernel a product with several right-hand sides takes: scattered
-columns, streams with and without packing scratch, and a registration
+"""Which kernel a product with several right-hand sides takes: small matrices,
+scattered columns, streams with and without packing scratch, and a registration
 for which there is no scratch memory left.
 
 Bound: a row sum of L products in precision u, in any order, is within
@@ -52,6 +52,17 @@ class Product:
         assert len(bad) == 0, (len(bad), bad[:3])
         self.db.zero()
         assert L.load().race_device_synchronize() == 0
+
+
+# lanes per row: 1 to 64 entries a row, the most entries and columns of the rule and
+# one step past them, rows of 65 entries
+@pytest.mark.parametrize("n,k,nrhs", [(1, 1, 2), (7, 7, 3), (37, 9, 2), (1000, 17, 5), (513, 64, 11), (513, 65, 3),
+                                      (15000, 30, 2), (15001, 30, 2), (5000, 60, 4), (5000, 60, 5), (9999, 8, 8),
+                                      (20000, 20, 3), (20000, 20, 4)])
+def test_small_matrices(n, k, nrhs):
+    for prec in (R.FP64, R.FP32):
+        print("case small", n, k, nrhs, prec, flush=True)
+        Product(*_regular(n, k, n), prec, nrhs).check()
 
 
 # scattered columns of regular rows: packed, and chunks side by side
