@@ -180,7 +180,7 @@ int race_register_device(race_handle h, const race_kernel_desc *desc, int *id);
  *                  for the earlier chains it conflicts with (per-chain
  *                  completion flags) instead of a launch boundary per phase;
  *                  calls of one function must not overlap.  0 = one launch
- *                  per phase.  Unless set, small matrices take the one-launch
+ *                  per phase.  -1 (default) = small matrices take the one-launch
  *                  sweep and others the phase launches (calls may overlap on
  *                  different streams).  Set before registering; results
  *                  identical

@@ -572,7 +572,7 @@ int race_set_option(race_handle h, const char* key, int value) {
         if (value != 0 && value != 1) return ERR_INVALID_ARG;
         h->optGraph = value;
     } else if (k == "flow") {
-        if (value != 0 && value != 1) return ERR_INVALID_ARG;
+        if (value < -1 || value > 1) return ERR_INVALID_ARG;
         h->optFlow = value;
     } else if (k == "bfs_block_max") {
         if (value < 0) return ERR_INVALID_ARG;
