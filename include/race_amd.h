@@ -182,8 +182,10 @@ int race_register_device(race_handle h, const race_kernel_desc *desc, int *id);
  *                  calls of one function must not overlap.  0 = one launch
  *                  per phase.  -1 (default) = small matrices take the one-launch
  *                  sweep and others the phase launches (calls may overlap on
- *                  different streams).  Set before registering; results
- *                  identical
+ *                  different streams; the first eight streams that a function
+ *                  runs on sweep in one launch, further ones and captured
+ *                  calls by phases; end a stream's calls before destroying
+ *                  it).  Set before registering; results identical
  * No counterpart in the reference (its executor has no layout choice). */
 int race_set_option(race_handle h, const char *key, int value);
 /* re-point a registered device function at other vectors */
@@ -315,7 +317,10 @@ int race_schedule_info(const void *buf, size_t size, int *nrow, int *dist, int *
 /* dependency waves of a registered GS/KACZ function (critical path length) */
 int race_get_wave_count(race_handle h, int id, int rev, int *waves);
 /* kernel launches one execution of a registered device function issues
- * (colour phases, MPK powers) */
+ * (colour phases, MPK powers) on the handle's stream.  Calls on streams without
+ * scratch of their own ("flow" unset; several right-hand sides) and captured
+ * calls may issue another number: the phases instead of one sweep, one product
+ * instead of packing and product. */
 int race_get_launch_count(race_handle h, int id, int rev, int *launches);
 /* one-launch ("flow") sweeps of a device function whose dependency waits gave
  * up after their poll budget (always 0 for a consistent schedule; a nonzero

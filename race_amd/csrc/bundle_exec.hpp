@@ -1406,8 +1406,11 @@ void launchPhase(int bs, int tpr, int E, int kind, int nrhs, const BundleDev<VT,
 // (about seconds; a correct dependency table never gets near it)
 constexpr int kFlowPollLimit = 1 << 22;
 // and of a launch that the caller did not ask for by the option (and whose
-// aborts it will not look for): far longer than any pause of the device
-constexpr int kAutoPollLimit = 1 << 30;
+// aborts it will not look for): 16 times as long, about a minute, longer than any
+// pause of the device.  A table that would need it is refused at registration
+// (FlowDev::init, BundleFn::init: every dependency on an earlier chain of an
+// earlier phase); should one be wrong all the same, the launch ends.
+constexpr int kAutoPollLimit = 1 << 26;
 
 // Device state of the one-launch sweep of one direction: the bundle range
 // and the dependencies of every chain, column ids with the coherent-read
@@ -1748,8 +1751,9 @@ class BundleFn : public DeviceFn {
     // Long chains are left out: their coherent stores cost more than the
     // launches (Chung-Lu graph of 20000 rows, 4 launches: 1916 / 2064).
     // Sweeps that overlap need sets of their own, so each of the first kSets
-    // streams gets one; other streams and captured launches run the phases.
-    static constexpr int kSets = 2, kAutoBundles = 4;
+    // streams gets one (a flag or two numbers per chain); other streams and
+    // captured launches run the phases.
+    static constexpr int kSets = 8, kAutoBundles = 4;
     static int autoChains(int kind) { return kind == RACE_K_GS ? 896 : sizeof(XT) == 8 ? 16384 : 1280; }
     bool autoFlow = false;
     StreamSets streamSets;
