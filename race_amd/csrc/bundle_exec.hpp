@@ -897,7 +897,7 @@ __global__ void __launch_bounds__(BS) k_gs_bundle_vl(
     const int* __restrict__ rowId, const XT* __restrict__ diag, const int* __restrict__ ext,
     const uint16_t* __restrict__ sidx, const VT* __restrict__ sval, long zero, XT* __restrict__ x0,
     const XT* __restrict__ b0, int n0, int nrhs, const int* __restrict__ chainPtr, int chain0, int nchain, int xcd,
-    int ldsLocal, int ldsRows, const int* __restrict__ lanePtr, const uint16_t* __restrict__ laneSlot,
+    int ldsLocal, const int* __restrict__ lanePtr, const uint16_t* __restrict__ laneSlot,
     XT* const* __restrict__ bX, const XT* const* __restrict__ bB, const int* __restrict__ bN) {
     constexpr int E = kVarE;
     extern __shared__ __align__(16) unsigned char smem[];
@@ -905,7 +905,6 @@ __global__ void __launch_bounds__(BS) k_gs_bundle_vl(
     XT* xl = reinterpret_cast<XT*>(smem);
     XT* part = xl + ldsLocal;                               // BS partial sums
     int* rl0 = reinterpret_cast<int*>(part + BS);           // row -> first lane
-    (void)ldsRows;
 
     const int q = bundleOfBlock(nchain, xcd);
     if (q < 0) return;
@@ -1372,7 +1371,7 @@ void launchBundlesVL(int kind, int nrhs, const BundleDev<VT, XT>& d, int c0, int
     else
         hipLaunchKernelGGL((k_gs_bundle_vl<BS, VT, XT, BATCH>), grid, dim3(BS), d.lds(p, BS).bytes, st, d.slot.p, d.wave.p,
                            d.off.p, d.len.p, d.extPtr.p, d.slotWave.p, d.rowId.p, d.diag.p, d.ext.p, d.sidx.p,
-                           d.sval.p, d.zero, x, b, n, nrhs, d.chainPtr.p, c0, nchain, xcd, d.h.phLocal[p], d.h.phRows[p],
+                           d.sval.p, d.zero, x, b, n, nrhs, d.chainPtr.p, c0, nchain, xcd, d.h.phLocal[p],
                            d.lanePtr.p, d.laneSlot.p, bX, bB, bN);
 }
 
@@ -1463,40 +1462,28 @@ struct FlowDev {
         lds = plan.bytes;
         spare = plan.spare;
         if (!(fits = lds <= d.maxLds)) return OK;  // not used
-        // tickets in chain order (phase order); tables indexed by ticket
-        // position
-        std::vector<int> order(nchain);
-        for (int c = 0; c < nchain; ++c) order[c] = c;
-        std::vector<int> pos(nchain), hlo(nchain), hhi(nchain), qp(nchain + 1, 0), qd;
-        for (int q = 0; q < nchain; ++q) pos[order[q]] = q;
-        qd.reserve(dd.size());
-        for (int q = 0; q < nchain; ++q) {
-            const int c = order[q];
-            hlo[q] = d.h.chainPtr[c];
-            hhi[q] = d.h.chainPtr[c + 1];
-            for (int j = dp[c]; j < dp[c + 1]; ++j) {
-                if (pos[dd[j]] >= q) return ERR_INTERNAL;  // a dependency after its chain
-                qd.push_back(pos[dd[j]]);
-            }
-            qp[q + 1] = (int)qd.size();
-        }
+        // tickets in chain order (phase order)
+        for (int c = 0; c < nchain; ++c)
+            for (int j = dp[c]; j < dp[c + 1]; ++j)
+                if (dd[j] >= c) return ERR_INTERNAL;  // a dependency after its chain
+        const std::vector<int>& cp = d.h.chainPtr;
         int e;
-        if ((e = upload(depPtr, qp.data(), qp.size()))) return e;
-        if ((e = upload(dep, qd.data(), qd.size()))) return e;
-        if ((e = upload(lo, hlo.data(), hlo.size()))) return e;
-        if ((e = upload(hi, hhi.data(), hhi.size()))) return e;
+        if ((e = upload(depPtr, dp.data(), dp.size()))) return e;
+        if ((e = upload(dep, dd.data(), dd.size()))) return e;
+        if ((e = upload(lo, cp.data(), (size_t)nchain))) return e;
+        if ((e = upload(hi, cp.data() + 1, (size_t)nchain))) return e;
         const std::vector<int> fx = flowExt(d.h, nkeys, colBase);
         if ((e = upload(ext, fx.data(), fx.size()))) return e;
         if (ready) {
-            std::vector<int> sp(nchain + 1, 0), sv(qd.size()), rv;
+            std::vector<int> sp(nchain + 1, 0), sv(dd.size()), rv;
             for (int c = 0; c < nchain; ++c)
-                for (int j = qp[c]; j < qp[c + 1]; ++j) ++sp[qd[j] + 1];
+                for (int j = dp[c]; j < dp[c + 1]; ++j) ++sp[dd[j] + 1];
             for (int c = 0; c < nchain; ++c) sp[c + 1] += sp[c];
             std::vector<int> fill(sp.begin(), sp.end() - 1);
             for (int c = 0; c < nchain; ++c)
-                for (int j = qp[c]; j < qp[c + 1]; ++j) sv[fill[qd[j]]++] = c;
+                for (int j = dp[c]; j < dp[c + 1]; ++j) sv[fill[dd[j]]++] = c;
             for (int c = 0; c < nchain; ++c)
-                if (qp[c + 1] == qp[c]) rv.push_back(c);
+                if (dp[c + 1] == dp[c]) rv.push_back(c);
             nroots = (int)rv.size();
             // queue positions are chain numbers (order is the identity)
             for (long p : chainLongestPaths(d.h, dp, dd, kBundleFixedWaves)) longestPath = std::max(longestPath, p);

@@ -513,8 +513,8 @@ int race_register_device(race_handle h, const race_kernel_desc* d, int* id) {
     if (power != (h->dist == DIST_POWER) && !free) return ERR_INVALID_ARG;
     if (!free && !h->colored) return ERR_INVALID_ARG;
     // power > highestPower is allowed, as in the reference (which only warns,
-    // src/interface.cpp:449-452): the wavefront is correct for any power,
-    // only the cache blocking was sized for highestPower
+    // src/interface.cpp:449-452): the powers run one after the other, whatever
+    // power the groups were sized for
     if (power && d->power < 1) return ERR_INVALID_ARG;
     // A kernel that writes the columns of its rows (Kaczmarz, colour-phase
     // SymmSpMV) relies on distance-2 independence of concurrent rows; rows

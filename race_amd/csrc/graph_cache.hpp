@@ -1,7 +1,7 @@
 // graph_cache.hpp -- a device function's launch sequence as a HIP graph.
 //
-// A colour-phase function issues one kernel per phase (32 for a symmetric
-// Gauss-Seidel step on 27-pt 128^3, 116 for k = 8 matrix powers).  The
+// A colour-phase function issues one kernel per phase (26 for a symmetric
+// Gauss-Seidel step on 27-pt 128^3), the matrix powers one per power.  The
 // sequence depends only on the function, the sweep direction, the vectors
 // and the power, so it is captured once per such key on a private stream,
 // instantiated, and replayed with one hipGraphLaunch on the caller's

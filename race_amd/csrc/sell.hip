@@ -577,6 +577,36 @@ class SellSpmvFn : public DeviceFn {
     }
 };
 
+// full CRS of a symmetric matrix from its upper triangle (diagonal first):
+// row r holds its upper entries, then (c, r) of the rows c < r
+static void expandUpper(const race_kernel_desc& d, std::vector<int>& rp, std::vector<int>& fc,
+                        std::vector<double>& fv) {
+    const int n = d.nrow;
+    std::vector<int> cnt(n + 1, 0);
+    for (int r = 0; r < n; ++r)
+        for (int j = d.rowPtr[r]; j < d.rowPtr[r + 1]; ++j) {
+            ++cnt[r + 1];
+            if (d.col[j] != r) ++cnt[d.col[j] + 1];
+        }
+    for (int r = 0; r < n; ++r) cnt[r + 1] += cnt[r];
+    rp = cnt;
+    fc.assign(cnt[n], 0);
+    fv.assign(cnt[n], 0.0);
+    std::vector<int> pos(cnt.begin(), cnt.end() - 1);
+    for (int r = 0; r < n; ++r)
+        for (int j = d.rowPtr[r]; j < d.rowPtr[r + 1]; ++j) {
+            fc[pos[r]] = d.col[j];
+            fv[pos[r]++] = d.val[j];
+        }
+    for (int r = 0; r < n; ++r)
+        for (int j = d.rowPtr[r]; j < d.rowPtr[r + 1]; ++j) {
+            const int c = d.col[j];
+            if (c == r) continue;
+            fc[pos[c]] = r;
+            fv[pos[c]++] = d.val[j];
+        }
+}
+
 // SymmSpMV b += A x from the upper triangle, in one launch:
 //  mode 2: SELL-C upper triangle, FP64 atomics for every write to b (FP64 only);
 //  mode 3: the full matrix (upper triangle and its transpose) built once at
@@ -594,35 +624,13 @@ class SymmSellFn : public DeviceFn {
         b = d.b;
         mode = mode_;
         nrhs = d.nrhs > 0 ? d.nrhs : 1;
-        const int n = d.nrow;
         if (mode == 2) {
             if (!std::is_same<VT, double>::value || !std::is_same<XT, double>::value) return ERR_NOT_IMPLEMENTED;
             return A.sell.build(d);
         }
-        // full pattern: row r holds its upper entries, then the transposed
-        // entries (c, r) of rows c < r, each in increasing c
-        std::vector<int> cnt(n + 1, 0);
-        for (int r = 0; r < n; ++r)
-            for (int j = d.rowPtr[r]; j < d.rowPtr[r + 1]; ++j) {
-                ++cnt[r + 1];
-                if (d.col[j] != r) ++cnt[d.col[j] + 1];
-            }
-        for (int r = 0; r < n; ++r) cnt[r + 1] += cnt[r];
-        std::vector<int> rp(cnt), fc(cnt[n]);
-        std::vector<double> fv(cnt[n]);
-        std::vector<int> pos(cnt.begin(), cnt.end() - 1);
-        for (int r = 0; r < n; ++r)
-            for (int j = d.rowPtr[r]; j < d.rowPtr[r + 1]; ++j) {
-                fc[pos[r]] = d.col[j];
-                fv[pos[r]++] = d.val[j];
-            }
-        for (int r = 0; r < n; ++r)
-            for (int j = d.rowPtr[r]; j < d.rowPtr[r + 1]; ++j) {
-                const int c = d.col[j];
-                if (c == r) continue;
-                fc[pos[c]] = r;
-                fv[pos[c]++] = d.val[j];
-            }
+        std::vector<int> rp, fc;
+        std::vector<double> fv;
+        expandUpper(d, rp, fc, fv);
         race_kernel_desc f = d;
         f.rowPtr = rp.data();
         f.col = fc.data();
@@ -883,42 +891,12 @@ __global__ void __launch_bounds__(kBlock) k_sellg_spmv(const SellGChunk* __restr
     }
 }
 
-// full CRS of a symmetric matrix from its upper triangle (diagonal first):
-// row r holds its upper entries, then (c, r) of the rows c < r
-static void expandUpper(const race_kernel_desc& d, std::vector<int>& rp, std::vector<int>& fc,
-                        std::vector<double>& fv) {
-    const int n = d.nrow;
-    std::vector<int> cnt(n + 1, 0);
-    for (int r = 0; r < n; ++r)
-        for (int j = d.rowPtr[r]; j < d.rowPtr[r + 1]; ++j) {
-            ++cnt[r + 1];
-            if (d.col[j] != r) ++cnt[d.col[j] + 1];
-        }
-    for (int r = 0; r < n; ++r) cnt[r + 1] += cnt[r];
-    rp = cnt;
-    fc.assign(cnt[n], 0);
-    fv.assign(cnt[n], 0.0);
-    std::vector<int> pos(cnt.begin(), cnt.end() - 1);
-    for (int r = 0; r < n; ++r)
-        for (int j = d.rowPtr[r]; j < d.rowPtr[r + 1]; ++j) {
-            fc[pos[r]] = d.col[j];
-            fv[pos[r]++] = d.val[j];
-        }
-    for (int r = 0; r < n; ++r)
-        for (int j = d.rowPtr[r]; j < d.rowPtr[r + 1]; ++j) {
-            const int c = d.col[j];
-            if (c == r) continue;
-            fc[pos[c]] = r;
-            fv[pos[c]++] = d.val[j];
-        }
-}
-
 // SpMV (b = A x) or SymmSpMV (b += A x, expanded from the upper triangle)
 // on a batch of matrices: one launch over the SELL chunks of all matrices
 // that fit the layout, one over the row blocks of those whose chunks would
 // store too many slots (raggedSlots) or be wider than 64 entries: with 8 right-hand sides a chunk holding a hub row runs its up to
 // 400 steps once per right-hand side.  16 matrices of 2000 to 40000 rows, FP32,
-// 8 right-hand sides: 864 us in chunks alone, 167 us.
+// 8 right-hand sides: 864 us in chunks of 64 rows alone, 80 us.
 template <typename XT>
 class SellBatchFn : public DeviceFn {
   public:
