@@ -23,6 +23,7 @@
 
 #include <algorithm>
 #include <cstdint>
+#include <functional>
 #include <type_traits>
 
 #include "exec.hpp"
@@ -893,10 +894,10 @@ __global__ void __launch_bounds__(kBlock) k_sellg_spmv(const SellGChunk* __restr
 
 // SpMV (b = A x) or SymmSpMV (b += A x, expanded from the upper triangle)
 // on a batch of matrices: one launch over the SELL chunks of all matrices
-// that fit the layout, one over the row blocks of those whose chunks would
-// store too many slots (raggedSlots) or be wider than 64 entries: with 8 right-hand sides a chunk holding a hub row runs its up to
-// 400 steps once per right-hand side.  16 matrices of 2000 to 40000 rows, FP32,
-// 8 right-hand sides: 864 us in chunks of 64 rows alone, 80 us.
+// that fit the layout, one over the row blocks of the others (chooseBlocks): with 8
+// right-hand sides a chunk holding a hub row runs its up to 400 steps once per
+// right-hand side.  16 matrices of 2000 to 40000 rows, FP32, 8 right-hand sides: 864 us
+// in chunks of 64 rows alone, 80 us.
 template <typename XT>
 class SellBatchFn : public DeviceFn {
   public:
@@ -909,6 +910,49 @@ class SellBatchFn : public DeviceFn {
     DevBuf<XT*> my;
     RowBlocks<XT> blocks;
     DevBuf<RowBlkVecs> vecs;
+
+    // The matrices that go to row blocks: those over 5 slots for 4 entries in
+    // chunks, or with a chunk wider than 64 entries.  Where none is over 11 for 8
+    // and they hold less than a 16th of the batch's entries, all stay in chunks: a
+    // second launch for a few small matrices costs more (stencils, 27-point 10^3 of
+    // 1.26 slots an entry among them, one side FP64, us: 13.6 in chunks, 17.2 in two
+    // launches).
+    std::vector<char> chooseBlocks(const std::vector<BatchItem>& items) const {
+        std::vector<char> in(items.size(), 0);
+        std::vector<int> len;
+        long entries = 0, over = 0;
+        bool far = false;
+        for (size_t m = 0; m < items.size(); ++m) {
+            const race_kernel_desc& d = items[m].d;
+            const int n = d.nrow;
+            len.assign(n, 0);
+            for (int r = 0; r < n; ++r)
+                for (int j = d.rowPtr[r]; j < d.rowPtr[r + 1]; ++j) {
+                    ++len[r];
+                    if (kind == RACE_K_SYMMSPMV && d.col[j] != r) ++len[d.col[j]];
+                }
+            if (perm)
+                for (int w0 = 0; w0 < n; w0 += sigma)
+                    std::sort(len.begin() + w0, len.begin() + std::min(n, w0 + sigma), std::greater<int>());
+            long slots = 0, nnz = 0;
+            int widest = 0;
+            for (int r0 = 0; r0 < n; r0 += C) {
+                int w = 0;
+                for (int r = r0; r < std::min(n, r0 + C); ++r) {
+                    w = std::max(w, len[r]);
+                    nnz += len[r];
+                }
+                slots += (long)w * C;
+                widest = std::max(widest, w);
+            }
+            entries += nnz;
+            in[m] = widest > 64 || slots * 4 > nnz * 5;
+            if (in[m]) over += nnz;
+            far = far || widest > 64 || slots * 8 > nnz * 11;
+        }
+        if (!far && over * 16 < entries) in.assign(items.size(), 0);
+        return in;
+    }
 
     int init(const std::vector<BatchItem>& items, const ExecContext& ctx) {
         kind = items[0].d.kind;
@@ -925,6 +969,7 @@ class SellBatchFn : public DeviceFn {
         std::vector<RowBlkVecs> hv;
         std::vector<int> rp, fc, order;
         std::vector<double> fv;
+        const std::vector<char> inBlocks = chooseBlocks(items);
         for (size_t m = 0; m < items.size(); ++m) {
             const race_kernel_desc& d = items[m].d;
             const int n = d.nrow;
@@ -946,19 +991,11 @@ class SellBatchFn : public DeviceFn {
                         return R[a + 1] - R[a] > R[b + 1] - R[b];
                     });
                 }
-            long slots = 0;
-            int widest = 0;
-            for (int r0 = 0; r0 < n; r0 += C) {
-                int w = 0;
-                for (int r = r0; r < std::min(n, r0 + C); ++r) w = std::max(w, R[order[r] + 1] - R[order[r]]);
-                slots += (long)w * C;
-                widest = std::max(widest, w);
-            }
             hx.push_back((const XT*)d.x);
             hy.push_back((XT*)d.b);
             hn.push_back(n);
             hv.push_back(RowBlkVecs{d.x, d.b, n});
-            if (widest > 64 || raggedSlots(slots, R[n], nrhs)) {
+            if (inBlocks[m]) {
                 blocks.add(n, R, Cc, V, (int)m);
                 continue;
             }
