@@ -1516,6 +1516,7 @@ struct FlowDev {
     // only find the tickets gone)
     int occupy(const void* kern, int bs, int most = INT32_MAX) {
         if (!kern) return ERR_INTERNAL;
+        if (!fits) return OK;  // not used
         int per = 0, dev = 0, cus = 0;
         RACE_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kern, bs, lds));
         RACE_HIP(hipGetDevice(&dev));
@@ -1602,14 +1603,9 @@ int launchKaczFlow(const BundleDev<VT, XT>& d, FlowDev& f, int set, XT* x, const
                                d.extPtr.p, d.slotWave.p, d.rowId.p, d.rowNorm.p, f.ext.p, d.sidx.p, d.sval.p, d.zero, x,
                                b, n, f.spare, bX, bB, bN, f.tables(set));
         };
-        if constexpr (BATCH)
-            if (f.held == kLeanSlots) {
-                launch(k_kacz_flow<BS, TPR, EE, VT, XT, BATCH, kLeanSlots>);
-                RACE_HIP(hipGetLastError());
-                return OK;
-            }
-        if (f.held == kFewSlots)
-            launch(k_kacz_flow<BS, TPR, EE, VT, XT, BATCH, kFewSlots>);
+        constexpr int fewer = BATCH ? kLeanSlots : kFewSlots;
+        if (f.held == fewer)
+            launch(k_kacz_flow<BS, TPR, EE, VT, XT, BATCH, fewer>);
         else
             launch(k_kacz_flow<BS, TPR, EE, VT, XT, BATCH, kColSlots>);
     }
@@ -1678,12 +1674,11 @@ const void* kaczFlowKernelOf(int tpr, int E) {
 }
 template <int BS, typename VT, typename XT, bool BATCH>
 const void* kaczFlowKernelBs(int held, int tpr, int E) {
-    if constexpr (BATCH)
-        if (held == kLeanSlots) return kaczFlowKernelOf<BS, kLeanSlots, VT, XT, BATCH>(tpr, E);
-    return held == kFewSlots ? kaczFlowKernelOf<BS, kFewSlots, VT, XT, BATCH>(tpr, E)
-                             : kaczFlowKernelOf<BS, kColSlots, VT, XT, BATCH>(tpr, E);
+    constexpr int fewer = BATCH ? kLeanSlots : kFewSlots;
+    return held == fewer ? kaczFlowKernelOf<BS, fewer, VT, XT, BATCH>(tpr, E)
+                         : kaczFlowKernelOf<BS, kColSlots, VT, XT, BATCH>(tpr, E);
 }
-// held: column ids a thread holds (kLeanSlots: batches only)
+// held: column ids a thread holds (kLeanSlots: batches only, kFewSlots: others)
 template <typename VT, typename XT, bool BATCH>
 const void* kaczFlowKernel(int held, int bs, int tpr, int E) {
     switch (bs) {
